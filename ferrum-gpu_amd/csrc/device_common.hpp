@@ -158,6 +158,11 @@ __device__ __forceinline__ T group_reduce(T v, Op op) {
 // GEMM's fused epilogue) uses this one definition, so their results are bit-identical.
 __device__ __forceinline__ float swiglu_act(float g, float u) { return __fmul_rn(g / (1.0f + expf(-g)), u); }
 
+// GELU, tanh form (ferrum_ref/src/kernels/nn.rs:12-15).
+__device__ __forceinline__ float gelu_act(float x) {
+    return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
+}
+
 template <class T, class Op>
 __device__ __forceinline__ T wave_reduce(T v, Op op) {
     v = group_reduce<16>(v, op);

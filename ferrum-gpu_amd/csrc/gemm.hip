@@ -2742,27 +2742,33 @@ hipError_t launch_make_b8(hipStream_t s, fh_kind kind, const uint8_t *qs, const 
     return hipGetLastError();
 }
 
-// x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned)
-size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n) {
+size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n) {
     uint32_t sp = precise_splits(rows, k, n), ssp = 1;
     if (stream_plan(rows, k, n, &ssp) && stream_supported(rows, k, n)) sp = max(sp, ssp);
-    return (rows * k * 4 + 255) / 256 * 256 + (sp > 1 ? (size_t)sp * rows * n * 4 : 0);
+    return sp > 1 ? (size_t)sp * rows * n * 4 : 0;
+}
+
+// x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned)
+size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n) {
+    return (rows * k * 4 + 255) / 256 * 256 + gemm_precise_partial_bytes(rows, k, n);
 }
 
 hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x,
-                               float *y, size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer) {
+                               float *y, size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer,
+                               float *partial) {
     _Float16 *xs = (_Float16 *)workspace;
-    const size_t xbytes = (rows * k * 4 + 255) / 256 * 256;
-    float *partial = gemm_precise_workspace_bytes(rows, k, n) > xbytes ? (float *)((uint8_t *)workspace + xbytes)
-                                                                       : nullptr;
+    if (!gemm_precise_partial_bytes(rows, k, n))
+        partial = nullptr;
+    else if (!partial)
+        partial = (float *)((uint8_t *)workspace + (rows * k * 4 + 255) / 256 * 256);
     const size_t items = rows * (k / 32);
     const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
     if (kind == FH_Q8_0) {
-        split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items);
+        if (x) split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items);
         return gemm_precise_dispatch<FH_Q8_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                               defer);
     }
-    split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items);
+    if (x) split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items);
     return gemm_precise_dispatch<FH_Q4_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                           defer);
 }

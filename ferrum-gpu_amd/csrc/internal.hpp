@@ -297,9 +297,42 @@ bool gemm_ext_kind(int kind);
 size_t gemm_ext_workspace_bytes(int kind, size_t rows, size_t k, size_t n);
 hipError_t launch_gemm_ext(hipStream_t s, int kind, const uint8_t *w, const float *x, float *y, size_t rows, size_t k,
                            size_t n, void *workspace);
+// x == nullptr: x is already split at the start of the workspace, in split_x_precise_kernel's order;
+// partial != nullptr: the K-split partial products go there (as launch_gemm's).
 hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x,
                                float *y, size_t rows, size_t k, size_t n, void *workspace,
-                               SplitOut *defer = nullptr);
+                               SplitOut *defer = nullptr, float *partial = nullptr);
+size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n);
+
+// prefill.hip: the GPT-2 prompt pass (one row per prompt token). prefill_row_kernel makes a row by mode
+// and writes it as a product's split x (launch_gemm_precise's), scaled by a power of two whose inverse
+// goes to out_scale[row]; the product's consumer multiplies by it (in_scale).
+enum { PREFILL_EMBED_LN = 0, PREFILL_RES_LN = 1, PREFILL_GELU = 2, PREFILL_PLAIN = 3 };
+struct PrefillRow {
+    const float *src;       // RES_LN, GELU: a product's K-split parts [splits][rows][k]; PLAIN: the rows
+    uint32_t splits;
+    size_t stride;          // floats from one part to the next
+    const float *in_scale;  // of the product
+    const float *bias;      // added to the product
+    float *x;               // the residual rows (written by EMBED_LN, updated by RES_LN)
+    const float *ln_g, *ln_b;
+    float eps;
+    const int32_t *tokens;  // EMBED_LN: the rows' tokens and position embeddings, the token embedding
+    const float *pos;
+    const uint8_t *emb_qs;
+    const uint16_t *emb_ds;
+    _Float16 *xs;
+    float *out_scale;
+    uint32_t k;             // values per row, a multiple of 32 up to 16384
+};
+bool prefill_head_supported(size_t hd);
+hipError_t launch_prefill_row(hipStream_t s, fh_kind kind, int mode, const PrefillRow &a, uint32_t rows);
+// The QKV product's rows to q [rows][d] and the caches' rows kc, vc.
+hipError_t launch_prefill_qkv(hipStream_t s, const SplitOut &src, const float *in_scale, const float *bias, float *q,
+                              float *kc, float *vc, uint32_t rows, uint32_t d);
+// Causal attention of rows at positions p0 .. over the caches' rows 0 .. p0 + rows - 1.
+hipError_t launch_prefill_attention(hipStream_t s, const float *q, const float *kc, const float *vc, float *att,
+                                    uint32_t p0, uint32_t rows, uint32_t heads, uint32_t hd, float scale);
 
 // The scoring head's product with the score folded into its epilogue: no logits are written;
 // per row and 256-column tile the tile's softmax statistics (maximum, sum of exp(v - maximum),

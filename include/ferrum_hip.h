@@ -403,8 +403,9 @@ FH_API size_t fh_gpt2_step_launches(const fh_gpt2 *m);
 FH_API fh_status fh_gpt2_feed(fh_device *dev, fh_gpt2 *m, size_t token, float *logits);
 /* Greedy generation from the current position: feed the prompt, then pick n_new tokens by argmax
  * (ferrum_model/src/sampling.rs:32-40), each fed back except the last (the reference's generate
- * loop, ferrum_gpu_core/src/engine/mod.rs:204-242). Picks stay on the device; out receives them
- * at the end, after the only wait. */
+ * loop, ferrum_gpu_core/src/engine/mod.rs:204-242). The prompt's tokens before its last one go
+ * through each product together where that is faster than a step each (their cache rows then differ
+ * from fh_gpt2_feed's in rounding). Picks stay on the device; out receives them at the end. */
 FH_API fh_status fh_gpt2_generate(fh_device *dev, fh_gpt2 *m, const int32_t *prompt, size_t n_prompt,
                                   size_t n_new, int32_t *out);
 
