@@ -30,6 +30,9 @@ struct fh_device {
     std::mutex ws_mu;
     void *ws = nullptr;
     size_t ws_bytes = 0;
+    // kTicketCount zeros: arrival counters of launches that split a product's K over workgroups; every
+    // such launch leaves them zero, and launches on the one stream use them in order.
+    uint32_t *tickets = nullptr;
     // This GPU's copy of the no-allocation entry point's static scratch array (its device
     // address, taken when the device is opened).
     void *scratch = nullptr;
@@ -229,6 +232,13 @@ uint32_t rows_tasks(size_t n, size_t k, size_t max_m);
 // Two launches: split x into `xsplit`, then the product.
 hipError_t launch_rows(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
                        size_t rows, size_t k, size_t n, void *xsplit, int cus);
+// One launch for one product of 2 to kRowsMax rows (fits: where it is the faster one); scratch holds
+// rows_call_scratch_bytes, tickets kTicketCount zeros (left zero).
+constexpr size_t kTicketCount = 8192;
+bool rows_call_fits(size_t rows, size_t k, size_t n, int cus);
+size_t rows_call_scratch_bytes(size_t rows, size_t k, size_t n, int cus);
+hipError_t launch_rows_call(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                            size_t rows, size_t k, size_t n, void *scratch, uint32_t *tickets, int cus);
 // Many products of one format: descs and map (device memory) as for launch_gemv_group; max_m the
 // most rows of any product, max_items the largest rows * k / 32.
 hipError_t launch_rows_group(hipStream_t s, fh_kind kind, const RowsDesc *descs, const uint32_t *map, uint32_t count,

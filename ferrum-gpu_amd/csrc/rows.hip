@@ -30,6 +30,8 @@
 // exact, so the result does not depend on which half arrives first. Per batch the workgroup stages x's split rows for the batch in LDS
 // (double buffered, one barrier per batch) and every wavefront reads its A fragments from there,
 // while its own weights for the next batch are already in flight. Workgroups loop over the tasks.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "internal.hpp"
 
@@ -423,6 +425,257 @@ hipError_t launch_rows_mt(hipStream_t s, const RowsDesc *descs, const uint32_t *
     }
 }
 
+
+// ---- one product per launch (linear_q, AUTO, 2 to 64 rows) ----
+// A single few-row product is bound by latency, not by bytes or by the matrix cores: an 896 x 1152
+// Q8_0 product of 24 rows is 1.1 MB of weights (0.2 us at HBM speed), and the two kernels above took 14 us
+// for it (an x split, a launch boundary, then 9 workgroups that each walk all of K with one batch in
+// flight). Here it is one launch: a workgroup takes 32 TN outputs, its eight wavefronts share the
+// blocks of K two at a time (the next two in flight), each splitting the x values it needs in
+// registers straight from x (every x element is split once per workgroup), and the wavefronts' sums
+// meet in LDS in a fixed order. Deep products with few outputs also split K over S workgroups: each
+// writes its sums agent-coherent and takes a ticket, and the last to arrive adds them in split order
+// (reproducible) and returns the ticket to zero. Same operand order and numerics as rows_kernel.
+// Qwen2-0.5B layer, 24 rows, Q8_0, four calls: 70.3 -> 31.9 us.
+constexpr int kCallWaves = 8;
+constexpr int kCallKB = 2;  // blocks a wavefront takes at a time
+
+typedef __attribute__((address_space(1))) uint32_t gl_u32;
+__device__ __forceinline__ void agent_store(float *p, float v) {
+    __hip_atomic_store((gl_u32 *)p, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float agent_load(const float *p) {
+    return __uint_as_float(__hip_atomic_load((gl_u32 *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// Eight x values (two float4) -> their hi and lo parts in operand order.
+__device__ __forceinline__ void split_frag(const f32x4 &a, const f32x4 &b, f16x8 &hi, f16x8 &lo) {
+    const float e[8] = {a.x, a.z, a.y, a.w, b.x, b.z, b.y, b.w};
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        const _Float16 v = (_Float16)fminf(fmaxf(e[q], -65504.0f), 65504.0f);
+        hi[q] = v;
+        lo[q] = (_Float16)(e[q] - (float)v);
+    }
+}
+
+template <int KIND, int MT, int TN>
+__global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void rows_call_kernel(
+    const uint8_t *__restrict__ qs, const uint16_t *__restrict__ ds, const float *__restrict__ x, float *__restrict__ y,
+    uint32_t m, uint32_t nb, uint32_t n, uint32_t splits, float *__restrict__ part, uint32_t *__restrict__ tickets) {
+    constexpr uint32_t QB = KIND == FH_Q8_0 ? 32 : 16;
+    __shared__ float red[kCallWaves][16][64];
+    __shared__ uint32_t arrived;
+    const uint32_t tid = threadIdx.x, lane = tid % 64, r = lane % 32, h = lane / 32;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const uint32_t groups = (n + 31) / 32, g0 = blockIdx.x * TN, nb8 = (nb + 7) / 8;
+    // this split's pairs of blocks, dealt to the wavefronts in turn
+    const uint32_t pairs = (nb + 1) / 2, per = (pairs + splits - 1) / splits;
+    const uint32_t p0 = blockIdx.y * per, p1 = min(pairs, p0 + per);
+    const auto rx = make_rsrc(x, m * nb * 128);
+    __amdgpu_buffer_rsrc_t rq[TN], rd[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const bool live = g0 + j < groups;  // a tile past the product: every load reads 0
+        rq[j] = make_rsrc(qs + (size_t)(live ? g0 + j : 0) * nb * 32 * QB, live ? nb * 32 * QB : 0);
+        rd[j] = make_rsrc(ds + (size_t)(live ? g0 + j : 0) * nb8 * 256, live ? nb8 * 512 : 0);
+    }
+    struct Batch {
+        f32x4 x[MT][kCallKB][2][2];            // [row tile][block][k step][half of eight]
+        u32x4 q[TN][KIND == FH_Q8_0 ? 2 : 1];  // Q8_0: a block each; Q4_0: lane half h holds block h's
+        uint32_t d[TN];                        // the two blocks' scales
+    };
+    auto load = [&](Batch &b, uint32_t p) {
+        const uint32_t b0 = 2 * p;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            if constexpr (KIND == FH_Q8_0) {
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    b.q[j][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                              rq[j], (int)((b0 + i) * 1024 + r * 32 + 16 * h), 0, 0));
+            } else {
+                b.q[j][0] = __builtin_bit_cast(
+                    u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq[j], (int)(b0 * 512 + lane * 16), 0, 0));
+            }
+            b.d[j] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rd[j], (int)(r * 16 + (b0 / 8) * 512 + (b0 % 8) * 2), 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int kb = 0; kb < kCallKB; kb++)
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    // element 16 s + 8 h (Q4_0) or 16 h + 8 s (Q8_0) of the block; rows past m and
+                    // blocks past the row read 0
+                    const uint32_t e = KIND == FH_Q4_0 ? 16 * s + 8 * h : 16 * h + 8 * s;
+                    const uint32_t off = b0 + kb < nb ? (((i * 32 + r) * nb + b0 + kb) * 32 + e) * 4 : 0x80000000u;
+#pragma unroll
+                    for (int c = 0; c < 2; c++)
+                        b.x[i][kb][s][c] =
+                            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(off + 16 * c), 0, 0));
+                }
+    };
+    f32x16 acc[MT][TN];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) acc[i][j][q] = 0.0f;
+    uint32_t magic = 0x64006400u;
+    asm volatile("" : "+v"(magic));  // kept in a vector register for and_or
+    auto compute = [&](const Batch &b) {
+        f16x8 bf[TN][kCallKB][2];
+        float dv[TN][kCallKB];
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            if constexpr (KIND == FH_Q8_0) {
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++) {
+                    const u32x4 q = b.q[j][kb] ^ 0x80808080u;
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        bf[j][kb][s] = __builtin_bit_cast(
+                            f16x8, u32x4{q8_pair(q[2 * s], 0x04020400u), q8_pair(q[2 * s], 0x04030401u),
+                                         q8_pair(q[2 * s + 1], 0x04020400u), q8_pair(q[2 * s + 1], 0x04030401u)});
+                }
+            } else {  // (the pair swap of rows_kernel)
+                const u32x4 q = b.q[j][0];
+                const auto s0 = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++) {
+                    const uint32_t w0 = s0[kb], w1 = s1[kb];
+                    bf[j][kb][0] = __builtin_bit_cast(f16x8, u32x4{q4_pair(w0, magic), q4_pair(w0 >> 8, magic),
+                                                                   q4_pair(w1, magic), q4_pair(w1 >> 8, magic)});
+                    bf[j][kb][1] = __builtin_bit_cast(f16x8, u32x4{q4_pair(w0 >> 4, magic), q4_pair(w0 >> 12, magic),
+                                                                   q4_pair(w1 >> 4, magic), q4_pair(w1 >> 12, magic)});
+                }
+            }
+            dv[j][0] = half_to_float(b.d[j] & 0xffffu);
+            dv[j][1] = half_to_float(b.d[j] >> 16);
+        }
+#pragma unroll
+        for (int kb = 0; kb < kCallKB; kb++)
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                f16x8 hi[2], lo[2];
+#pragma unroll
+                for (int s = 0; s < 2; s++) split_frag(b.x[i][kb][s][0], b.x[i][kb][s][1], hi[s], lo[s]);
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    f32x16 p = {};
+                    p = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[0], bf[j][kb][0], p, 0, 0, 0);
+                    p = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[1], bf[j][kb][1], p, 0, 0, 0);
+                    p = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[0], bf[j][kb][0], p, 0, 0, 0);
+                    p = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[1], bf[j][kb][1], p, 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 16; q++) acc[i][j][q] = fmaf(dv[j][kb], p[q], acc[i][j][q]);
+                }
+            }
+    };
+    Batch cur, nxt;
+    uint32_t p = p0 + wave;
+    if (p < p1) load(cur, p);
+    for (; p < p1; p += kCallWaves) {
+        const bool more = p + kCallWaves < p1;
+        if (more) load(nxt, p + kCallWaves);
+        compute(cur);
+        if (more) cur = nxt;
+    }
+    // The wavefronts' sums in order, tile by tile: thread t adds registers t / 64 and t / 64 + 8 of lane
+    // t % 64 (C layout: register q of lane l is row 8 (q / 4) + 4 (l / 32) + q % 4, output l % 32)
+    float sum[MT][TN][2];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            if (i + j) __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 16; q++) red[wave][q][lane] = acc[i][j][q];
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                float t = red[0][wave + 8 * c][lane];
+#pragma unroll
+                for (int w = 1; w < kCallWaves; w++) t += red[w][wave + 8 * c][lane];
+                sum[i][j][c] = t;
+            }
+        }
+    if (splits > 1) {
+        constexpr uint32_t N = MT * TN * 2;
+        float *mine = part + ((size_t)blockIdx.x * splits) * (N * 512);
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+                    agent_store(mine + (size_t)blockIdx.y * (N * 512) + ((i * TN + j) * 2 + c) * 512 + tid, sum[i][j][c]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the sums have landed
+        __syncthreads();
+        if (tid == 0)
+            arrived = __hip_atomic_fetch_add((gl_u32 *)(tickets + blockIdx.x), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (arrived + 1 != splits) return;  // (the whole workgroup)
+        if (tid == 0)
+            __hip_atomic_store((gl_u32 *)(tickets + blockIdx.x), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    const float *src = mine + ((i * TN + j) * 2 + c) * 512 + tid;
+                    float t = 0.0f;
+                    for (uint32_t s = 0; s < splits; s++) t += agent_load(src + (size_t)s * (N * 512));
+                    sum[i][j][c] = t;
+                }
+    }
+    typedef __attribute__((address_space(1))) float gfloat;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const uint32_t q = wave + 8 * c, row = i * 32 + 8 * (q / 4) + 4 * h + q % 4, col = (g0 + j) * 32 + r;
+                if (row < m && col < n) ((gfloat *)y)[(size_t)row * n + col] = sum[i][j][c];
+            }
+}
+
+struct CallPlan {
+    uint32_t tn, wgs, splits;
+};
+// Outputs per workgroup: 32, or 64 where 32 would make more than one workgroup per CU (each repeats the
+// x split: 896 x 9728 at 24 rows 9.4 us with 32, 7.8 with 64). K splits: up to one workgroup per CU,
+// each wavefront keeping at least one pair of blocks.
+CallPlan call_plan(size_t k, size_t n, int cus) {
+    const size_t groups = (n + 31) / 32, c = cus > 0 ? (size_t)cus : 256;
+    CallPlan p;
+    p.tn = groups > c ? 2 : 1;
+    p.wgs = (uint32_t)((groups + p.tn - 1) / p.tn);
+    const size_t most = std::min<size_t>(std::min<size_t>(k / 32 / (2 * kCallWaves), c / p.wgs), 8);
+    p.splits = (uint32_t)std::max<size_t>(most, 1);
+    return p;
+}
+
+template <int KIND>
+hipError_t launch_rows_call_kind(hipStream_t s, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                                 uint32_t m, uint32_t nb, uint32_t n, const CallPlan &p, float *part, uint32_t *tickets) {
+    const dim3 grid(p.wgs, p.splits);
+    if (m <= 32 && p.tn == 1)
+        rows_call_kernel<KIND, 1, 1><<<grid, 512, 0, s>>>(qs, ds, x, y, m, nb, n, p.splits, part, tickets);
+    else if (m <= 32)
+        rows_call_kernel<KIND, 1, 2><<<grid, 512, 0, s>>>(qs, ds, x, y, m, nb, n, p.splits, part, tickets);
+    else if (p.tn == 1)
+        rows_call_kernel<KIND, 2, 1><<<grid, 512, 0, s>>>(qs, ds, x, y, m, nb, n, p.splits, part, tickets);
+    else
+        rows_call_kernel<KIND, 2, 2><<<grid, 512, 0, s>>>(qs, ds, x, y, m, nb, n, p.splits, part, tickets);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 bool rows_supported(size_t rows, size_t k, size_t n) {
@@ -430,6 +683,34 @@ bool rows_supported(size_t rows, size_t k, size_t n) {
     const size_t nb = k / 32;
     return rows >= 1 && rows <= kRowsMax && nb > 0 && rows * nb * 128 < ((size_t)1 << 31) &&
            nb * 32 * 32 < ((size_t)1 << 31) && (n + 31) / 32 * 32 <= ((size_t)1 << 30);
+}
+
+// Where the one-launch kernel is the faster one for a single product (us, Q4_0, this kernel / rows_kernel
+// and its split / the precise GEMM): up to 32 rows while its workgroups run at once (24 rows: 896 x 1152
+// 5.9 / 13.2 / 15.9, 4864 x 896 11.0 / 27.8 / 31.6, 2048 x 11264, 176 workgroups, 13.0 / 16.3 / 25.8; but
+// 2048 x 20000, 313 workgroups, 24.0 / 20.4 / 28.6); past 32 rows, with twice the x to split, also up to
+// 64 tile blocks per CU (48 rows: 896 x 9728 14.8 / 18.7 / 21.8, 5632 x 2048 20.1 / 45.2 / 31.1; but
+// 2048 x 11264 23.8 / 22.7 / 28.5). k <= 16384 keeps the K splits' scratch small.
+bool rows_call_fits(size_t rows, size_t k, size_t n, int cus) {
+    if (rows < 2 || rows > kRowsMax || !rows_supported(rows, k, n) || k > 16384) return false;
+    const size_t c = cus > 0 ? (size_t)cus : 256;
+    const CallPlan p = call_plan(k, n, cus);
+    return p.wgs <= c && p.wgs <= kTicketCount && (rows <= 32 || k / 32 * ((n + 31) / 32) <= 64 * c);
+}
+
+size_t rows_call_scratch_bytes(size_t rows, size_t k, size_t n, int cus) {
+    const CallPlan p = call_plan(k, n, cus);
+    return p.splits > 1 ? (size_t)p.wgs * p.splits * p.tn * (rows > 32 ? 2 : 1) * 4096 : 0;
+}
+
+hipError_t launch_rows_call(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                            size_t rows, size_t k, size_t n, void *scratch, uint32_t *tickets, int cus) {
+    const CallPlan p = call_plan(k, n, cus);
+    if (kind == FH_Q8_0)
+        return launch_rows_call_kind<FH_Q8_0>(s, qs, ds, x, y, (uint32_t)rows, (uint32_t)(k / 32), (uint32_t)n, p,
+                                              (float *)scratch, tickets);
+    return launch_rows_call_kind<FH_Q4_0>(s, qs, ds, x, y, (uint32_t)rows, (uint32_t)(k / 32), (uint32_t)n, p,
+                                          (float *)scratch, tickets);
 }
 
 size_t rows_xsplit_bytes(size_t rows, size_t k) { return rows * (k / 32) * 128; }

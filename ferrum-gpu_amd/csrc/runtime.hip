@@ -124,6 +124,7 @@ void dev_release(fh_device *dev) {
     (void)hipSetDevice(dev->ordinal);
     (void)hipStreamSynchronize(dev->stream);
     if (dev->ws) (void)hipFree(dev->ws);
+    (void)hipFree(dev->tickets);
     (void)hipStreamDestroy(dev->stream);
     delete dev;
 }
@@ -371,6 +372,14 @@ fh_status fh_device_open(int ordinal, fh_device **out) {
         (void)hipStreamDestroy(d->stream);
         delete d;
         return hip_fail(nullptr, e, "kernel LDS limits");
+    }
+    if ((e = hipMalloc((void **)&d->tickets, kTicketCount * 4)) != hipSuccess ||
+        (e = hipMemsetAsync(d->tickets, 0, kTicketCount * 4, d->stream)) != hipSuccess ||
+        (e = hipStreamSynchronize(d->stream)) != hipSuccess) {
+        (void)hipFree(d->tickets);
+        (void)hipStreamDestroy(d->stream);
+        delete d;
+        return hip_fail(nullptr, e, "device tickets");
     }
     *out = d;
     return FH_OK;
@@ -751,8 +760,16 @@ static fh_status command_scratch(fh_device *dev, void *fixed, size_t bytes, void
 
 static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, float *y, size_t rows,
                         fh_path path, void *fixed = nullptr) {
-    if (path == FH_PATH_AUTO) path = fh_choose(rows, w->kind, w->k, w->n);
     fh_status st;
+    if (path == FH_PATH_AUTO && kind_ok(w->kind) && rows_call_fits(rows, w->k, w->n, dev->cus)) {  // one launch
+        void *part = nullptr;
+        const size_t bytes = rows_call_scratch_bytes(rows, w->k, w->n, dev->cus);
+        if (bytes && (st = command_scratch(dev, fixed, bytes, &part))) return st;
+        if ((st = begin_command(dev, "linear_q"))) return st;
+        (void)launch_rows_call(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, part, dev->tickets, dev->cus);
+        return end_command(dev, "linear_q");
+    }
+    if (path == FH_PATH_AUTO) path = fh_choose(rows, w->kind, w->k, w->n);
     if (ext_kind(w->kind)) {  // decoded on the fly (formats.hip; the multi-row MFMA GEMM in gemm.hip)
         if (path != FH_PATH_NAIVE && path != FH_PATH_GEMV && path != FH_PATH_TILED)
             return fail(FH_ERR_UNSUPPORTED, "kernel path %d does not take %s weights", (int)path, ext_label(w->kind));

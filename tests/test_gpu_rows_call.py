@@ -1,0 +1,53 @@
+"""AUTO's one-launch few-row product (2 to 64 rows, one linear_q per product) against the float64
+product of the stored weights, every output held to the summation error bound of any order (as
+test_gpu_rows.py: (k + 8) 2^-24 sum_k |x_k w_k|).
+
+Sizes: one and two 32-row tiles and their edges; block counts below a wavefront's pair, odd, not a
+multiple of the eight wavefronts' pairs, and deep enough to split K over workgroups (with a remainder);
+outputs that are not whole tiles, one and two tiles per workgroup (past 512 tiles); x at a 4-byte
+offset. Each product runs twice with another between them: the K splits' tickets must be left at zero
+and the sums must not depend on which workgroup ends last."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def fh():
+    import ferrum_hip
+
+    return ferrum_hip
+
+
+@pytest.fixture(scope="module")
+def g(fh):
+    gpu = fh.Gpu.open_for_test()
+    if gpu is None:
+        pytest.skip("no gfx950 device")
+    yield gpu
+    gpu.close()
+
+
+@pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
+@pytest.mark.parametrize("k,n", [(32, 1), (96, 33), (544, 300), (1056, 40), (4864, 100), (3104, 257), (64, 16450)])
+def test_one_launch_product(fh, g, orc, kind_name, k, n):
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(k + n)
+    b = orc.quantise_matrix(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32), k, n)
+    w = orc.dequantised_in_out(int(kind), b, k, n).reshape(k, n).astype(np.float64)
+    qw = fh.upload_qweight(g, kind, b, k, n)
+    for m in (2, 3, 31, 32, 33, 64):
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        gx, gy = g.upload(np.concatenate([[0.0], x.reshape(-1)])), g.zeros(m * n)
+        other = g.zeros(m * n)
+        fh.linear_q_ptr(g, gx.device_ptr() + 4, qw, gy.device_ptr(), m)
+        first = g.read(gy)
+        fh.linear_q_ptr(g, gx.device_ptr(), qw, other.device_ptr(), m)
+        fh.linear_q_ptr(g, gx.device_ptr() + 4, qw, gy.device_ptr(), m)
+        got = g.read(gy)
+        assert np.array_equal(first.view(np.uint32), got.view(np.uint32)), (kind_name, k, n, m)
+        bound = (k + 8) * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(w))
+        err = np.abs(got.reshape(m, n) - x.astype(np.float64) @ w)
+        assert np.all(err <= bound), (kind_name, k, n, m, float((err / np.maximum(bound, 1e-38)).max()))
+        print(f"{kind_name} {k}x{n} rows {m}: {float((err / np.maximum(bound, 1e-38)).max()):.3f} of the bound", flush=True)
