@@ -9,8 +9,9 @@
 // block's exact dot product by the block's f32 scale after the matrix cores (acc += d * P), so
 // the weights carry no rounding; they differ in how finely x is carried:
 //
-// gemm_precise_kernel (FH_PATH_TILED, within the reference's 1e-5 product tolerance,
-// ferrum_wgpu/src/tolerance.rs:7): x = hi + lo, two f16 parts (about 22 bits), split once per
+// The precise kernels (FH_PATH_TILED, within the reference's 1e-5 product tolerance,
+// ferrum_wgpu/src/tolerance.rs:7; gemm_stream_precise_kernel here and gemm_ring_kernel in
+// gemm_ring.hip, gemm_precise_kernel for what is too large for both): x = hi + lo, two f16 parts (about 22 bits), split once per
 // element by split_x_precise_kernel; per 32 x 32 tile and block four v_mfma_f32_32x32x16_f16.
 //
 // gemm_kernel (FH_PATH_TILED_FAST, the scoring GEMM, within |g - w| <= 1e-3 + 2e-3 |w|): x = hi
@@ -33,20 +34,12 @@
 #include <type_traits>
 
 #include "device_common.hpp"
+#include "gemm_parts.hpp"
 #include "internal.hpp"
 #include "xsplit.hpp"
 
 namespace fh {
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ float half_to_float(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
-}
 
 // A raw buffer resource over [base, base + bytes): loads at offsets at or past `bytes` return 0.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, uint32_t bytes) {
@@ -158,7 +151,8 @@ __global__ __launch_bounds__(256) void make_b8_kernel(const uint8_t *__restrict_
 
 // ---- x -> (hi, lo) f16, per block in operand order: xs[m][b] = 32 hi halves then 32 lo ----
 // Eight lanes per (row, block), lane j loading elements 4j..4j+3 (a wavefront reads 1 KiB of
-// contiguous x per instruction). |x| beyond the f16 range saturates hi (|x| < 65504 is exact).
+// contiguous x per instruction). |x| beyond the f16 range saturates hi (|x| < 65504 is exact). zero: floats
+// a product with two K splits adds into.
 __device__ __forceinline__ void split1(float e, _Float16 &h, _Float16 &l) {
     h = (_Float16)fminf(fmaxf(e, -65504.0f), 65504.0f);
     l = (_Float16)(e - (float)h);
@@ -166,8 +160,9 @@ __device__ __forceinline__ void split1(float e, _Float16 &h, _Float16 &l) {
 
 template <int KIND>
 __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__restrict__ x, _Float16 *__restrict__ xs,
-                                                      size_t items) {
+                                                      size_t items, float *__restrict__ zero, size_t zeros) {
     const int j = threadIdx.x % 8;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < zeros; i += (size_t)gridDim.x * 256) zero[i] = 0.0f;
     for (size_t t = ((size_t)blockIdx.x * 256 + threadIdx.x) / 8; t < items; t += (size_t)gridDim.x * 32) {
         const f32x4 v = __builtin_nontemporal_load((const f32x4 *)(x + t * 32) + j);
         _Float16 *out = xs + t * 64;
@@ -220,11 +215,6 @@ __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__res
 }
 
 // ---- weight quants -> f16 pairs in operand order ----
-__device__ __forceinline__ uint32_t f16x2_add(uint32_t w, _Float16 bias) {
-    const f16x2 v = __builtin_bit_cast(f16x2, w) + f16x2{bias, bias};
-    return __builtin_bit_cast(uint32_t, v);
-}
-
 // 16 quant bytes of a Q4_0 block -> its 32 elements as f16, positions 0..31 (8 per dword).
 __device__ __forceinline__ void unpack_q4(const u32x4 q, u32x4 (&out)[4]) {
 #pragma unroll
@@ -851,16 +841,9 @@ __global__ __launch_bounds__(256, 2) void gemm_precise_kernel(const _Float16 *__
         }
 }
 
-// The precise kernel's tile shape by rows and its K split (the rule of gemm_splits).
-void precise_tile(size_t rows, size_t *bm, size_t *bn) {
-    *bm = rows <= 32 ? 32 : rows <= 64 ? 64 : 128;
-    *bn = rows <= 32 ? 256 : 128;
-}
-
+// The K splits of its 128 x 128 tiles (the rule of gemm_splits).
 uint32_t precise_splits(size_t rows, size_t k, size_t n) {
-    size_t bm, bn;
-    precise_tile(rows, &bm, &bn);
-    const uint64_t tiles = (uint64_t)((rows + bm - 1) / bm) * ((n + bn - 1) / bn);
+    const uint64_t tiles = (uint64_t)((rows + 127) / 128) * ((n + 127) / 128);
     return gemm_splits(tiles, (uint32_t)((k / 32 + kBKB - 1) / kBKB));
 }
 
@@ -929,28 +912,6 @@ __device__ __forceinline__ void unpack_q4_half(uint32_t w0, uint32_t w1, u32x4 &
     }
     o0 = o[0];
     o1 = o[1];
-}
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
-
-// A raw buffer descriptor in scalar registers over [base, base + bytes) (the make_rsrc layout).
-__device__ __forceinline__ i32x4 sgpr_rsrc(const void *base, uint32_t bytes) {
-    const uint64_t a = (uint64_t)base;
-    return i32x4{__builtin_amdgcn_readfirstlane((int32_t)(uint32_t)a),
-                 __builtin_amdgcn_readfirstlane((int32_t)((uint32_t)(a >> 32) & 0xffffu)),
-                 __builtin_amdgcn_readfirstlane((int32_t)bytes), 0x00020000};
-}
-// 16 (4) bytes per lane from r at voff into LDS at lds + 16 (4) * lane; lds wave-uniform. An M0
-// write needs one wait state before a load that reads it.
-__device__ __forceinline__ void asm_load_lds16(i32x4 r, uint32_t lds, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(voff),
-                 "s"(r)
-                 : "m0");
-}
-__device__ __forceinline__ void asm_load_lds4(i32x4 r, uint32_t lds, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(r)
-                 : "m0");
 }
 
 // ---- the scoring head's score epilogue (both streaming kernels) ----
@@ -1688,14 +1649,40 @@ hipError_t run_gemm_stream_precise(hipStream_t s, const _Float16 *xs, const uint
     return hipGetLastError();
 }
 
+// Which kernel runs a precise product, and its K splits. The ring kernel (gemm_ring.hip) wherever its 32-bit
+// offsets reach, but the streaming kernel where its 256 x 256 tiles fill rounds of the chip better: about
+// 1.75 us a stage and round, 6 us of its own, and the reduction pass when K is split (4 bytes per output and
+// part at 4 TB/s). Measured, us, streaming / ring: 1024 x 2048 x 11264 149 / 123, 1500 rows 250 / 197, 4096 rows
+// 356 / 451; 2048 x 896 x 9728 107 / 121. The 128 x 128 kernel takes what is too large for both.
+struct PrecisePlan {
+    enum { STREAM, RING, TILES } kernel;
+    uint32_t splits;
+};
+PrecisePlan precise_plan(size_t rows, size_t k, size_t n) {
+    const bool ring = ring_supported(rows, k, n);
+    uint32_t sp = 1;
+    if (stream_plan(rows, k, n, &sp) && stream_supported(rows, k, n)) {
+        const uint64_t tiles = (uint64_t)((rows + 255) / 256) * ((n + 255) / 256), rounds = (tiles * sp + 255) / 256;
+        const float us = 1.75f * (float)rounds * (float)((k / 32 + sp - 1) / sp) + 6.0f +
+                         (sp > 1 ? (float)(sp + 1) * (float)rows * (float)n * 1e-6f : 0.0f);
+        if (!ring || ring_us(rows, k, n) > 0.98f * us) return {PrecisePlan::STREAM, sp};
+    }
+    if (ring) return {PrecisePlan::RING, ring_splits(rows, k, n)};
+    return {PrecisePlan::TILES, precise_splits(rows, k, n)};
+}
+
 template <int KIND>
 hipError_t gemm_precise_dispatch(hipStream_t s, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *y,
                                  float *partial, uint32_t M, uint32_t K, uint32_t N, SplitOut *defer) {
-    uint32_t sp = 1;
-    if (stream_plan(M, K, N, &sp) && stream_supported(M, K, N) && (sp == 1 || partial))
-        return run_gemm_stream_precise<KIND>(s, xs, qs, ds, y, partial, M, K, N, sp, defer);
-    if (M <= 32) return run_gemm_precise<KIND, 32, 256, 1>(s, xs, qs, ds, y, partial, M, K, N, defer);
-    if (M <= 64) return run_gemm_precise<KIND, 64, 128, 2>(s, xs, qs, ds, y, partial, M, K, N, defer);
+    const PrecisePlan p = precise_plan(M, K, N);
+    if (p.kernel == PrecisePlan::STREAM)
+        return run_gemm_stream_precise<KIND>(s, xs, qs, ds, y, partial, M, K, N, p.splits, defer);
+    if (p.kernel == PrecisePlan::RING) {
+        const bool parts = defer && p.splits > 1;
+        if (defer) *defer = parts ? SplitOut{partial, p.splits} : SplitOut{y, 1u};
+        return launch_gemm_ring(s, (fh_kind)KIND, xs, qs, ds, parts ? partial : y, M, K, N, p.splits,
+                                p.splits > 1 && !defer);
+    }
     return run_gemm_precise<KIND, 128, 128, 2>(s, xs, qs, ds, y, partial, M, K, N, defer);
 }
 
@@ -2742,9 +2729,9 @@ hipError_t launch_make_b8(hipStream_t s, fh_kind kind, const uint8_t *qs, const 
     return hipGetLastError();
 }
 
+// (Sized for a consumer that takes the ring kernel's two parts, which otherwise add into y.)
 size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n) {
-    uint32_t sp = precise_splits(rows, k, n), ssp = 1;
-    if (stream_plan(rows, k, n, &ssp) && stream_supported(rows, k, n)) sp = max(sp, ssp);
+    const uint32_t sp = precise_plan(rows, k, n).splits;
     return sp > 1 ? (size_t)sp * rows * n * 4 : 0;
 }
 
@@ -2763,12 +2750,14 @@ hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, c
         partial = (float *)((uint8_t *)workspace + (rows * k * 4 + 255) / 256 * 256);
     const size_t items = rows * (k / 32);
     const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
+    const PrecisePlan plan = precise_plan(rows, k, n);  // two ring splits add into y, zeroed by the x split
+    const size_t zeros = plan.kernel == PrecisePlan::RING && plan.splits > 1 && !defer ? rows * n : 0;
     if (kind == FH_Q8_0) {
-        if (x) split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items);
+        if (x) split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
         return gemm_precise_dispatch<FH_Q8_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                               defer);
     }
-    if (x) split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items);
+    if (x) split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
     return gemm_precise_dispatch<FH_Q4_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                           defer);
 }
@@ -2790,7 +2779,7 @@ hipError_t launch_gemm_ext(hipStream_t s, int kind, const uint8_t *w, const floa
                          : nullptr;
     const size_t items = rows * (k / 32);
     const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
-    split_x_precise_kernel<0><<<g, 256, 0, s>>>(x, xs, items);
+    split_x_precise_kernel<0><<<g, 256, 0, s>>>(x, xs, items, nullptr, 0);
     const uint32_t M = (uint32_t)rows, K = (uint32_t)k, N = (uint32_t)n;
     switch (kind) {
     case FH_F16: return gemm_ext_dispatch<FH_F16>(s, xs, w, y, partial, M, K, N);
@@ -2952,10 +2941,10 @@ hipError_t launch_gemm_score(hipStream_t s, fh_path path, fh_kind kind, const ui
     const size_t items = rows * (k / 32);
     const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
     if (kind == FH_Q8_0) {
-        split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items);
+        split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, nullptr, 0);
         return run_gemm_score<FH_Q8_0>(s, path, xs, nullptr, nullptr, qs, ds, nullptr, nullptr, M, K, N, so);
     }
-    split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items);
+    split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, nullptr, 0);
     return run_gemm_score<FH_Q4_0>(s, path, xs, nullptr, nullptr, qs, ds, nullptr, nullptr, M, K, N, so);
 }
 

@@ -1,0 +1,53 @@
+"""The ring kernel of the precise GEMM (QPath.Tiled below the streaming kernel's sizes) against the
+float64 product of the stored weights, every output held to the summation error bound of any order (as
+test_gpu_rows.py: (k + 8) 2^-24 sum_k |x_k w_k|).
+
+Sizes: one block of K and block counts that are not a multiple of the wavefront groups (some groups then
+add zeros), fewer than the ring's depth, and deep enough for two K splits that add into y (run twice:
+the same bits whichever lands first); row tiles of 32 and 64 and their edges; columns below, at and past a
+wavefront's 64 and the two tile widths; shapes whose plan takes the 256-column tiles."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def fh():
+    import ferrum_hip
+
+    return ferrum_hip
+
+
+@pytest.fixture(scope="module")
+def g(fh):
+    gpu = fh.Gpu.open_for_test()
+    if gpu is None:
+        pytest.skip("no gfx950 device")
+    yield gpu
+    gpu.close()
+
+
+@pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
+@pytest.mark.parametrize("k,n,rows", [(32, 1, (2, 33)), (96, 65, (31, 32, 33, 65)), (160, 129, (64, 130)),
+                                      (512, 300, (5, 40, 129)), (1056, 257, (33, 64, 200)), (4896, 127, (17, 100)),
+                                      (896, 9728, (300,)), (2048, 2560, (1024,))])
+def test_ring_product(fh, g, orc, kind_name, k, n, rows):
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(k + n)
+    b = orc.quantise_matrix(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32), k, n)
+    w = orc.dequantised_in_out(int(kind), b, k, n).reshape(k, n).astype(np.float64)
+    qw = fh.upload_qweight(g, kind, b, k, n)
+    for m in rows:
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        gx, gy = g.upload(x), g.upload(np.full(m * n, np.nan, np.float32))
+        fh.linear_q_with(g, gx, qw, gy, m, fh.QPath.Tiled)
+        first = g.read(gy)
+        fh.linear_q_with(g, gx, qw, gy, m, fh.QPath.Tiled)
+        got = g.read(gy)
+        assert np.array_equal(first.view(np.uint32), got.view(np.uint32)), (kind_name, k, n, m)
+        bound = (k + 8) * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(w))
+        err = np.abs(got.reshape(m, n) - x.astype(np.float64) @ w)
+        worst = float((err / np.maximum(bound, 1e-38)).max())
+        print(f"{kind_name} {m} x {k} x {n}: {worst:.3f} of the bound", flush=True)
+        assert np.all(err <= bound), (kind_name, k, n, m, worst)
