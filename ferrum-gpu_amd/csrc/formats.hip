@@ -461,24 +461,23 @@ __global__ __launch_bounds__(256) void ext_gemv_kernel(const uint8_t *__restrict
 }
 
 // ---- batch-1 GEMV on resident rows, the one-row path ----
-// A lane takes whole segments of a row (F16: 8 elements, FP8: 16, MXFP4: a block of 32, Q2_K: 32
-// elements of one half super-block), loads the segment's x once and uses it for R rows (1, 2, 4 or
-// 8), decodes the weights in registers and accumulates in f32: per segment the block's integer-valued
-// codes are summed against x and the block scale is applied once (FP8 and Q2_K: the scale times
-// the segment's sum, MXFP4: the power-of-two scale likewise). L lanes share a group of rows
-// (segments l, l + L, ...), summed by shuffles and, for L > 64, through LDS. Rows are GGUF rows
-// of B-byte blocks at any byte offset: a segment that is not 4-byte aligned is loaded as the
-// dwords around it and realigned with v_alignbyte (allocations carry 256 zero bytes past their
-// end, so the last block's over-read stays inside its buffer).
+// A lane takes whole segments of a row (8 elements; Q2_K: 32 elements of one half super-block), loads the
+// segment's x once and uses it for R rows (1, 2, 4 or 8), decodes the weights in registers and
+// accumulates in f32: per segment the block's integer-valued codes are summed against x and the block
+// scale is applied once (FP8 and Q2_K: the scale times the segment's sum, MXFP4: the power-of-two scale
+// likewise). L lanes share a group of rows (segments l, l + L, ...), summed by shuffles and, for L > 64,
+// through LDS. Rows are GGUF rows of B-byte blocks at any byte offset.
+// What bounds it for the formats below 8 bits is not HBM but the vector memory pipeline: a wavefront's load
+// takes a cycle per cache line that its lanes touch. With a whole MXFP4 block (32 elements) per lane every
+// x load touched 64 lines, 512 cycles a block row against 96 for its 17 bytes of weights; a quarter
+// block per lane puts four lanes on a line (TinyLlama layer, one row, four calls: 25.9 -> 18.6 us; FP8,
+// which took 16 elements a lane, 20.1 -> 19.0 us).
 
 __device__ __forceinline__ uint32_t ld32(const uint8_t *p) { return *(const uint32_t *)p; }
-// bytes [p, p + 16) for any p: five dwords from p rounded down, realigned
-__device__ __forceinline__ u32x4 ld16_any(const uint8_t *p) {
-    const uint32_t sh = (uint32_t)((uintptr_t)p & 3);
-    const uint8_t *q = p - sh;  // derived from p, so the loads stay global ones
-    const uint32_t d0 = ld32(q), d1 = ld32(q + 4), d2 = ld32(q + 8), d3 = ld32(q + 12), d4 = ld32(q + 16);
-    return u32x4{__builtin_amdgcn_alignbyte(d1, d0, sh), __builtin_amdgcn_alignbyte(d2, d1, sh),
-                 __builtin_amdgcn_alignbyte(d3, d2, sh), __builtin_amdgcn_alignbyte(d4, d3, sh)};
+// N dwords from any byte (one load: the hardware takes unaligned addresses)
+template <int N>
+__device__ __forceinline__ void ld_any(uint32_t (&v)[N], const uint8_t *p) {
+    __builtin_memcpy(v, p, 4 * N);
 }
 __device__ __forceinline__ float lo_half(uint32_t v) { return (float)__builtin_bit_cast(_Float16, (uint16_t)v); }
 __device__ __forceinline__ float hi_half(uint32_t v) {
@@ -491,7 +490,7 @@ struct ExtSeg;
 
 template <>
 struct ExtSeg<FH_F16> {  // segment s: halves 8 s .. 8 s + 7 of the row (16-byte aligned)
-    static constexpr uint32_t SPB = 4, XN = 8;
+    static constexpr uint32_t SPB = 4, XN = 8, XSTEP = 4;
     struct W {
         u32x4 q;
     };
@@ -508,26 +507,25 @@ struct ExtSeg<FH_F16> {  // segment s: halves 8 s .. 8 s + 7 of the row (16-byte
     }
 };
 
-// FP8 (fp8.rs:34-63): segment s = codes 16 p .. 16 p + 15 of block s / 2, p = s % 2, times the
+// FP8 (fp8.rs:34-63): segment s = codes 8 p .. 8 p + 7 of block s / 4, p = s % 4, times the
 // block's f16 scale. gfx950's conversions read OCP E4M3 / E5M2 (the reference's formats: E4M3
 // NaN at 0x7f and 0xff only, E5M2 with infinities), two codes per instruction.
 template <bool E5M2>
 struct Fp8Seg {
-    static constexpr uint32_t SPB = 2, XN = 16;
+    static constexpr uint32_t SPB = 4, XN = 8, XSTEP = 4;
     struct W {
-        uint32_t d;
-        u32x4 c;
+        uint32_t d, c[2];
     };
     __device__ static void load(const uint8_t *row, uint32_t s, W &w) {
-        const uint8_t *blk = row + 34 * (s / 2);
+        const uint8_t *blk = row + 34 * (s / 4);
         w.d = *(const uint16_t *)blk;
-        w.c = ld16_any(blk + 2 + 16 * (s % 2));
+        ld_any(w.c, blk + 2 + 8 * (s % 4));
     }
-    __device__ static uint32_t xat(uint32_t s) { return 16 * s; }
+    __device__ static uint32_t xat(uint32_t s) { return 8 * s; }
     __device__ static float dot(const W &w, const float (&x)[XN]) {
         float a = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < 2; i++) {
             const int v = (int)w.c[i];
             const auto p0 = E5M2 ? __builtin_amdgcn_cvt_pk_f32_bf8(v, false) : __builtin_amdgcn_cvt_pk_f32_fp8(v, false);
             const auto p1 = E5M2 ? __builtin_amdgcn_cvt_pk_f32_bf8(v, true) : __builtin_amdgcn_cvt_pk_f32_fp8(v, true);
@@ -544,41 +542,36 @@ struct ExtSeg<FH_FP8_E4M3> : Fp8Seg<false> {};
 template <>
 struct ExtSeg<FH_FP8_E5M2> : Fp8Seg<true> {};
 
-// MXFP4 (mxfp4.rs:13-33): segment = block s (E8M0 byte, then element i < 16 in the low nibble of
-// byte 1 + i, element 16 + i in its high nibble). gfx950's scaled FP4 conversion turns one byte
-// into its two E2M1 values (0, 0.5, 1, 1.5, 2, 3, 4, 6 and negatives: the reference's table halved),
-// so sum(x v) = 2 sum(x e2m1) exactly, then times the half scale.
+// MXFP4 (mxfp4.rs:13-33): segment = quarter p = s % 4 of block s / 4 (E8M0 byte, then element i < 16 in
+// the low nibble of byte 1 + i, element 16 + i in its high nibble): bytes 1 + 4 p .. 4 + 4 p, elements
+// 4 p .. 4 p + 3 and 16 + 4 p ... gfx950's scaled FP4 conversion turns one byte into its two E2M1 values
+// (0, 0.5, 1, 1.5, 2, 3, 4, 6 and negatives: the reference's table halved), so sum(x v) = 2 sum(x e2m1)
+// exactly, then times the half scale.
 template <>
 struct ExtSeg<FH_MXFP4> {
-    static constexpr uint32_t SPB = 1, XN = 32;
+    static constexpr uint32_t SPB = 4, XN = 8, XSTEP = 16;
     struct W {
-        uint32_t e;
-        u32x4 q;
+        uint32_t e, q[1];
     };
     __device__ static void load(const uint8_t *row, uint32_t s, W &w) {
-        const uint8_t *blk = row + 17 * s;
+        const uint8_t *blk = row + 17 * (s / 4);
         w.e = blk[0];
-        w.q = ld16_any(blk + 1);
+        ld_any(w.q, blk + 1 + 4 * (s % 4));
     }
-    __device__ static uint32_t xat(uint32_t s) { return 32 * s; }
+    __device__ static uint32_t xat(uint32_t s) { return 32 * (s / 4) + 4 * (s % 4); }
     __device__ static float dot(const W &w, const float (&x)[XN]) {
-        float a = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            // byte 4 i + b: elements 4 i + b (low nibble) and 16 + 4 i + b (high nibble)
-            const auto v0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[i], 1.0f, 0);
-            const auto v1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[i], 1.0f, 1);
-            const auto v2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[i], 1.0f, 2);
-            const auto v3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[i], 1.0f, 3);
-            a = fmaf(x[4 * i], v0[0], a);
-            a = fmaf(x[16 + 4 * i], v0[1], a);
-            a = fmaf(x[4 * i + 1], v1[0], a);
-            a = fmaf(x[16 + 4 * i + 1], v1[1], a);
-            a = fmaf(x[4 * i + 2], v2[0], a);
-            a = fmaf(x[16 + 4 * i + 2], v2[1], a);
-            a = fmaf(x[4 * i + 3], v3[0], a);
-            a = fmaf(x[16 + 4 * i + 3], v3[1], a);
-        }
+        const auto v0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[0], 1.0f, 0);
+        const auto v1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[0], 1.0f, 1);
+        const auto v2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[0], 1.0f, 2);
+        const auto v3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w.q[0], 1.0f, 3);
+        float a = x[0] * v0[0];
+        a = fmaf(x[4], v0[1], a);
+        a = fmaf(x[1], v1[0], a);
+        a = fmaf(x[5], v1[1], a);
+        a = fmaf(x[2], v2[0], a);
+        a = fmaf(x[6], v2[1], a);
+        a = fmaf(x[3], v3[0], a);
+        a = fmaf(x[7], v3[1], a);
         return (a * 2.0f) * mx_half_scale(w.e);
     }
 };
@@ -640,7 +633,7 @@ __device__ __forceinline__ void ext_load_x(const float *__restrict__ x, uint32_t
     } else {
 #pragma unroll
         for (int i = 0; i < (int)S::XN / 4; i++) {
-            const f32x4 a = *(const f32x4 *)(x + S::xat(s) + 4 * i);
+            const f32x4 a = *(const f32x4 *)(x + S::xat(s) + S::XSTEP * i);
 #pragma unroll
             for (int l = 0; l < 4; l++) xv[4 * i + l] = a[l];
         }
