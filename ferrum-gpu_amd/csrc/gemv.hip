@@ -310,6 +310,90 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
     }
 }
 
+// Products too wide for the LDS records (nb > kGemvLdsBlocks): a task's batches are dealt to the four
+// wavefronts of a workgroup, whose row sums meet in LDS in a fixed order. A wavefront per task left such a
+// launch with few wavefronts, each a chain of many batches: 24 products of 4864 x 896 are 672 tasks of 19
+// batches for the chip's 2048 wavefronts (20.7 -> 14.1 us, 2.9 -> 4.2 TB/s). Every wavefront streams its batches of
+// the workgroup's tasks as gemv_kernel does, the next one in flight across task boundaries and across
+// the barrier that ends each task.
+template <int KIND>
+__global__ __launch_bounds__(256) void gemv_wide_kernel(const GemvDesc *__restrict__ descs,
+                                                        const uint32_t *__restrict__ map, GemvDesc one, uint32_t count,
+                                                        uint32_t tasks, uint32_t per) {
+    constexpr uint32_t kStep = 4 * kBatch;
+    __shared__ float parts[2][4][32];
+    const int lane = threadIdx.x % 64, r = lane % 32;
+    const bool upper = lane >= 32;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t t0 = xcd_order(blockIdx.x, gridDim.x) * per, t1 = min(tasks, t0 + per);
+    if (t0 >= tasks) return;  // the whole workgroup
+    const LaneOffsets o{KIND == FH_Q8_0 ? (uint32_t)(r * 32 + 16 * upper) : (uint32_t)(lane * 16), (uint32_t)(r * 16),
+                        prep_a_offset(lane), prep_tail_offset<KIND>(lane)};
+    Cursor cur{descs, count, tasks, 0, 0, {}};
+    cur.seek(t0, map, one);
+    Task<KIND> ltk;
+    Pos lp{t0, kBatch * wv, t0 - cur.d.task0, cur.d.n, cur.d.nb, cur.d.y};
+    ltk.set(cur.d, lp.g);
+    auto advance = [&]() {
+        lp.b += kStep;
+        if (lp.b >= lp.nb) {
+            lp.t++;
+            lp.b = kBatch * wv;  // (nb > kStep: every wavefront has a batch of every task)
+            if (lp.t < t1) {
+                cur.advance(lp.t);
+                lp.g = lp.t - cur.d.task0;
+                lp.n = cur.d.n;
+                lp.nb = cur.d.nb;
+                lp.y = cur.d.y;
+                ltk.set(cur.d, lp.g);
+            } else {
+                ltk.clear(cur.d);
+            }
+        }
+    };
+    float acc = 0.0f;
+    // After computing batch cp: on the wavefront's last batch of a task, its row sums (even and odd blocks) to
+    // LDS; the task's wavefront t % 4 adds the four and stores the row.
+    auto finish = [&](const Pos &cp) {
+        if (cp.b + kStep < cp.nb) return;
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+        const float sum = acc + __uint_as_float(upper ? sw[0] : sw[1]);
+        if (!upper) parts[cp.t & 1][wv][r] = sum;
+        acc = 0.0f;
+        __syncthreads();  // (the other half of parts is read before the next task's barrier)
+        if (wv == (cp.t & 3) && !upper) {
+            const float *p = &parts[cp.t & 1][0][r];
+            const uint32_t row = cp.g * 32 + r;
+            if (row < cp.n) ((__attribute__((address_space(1))) float *)cp.y)[row] = (p[0] + p[32]) + (p[64] + p[96]);
+        }
+    };
+    auto compute = [&](const Batch<KIND> &b, const Pos &cp) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (cp.b + kBatch / 2 >= cp.nb)
+            compute_batch<KIND, kBatch / 4>(b, upper, acc);  // a task's last half batch
+        else
+            compute_batch<KIND>(b, upper, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        finish(cp);
+    };
+    Batch<KIND> b0, b1;
+    load_batch<KIND, false>(b0, ltk, lp.b, o, 0);
+    Pos cp = lp;
+    advance();
+    for (;;) {
+        load_batch<KIND, false>(b1, ltk, lp.b, o, 0);
+        compute(b0, cp);
+        if (lp.t >= t1) break;
+        cp = lp;
+        advance();
+        load_batch<KIND, false>(b0, ltk, lp.b, o, 0);
+        compute(b1, cp);
+        if (lp.t >= t1) break;
+        cp = lp;
+        advance();
+    }
+}
+
 // Wavefronts per CU a launch aims for (FERRUM_HIP_GEMV_WAVES_PER_CU overrides, 1..32), at most
 // what fits.
 uint32_t waves_per_cu() {
@@ -373,11 +457,31 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
                                                            (int)(4 * kMaxLdsBlocks * kPrepBytes));
         (void)attr;
     }
+    const uint32_t ncus = (uint32_t)(cus > 0 ? cus : 256);
+    if (max_nb > kMaxLdsBlocks) {  // (a launch of a plan holds only such products, or none)
+        static const int groups = [] {
+            int b = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, gemv_wide_kernel<KIND>, 256, 0) != hipSuccess || b < 1) b = 1;
+            return b;
+        }();
+        const uint32_t wper = (tasks + ncus * (uint32_t)groups - 1) / (ncus * (uint32_t)groups);
+        gemv_wide_kernel<KIND><<<(tasks + wper - 1) / wper, 256, 0, s>>>(descs, map, one, count, tasks, wper);
+        return hipGetLastError();
+    }
     // as many wavefronts as fit on the chip at once (or the requested per-CU count), each an
-    // equal share of the tasks
-    const int resident = 4 * (ldsx ? resident_groups<KIND, true>(lds_bytes) : resident_groups<KIND, false>(0));
-    const uint32_t per_cu = min((uint32_t)resident, waves_per_cu());
-    const uint32_t max_waves = (uint32_t)(cus > 0 ? cus : 256) * per_cu;
+    // equal share of the tasks; past the requested count, up to what fits, where that leaves less of the
+    // last round idle (8832 tasks: 5 each for 1767 of 2048 wavefronts, 3 each for 2944 of 3072)
+    const uint32_t resident = 4u * (uint32_t)(ldsx ? resident_groups<KIND, true>(lds_bytes) : resident_groups<KIND, false>(0));
+    uint32_t max_waves = 0;
+    float best = 0.0f;
+    for (uint32_t w = min(resident, waves_per_cu()); w <= resident; w += 4) {
+        const uint32_t waves = ncus * w, per = (tasks + waves - 1) / waves;
+        const float used = (float)tasks / (float)(per * waves);
+        if (used > 1.05f * best) {
+            best = used;
+            max_waves = waves;
+        }
+    }
     const uint32_t per = (tasks + max_waves - 1) / max_waves;
     const uint32_t waves = (tasks + per - 1) / per;
     if (ldsx)
