@@ -3,8 +3,8 @@
 // GGUF tensor order) and "cols" form (blocks running down the columns of an [in, out] matrix).
 // Bit-exact with ferrum_gguf/src/codec/quant.rs:50-136 and ferrum_ref/src/training/qat.rs:20-54.
 //
-// All of this is HBM-bound byte work. The rows kernels give each block to 8 lanes, each lane a
-// 16-byte f32x4 of the block, so a wavefront reads or writes 1 KiB of f32 per instruction,
+// All of this is HBM-bound byte work. The rows kernels (but the encode) give each block to 8 lanes, each
+// lane a 16-byte f32x4 of the block, so a wavefront reads or writes 1 KiB of f32 per instruction,
 // perfectly coalesced; the odd-sized packed side (34 or 18 bytes per block) is staged through
 // LDS so it, too, moves as aligned 16-byte chunks. The cols kernels map consecutive lanes to
 // consecutive columns, which makes the column walks coalesced across the wavefront.
@@ -33,105 +33,86 @@ struct Fmt<FH_Q4_0> {
     static constexpr int bytes = 18;
 };
 
-// Reduce over the 8 lanes of a block (lanes 8b..8b+7 of the wavefront).
-__device__ __forceinline__ float max8(float v) {
-    v = fmaxf(v, __shfl_xor(v, 1));
-    v = fmaxf(v, __shfl_xor(v, 2));
-    v = fmaxf(v, __shfl_xor(v, 4));
-    return v;
-}
-
-// The signed value of largest magnitude, the lowest index winning ties (the reference's strict
-// `>` fold from 0.0, quant.rs:123-126). `mine` is this lane's candidate for elements
-// 4j..4j+3; lanes are ordered by element index.
-__device__ __forceinline__ float argmax_abs8(float mine, int lane) {
+// The snap's quantisation step: from this lane's 4 values of a block held by 8 lanes, the 4 Q8_0 codes and the
+// f16 scale bits.
+__device__ __forceinline__ void quantise4(const f32x4 v, int32_t (&q)[4], uint32_t &h) {
+    const float amax = group_reduce<8>(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))), MaxOp());
+    const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+    h = float_to_half_bits(d);
 #pragma unroll
-    for (int s = 1; s < 8; s <<= 1) {
-        float other = __shfl_xor(mine, s);
-        bool lower = (lane & s) == 0;  // this lane's elements come first
-        float lo = lower ? mine : other, hi = lower ? other : mine;
-        mine = fabsf(hi) > fabsf(lo) ? hi : lo;
-    }
-    return mine;
-}
-
-// One quantisation step shared by encode and snap: from this lane's 4 values and the block's
-// statistics, the 4 quant codes (Q8_0: signed q; Q4_0: nibble 0..15) and the f16 scale bits.
-template <int KIND>
-__device__ __forceinline__ void quantise4(const f32x4 v, int lane, int32_t (&q)[4], uint32_t &h) {
-    if constexpr (KIND == FH_Q8_0) {
-        float amax = fmaxf(fmaxf(fmaxf(0.0f, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w));
-        amax = max8(amax);
-        float d = amax / 127.0f;
-        float id = d != 0.0f ? 1.0f / d : 0.0f;
-        h = float_to_half_bits(d);
-        q[0] = round_sat_i8(v.x * id);
-        q[1] = round_sat_i8(v.y * id);
-        q[2] = round_sat_i8(v.z * id);
-        q[3] = round_sat_i8(v.w * id);
-    } else {
-        float m = 0.0f;
-        if (fabsf(v.x) > fabsf(m)) m = v.x;
-        if (fabsf(v.y) > fabsf(m)) m = v.y;
-        if (fabsf(v.z) > fabsf(m)) m = v.z;
-        if (fabsf(v.w) > fabsf(m)) m = v.w;
-        m = argmax_abs8(m, lane);
-        float d = m / -8.0f;
-        float id = d != 0.0f ? 1.0f / d : 0.0f;
-        h = float_to_half_bits(d);
-        q[0] = trunc_clamp_0_15(v.x * id + 8.5f);
-        q[1] = trunc_clamp_0_15(v.y * id + 8.5f);
-        q[2] = trunc_clamp_0_15(v.z * id + 8.5f);
-        q[3] = trunc_clamp_0_15(v.w * id + 8.5f);
-    }
+    for (int i = 0; i < 4; i++) q[i] = round_sat_i8(v[i] * id);
 }
 
 // ---- encode, rows: f32[nblocks * 32] -> GGUF blocks ----
+// Two lanes per block, sixteen values a lane, 128 blocks per workgroup. What bounds it is the VALU: a block's
+// statistics, two divisions and the f16 conversion cost every lane of the block the same, so eight lanes
+// per block (4 values each) made them three quarters of the work (2048 x 5632: Q8_0 16.8 -> 11.0 us, Q4_0
+// 12.5 -> 10.0 us). A lane's values are 64 contiguous bytes, four cache lines of a wavefront's loads shared.
 template <int KIND>
 __global__ __launch_bounds__(kThreads) void encode_rows_kernel(const float *__restrict__ src,
                                                                uint8_t *__restrict__ dst,
                                                                size_t nblocks) {
     constexpr int BB = Fmt<KIND>::bytes;
-    constexpr int OUT = kTaskBlocks * BB;  // staged output bytes per task (16-byte multiple)
+    constexpr int kBlocks = kThreads / 2;
+    constexpr int OUT = kBlocks * BB;  // staged output bytes per task (16-byte multiple)
     __shared__ __attribute__((aligned(16))) uint8_t stage[OUT];
-    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const size_t ntasks = (nblocks + kTaskBlocks - 1) / kTaskBlocks;
+    const int tid = threadIdx.x, lb = tid / 2, half = tid % 2;
+    const size_t ntasks = (nblocks + kBlocks - 1) / kBlocks;
     for (size_t task = blockIdx.x; task < ntasks; task += gridDim.x) {
-        const size_t blk0 = task * kTaskBlocks;
-        f32x4 v[kUnroll];
+        const size_t blk0 = task * kBlocks, b = blk0 + lb;
+        f32x4 v[4];
 #pragma unroll
-        for (int u = 0; u < kUnroll; u++) {
-            size_t blk = blk0 + (size_t)(wave * kUnroll + u) * 8 + lane / 8;
-            v[u] = blk < nblocks ? __builtin_nontemporal_load((const f32x4 *)src + blk * 8 + lane % 8)
-                                 : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 4; i++)
+            v[i] = b < nblocks ? ((const f32x4 *)src)[b * 8 + half * 4 + i] : f32x4{0.f, 0.f, 0.f, 0.f};
+        uint8_t *blk = stage + lb * BB;
+        u32x4 w;  // the lane's sixteen codes, a byte each
+        uint32_t h;
+        if constexpr (KIND == FH_Q8_0) {
+            float amax = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 16; e++) amax = fmaxf(amax, fabsf(v[e / 4][e % 4]));
+            amax = group_reduce<2>(amax, MaxOp());
+            const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+            h = float_to_half_bits(d);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                w[i] = (round_sat_i8(v[i].x * id) & 0xff) | (round_sat_i8(v[i].y * id) & 0xff) << 8 |
+                       (round_sat_i8(v[i].z * id) & 0xff) << 16 | (uint32_t)round_sat_i8(v[i].w * id) << 24;
+        } else {
+            // the value of largest magnitude, the first of equals (quant.rs:123-126)
+            float m = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                if (fabsf(v[e / 4][e % 4]) > fabsf(m)) m = v[e / 4][e % 4];
+            const float o = dpp_mov<0xB1>(m), lo = half ? o : m, hi = half ? m : o;
+            m = fabsf(hi) > fabsf(lo) ? hi : lo;
+            const float d = m / -8.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+            h = float_to_half_bits(d);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                w[i] = trunc_clamp_0_15(v[i].x * id + 8.5f) | trunc_clamp_0_15(v[i].y * id + 8.5f) << 8 |
+                       trunc_clamp_0_15(v[i].z * id + 8.5f) << 16 | (uint32_t)trunc_clamp_0_15(v[i].w * id + 8.5f) << 24;
         }
         __syncthreads();  // the previous task's stage has been written out
+        if (half == 0) *(uint16_t *)blk = (uint16_t)h;
+        if constexpr (KIND == FH_Q8_0) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; u++) {
-            const int lb = (wave * kUnroll + u) * 8 + lane / 8;  // block within the task
-            const int j = lane % 8;
-            int32_t q[4];
-            uint32_t h;
-            quantise4<KIND>(v[u], lane, q, h);
-            uint8_t *blk = stage + lb * BB;
-            if (j == 0) *(uint16_t *)blk = (uint16_t)h;
-            if constexpr (KIND == FH_Q8_0) {
-                uint32_t w = (q[0] & 0xff) | (q[1] & 0xff) << 8 | (q[2] & 0xff) << 16 | (uint32_t)(q[3] & 0xff) << 24;
-                *(uint16_t *)(blk + 2 + 4 * j) = (uint16_t)w;
-                *(uint16_t *)(blk + 4 + 4 * j) = (uint16_t)(w >> 16);
-            } else {
-                // lanes j < 4 hold elements 4j.. (low nibbles), lane j + 4 the elements 16 + 4j..
-                uint32_t lo = q[0] | q[1] << 8 | q[2] << 16 | (uint32_t)q[3] << 24;
-                uint32_t hi = (uint32_t)__shfl_xor((int)lo, 4);
-                if (j < 4) {
-                    uint32_t w = lo | hi << 4;
-                    *(uint16_t *)(blk + 2 + 4 * j) = (uint16_t)w;
-                    *(uint16_t *)(blk + 4 + 4 * j) = (uint16_t)(w >> 16);
-                }
+            for (int i = 0; i < 4; i++) {
+                *(uint16_t *)(blk + 2 + 16 * half + 4 * i) = (uint16_t)w[i];
+                *(uint16_t *)(blk + 4 + 16 * half + 4 * i) = (uint16_t)(w[i] >> 16);
+            }
+        } else {
+            // lane 0 holds the low nibbles of bytes 0..15, lane 1 the high ones; each writes eight bytes
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const uint32_t mine = half ? w[2 + i] : w[i], other = dpp_mov<0xB1>(half ? w[i] : w[2 + i]);
+                const uint32_t bytes = half ? other | mine << 4 : mine | other << 4;
+                *(uint16_t *)(blk + 2 + 8 * half + 4 * i) = (uint16_t)bytes;
+                *(uint16_t *)(blk + 4 + 8 * half + 4 * i) = (uint16_t)(bytes >> 16);
             }
         }
         __syncthreads();
-        const size_t nvalid = nblocks - blk0 < (size_t)kTaskBlocks ? nblocks - blk0 : kTaskBlocks;
+        const size_t nvalid = nblocks - blk0 < (size_t)kBlocks ? nblocks - blk0 : kBlocks;
         const size_t valid = nvalid * BB;
         uint8_t *out = dst + blk0 * BB;
         for (int c = tid; c < OUT / 16; c += kThreads) {
@@ -139,7 +120,7 @@ __global__ __launch_bounds__(kThreads) void encode_rows_kernel(const float *__re
             if (off + 16 <= valid) {
                 *(u32x4 *)(out + off) = *(const u32x4 *)(stage + off);
             } else if (off < valid) {
-                for (size_t b = off; b < valid; b += 2) *(uint16_t *)(out + b) = *(const uint16_t *)(stage + b);
+                for (size_t p = off; p < valid; p += 2) *(uint16_t *)(out + p) = *(const uint16_t *)(stage + p);
             }
         }
     }
@@ -227,7 +208,7 @@ __global__ __launch_bounds__(kThreads) void snap_rows_kernel(const float *__rest
         for (int u = 0; u < kUnroll; u++) {
             int32_t q[4];
             uint32_t h;
-            quantise4<FH_Q8_0>(v[u], lane, q, h);
+            quantise4(v[u], q, h);
             float d = half_bits_to_float(h);
             f32x4 o = {d * (float)q[0], d * (float)q[1], d * (float)q[2], d * (float)q[3]};
             size_t blk = (g0 + u) * 8 + lane / 8;
@@ -500,7 +481,7 @@ __global__ __launch_bounds__(kThreads) void snap_group_kernel(const SnapDesc *__
             for (int u = 0; u < kUnroll; u++) {
                 int32_t q[4];
                 uint32_t h;
-                quantise4<FH_Q8_0>(v[u], lane, q, h);
+                quantise4(v[u], q, h);
                 const float dd = half_bits_to_float(h);
                 const f32x4 o = {dd * (float)q[0], dd * (float)q[1], dd * (float)q[2], dd * (float)q[3]};
                 const size_t blk = (g0 + u) * 8 + lane / 8;

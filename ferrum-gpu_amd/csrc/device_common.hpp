@@ -73,21 +73,24 @@ __device__ __forceinline__ uint32_t float_to_half_bits(float x) {
     return sign | (half + up);
 }
 
-// Rust `f as i8` after f32::round: round half away from zero, saturate, NaN -> 0.
+// f truncated toward zero to an integer, saturating, NaN -> 0 (what the instruction does; the C++ cast
+// leaves those cases undefined).
+__device__ __forceinline__ int32_t cvt_i32(float f) {
+    int32_t r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(f));
+    return r;
+}
+
+// Rust `f as i8` after f32::round: round half away from zero, saturate, NaN -> 0. The fraction of |f| is
+// exact; that of an infinity or NaN compares false.
 __device__ __forceinline__ int32_t round_sat_i8(float f) {
-    if (f != f) return 0;
-    float r = roundf(f);  // llvm.round: exact half-away-from-zero
-    r = fminf(fmaxf(r, -128.0f), 127.0f);
-    return (int32_t)r;
+    int32_t r = cvt_i32(f);
+    r += __builtin_amdgcn_fractf(fabsf(f)) >= 0.5f ? (int32_t)__float_as_uint(f) >> 31 | 1 : 0;
+    return min(max(r, -128), 127);
 }
 
 // Rust `(f as i32).clamp(0, 15)`: truncate toward zero, saturate, NaN -> 0, then clamp.
-__device__ __forceinline__ int32_t trunc_clamp_0_15(float f) {
-    if (f != f) return 0;
-    float t = truncf(f);
-    t = fminf(fmaxf(t, 0.0f), 15.0f);
-    return (int32_t)t;
-}
+__device__ __forceinline__ int32_t trunc_clamp_0_15(float f) { return min(max(cvt_i32(f), 0), 15); }
 
 // A GGUF block starts at an even byte offset. Load the dword-aligned window that holds it
 // (WORDS dwords starting at the block's offset rounded down to 4); the block's first byte is
