@@ -1,0 +1,73 @@
+"""The two-lanes-per-block encoders and the four-per-thread decoder against the oracle, byte for byte: part-filled
+workgroups (one block, one short of and one past a workgroup's 128), values at the midpoints of the code
+tables and one unit to either side, signed zeros, subnormal and huge scales, NaN and infinities."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+KINDS = ("Q8_0", "Q4_0", "F16", "Fp8E4M3", "Fp8E5M2", "Fp4")
+
+
+@pytest.fixture(scope="module")
+def fh():
+    import ferrum_hip
+
+    return ferrum_hip
+
+
+@pytest.fixture(scope="module")
+def g(fh):
+    gpu = fh.Gpu.open_for_test()
+    if gpu is None:
+        pytest.skip("no gfx950 device")
+    yield gpu
+    gpu.close()
+
+
+def blocks(nblocks, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((nblocks, 32)).astype(np.float32)
+    # a quarter of the blocks: midpoints of the code tables (eighths, for a block maximum that makes the scale a
+    # power of two), and their neighbours
+    grid = rng.integers(-96, 97, (nblocks, 32)).astype(np.float32) / np.float32(8)
+    grid[:, 0] = rng.choice(np.float32([12, 448, 57344, 127, 8, 7.999999]), nblocks)
+    step = rng.integers(-1, 2, (nblocks, 32))
+    grid = np.where(step < 0, np.nextafter(grid, np.float32(-np.inf)),
+                    np.where(step > 0, np.nextafter(grid, np.float32(np.inf)), grid)).astype(np.float32)
+    x = np.where((np.arange(nblocks) % 4 == 1)[:, None], grid, x)
+    x *= np.exp2(rng.integers(-6, 7, nblocks)).astype(np.float32)[:, None]
+    wide = np.arange(nblocks) % 8 == 2  # from subnormal to the largest floats
+    x[wide] *= np.exp2(rng.integers(-140, 120, wide.sum()).astype(np.float64)).astype(np.float32)[:, None]
+    x[rng.random(x.shape) < 0.05] = np.float32(-0.0)
+    x[np.arange(nblocks) % 8 == 6] *= np.float32(0)
+    return x
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_encode_and_decode_at_the_edges(fh, g, orc, kind):
+    kind = getattr(fh.QKind, kind)
+    for nblocks in (1, 2, 127, 128, 129, 1031):
+        x = blocks(nblocks, nblocks).reshape(-1)
+        want = orc.encode(int(kind), x)
+        packed = fh.encode(g, kind, g.upload(x), x.size)
+        got = g.read_bytes(packed)[: want.size]
+        assert np.array_equal(got, want), (kind, nblocks, np.flatnonzero(got != want)[:8])
+        back = orc.decode(int(kind), want, x.size)
+        dev = g.read(fh.decode(g, kind, packed, x.size))[: x.size]
+        nan = np.isnan(back)
+        assert np.array_equal(np.isnan(dev), nan)
+        assert np.array_equal(dev[~nan].view(np.uint32), back[~nan].view(np.uint32)), (kind, nblocks)
+
+
+@pytest.mark.parametrize("kind", ("Fp8E4M3", "Fp8E5M2", "Fp4"))
+def test_encode_of_nan_and_infinity(fh, g, orc, kind):
+    kind = getattr(fh.QKind, kind)
+    x = blocks(160, 3)
+    x[5, 3], x[5, 19], x[140, 31] = np.nan, -np.nan, np.nan
+    x[9, 0], x[77, 16], x[78, 1] = np.inf, -np.inf, -np.inf
+    x[78, 2] = np.nan
+    x[79] = np.nan
+    want = orc.encode(int(kind), x.reshape(-1))
+    got = g.read_bytes(fh.encode(g, kind, g.upload(x.reshape(-1)), x.size))[: want.size]
+    assert np.array_equal(got, want), np.flatnonzero(got != want)[:8] // (want.size // 160)
