@@ -194,14 +194,21 @@ __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__res
             *(f16x4 *)(out + 32 + 4 * j) = lo;
         } else {
             // positions 8i..8i+7 hold elements 4i + {0, 2, 1, 3} (lane i) and 16 + 4i + {0, 2, 1, 3}
-            // (lane i + 4): lane i < 4 writes the hi part of group i, lane i + 4 the lo part
+            // (lane i + 4); MXFP4: 4i, 16 + 4i, 4i + 1, 17 + 4i, ... (a byte's two elements side by side). Lane i < 4 writes the hi part of group i, lane i + 4 the lo part
             f32x4 o;
             o.x = __shfl_xor(v.x, 4, 8);
             o.y = __shfl_xor(v.y, 4, 8);
             o.z = __shfl_xor(v.z, 4, 8);
             o.w = __shfl_xor(v.w, 4, 8);
             const f32x4 a = j < 4 ? v : o, b = j < 4 ? o : v;  // elements 4i.. and 16 + 4i..
-            const float e[8] = {a.x, a.z, a.y, a.w, b.x, b.z, b.y, b.w};
+            const float e[8] = {a.x,
+                                KIND == FH_MXFP4 ? b.x : a.z,
+                                a.y,
+                                KIND == FH_MXFP4 ? b.y : a.w,
+                                KIND == FH_MXFP4 ? a.z : b.x,
+                                b.z,
+                                KIND == FH_MXFP4 ? a.w : b.y,
+                                b.w};
             f16x8 part;
 #pragma unroll
             for (int q = 0; q < 8; q++) {
@@ -1665,9 +1672,9 @@ PrecisePlan precise_plan(size_t rows, size_t k, size_t n) {
         const uint64_t tiles = (uint64_t)((rows + 255) / 256) * ((n + 255) / 256), rounds = (tiles * sp + 255) / 256;
         const float us = 1.75f * (float)rounds * (float)((k / 32 + sp - 1) / sp) + 6.0f +
                          (sp > 1 ? (float)(sp + 1) * (float)rows * (float)n * 1e-6f : 0.0f);
-        if (!ring || ring_us(rows, k, n) > 0.98f * us) return {PrecisePlan::STREAM, sp};
+        if (!ring || ring_us(FH_Q8_0, rows, k, n) > 0.98f * us) return {PrecisePlan::STREAM, sp};
     }
-    if (ring) return {PrecisePlan::RING, ring_splits(rows, k, n)};
+    if (ring) return {PrecisePlan::RING, ring_splits(FH_Q8_0, rows, k, n)};
     return {PrecisePlan::TILES, precise_splits(rows, k, n)};
 }
 
@@ -1680,7 +1687,7 @@ hipError_t gemm_precise_dispatch(hipStream_t s, const _Float16 *xs, const uint8_
     if (p.kernel == PrecisePlan::RING) {
         const bool parts = defer && p.splits > 1;
         if (defer) *defer = parts ? SplitOut{partial, p.splits} : SplitOut{y, 1u};
-        return launch_gemm_ring(s, (fh_kind)KIND, xs, qs, ds, parts ? partial : y, M, K, N, p.splits,
+        return launch_gemm_ring(s, KIND, xs, qs, ds, parts ? partial : y, M, K, N, p.splits,
                                 p.splits > 1 && !defer);
     }
     return run_gemm_precise<KIND, 128, 128, 2>(s, xs, qs, ds, y, partial, M, K, N, defer);
@@ -1777,9 +1784,6 @@ hipError_t run_gemm_score(hipStream_t s, fh_path path, const void *xa, const uin
 // dwords around it, realigned with v_alignbyte; allocations carry 256 zero bytes past their end)
 // into 32 f16 in LDS and the block's scale; the next stage's bytes are requested before the
 // current stage's MFMAs.
-__device__ __forceinline__ float e8m0_half_scale(uint32_t e) {  // mxfp4.rs:26-33
-    return e < 2 ? __uint_as_float(0x00200000u << e) : __uint_as_float((e - 1) << 23);
-}
 __device__ __forceinline__ uint32_t mx_biased(uint32_t n) {  // 4 nibbles (one per byte) -> value + 16 per byte
     const uint32_t m = n & 0x07070707u;
     const uint32_t pos = __builtin_amdgcn_perm(0x1c181614u, 0x13121110u, m);
@@ -2090,11 +2094,11 @@ __global__ __launch_bounds__(256, 2) void gemm_ext_kernel(const _Float16 *__rest
         }
 }
 
-// The other formats' GEMM tile (64-row tiles up to kMidRows rows, and always for Q2_K) and its K
-// split (the rule of gemm_splits over those tiles).
+// The other formats' GEMM tile (64-row tiles up to kMidRows rows, and always for Q2_K, whose products of up to 32
+// rows take 32-row ones; the other formats' come here only past the ring kernel's offsets) and its K split (the rule of gemm_splits over those tiles).
 void ext_tile(int kind, size_t rows, size_t *bm, size_t *bn) {
-    *bm = rows <= 32 ? 32 : (rows <= kMidRows || kind == FH_Q2_K) ? 64 : 128;
-    *bn = rows <= 32 ? 256 : 128;
+    *bm = rows <= 32 && kind == FH_Q2_K ? 32 : (rows <= kMidRows || kind == FH_Q2_K) ? 64 : 128;
+    *bn = *bm == 32 ? 256 : 128;
 }
 uint32_t ext_splits(int kind, size_t rows, size_t k, size_t n) {
     size_t bm, bn;
@@ -2128,9 +2132,12 @@ hipError_t gemm_ext_dispatch(hipStream_t s, const _Float16 *xs, const uint8_t *w
                              uint32_t M, uint32_t K, uint32_t N) {
     size_t bm, bn;
     ext_tile((int)T, M, &bm, &bn);  // (Q2_K's per-sub-block terms would spill in a 128-row tile)
-    if (bm == 32) return run_gemm_ext<T, 32, 256, 1>(s, xs, w, y, partial, M, K, N);
-    if (bm == 64) return run_gemm_ext<T, 64, 128, 2>(s, xs, w, y, partial, M, K, N);
-    return run_gemm_ext<T, 128, 128, 2>(s, xs, w, y, partial, M, K, N);
+    if constexpr (T == FH_Q2_K) {
+        if (bm == 32) return run_gemm_ext<T, 32, 256, 1>(s, xs, w, y, partial, M, K, N);
+    } else {
+        if (bm == 128) return run_gemm_ext<T, 128, 128, 2>(s, xs, w, y, partial, M, K, N);
+    }
+    return run_gemm_ext<T, 64, 128, 2>(s, xs, w, y, partial, M, K, N);
 }
 
 // ---- the dequant-f16 GEMM (FH_PATH_TILED_F16): weights dequantised into LDS, plain f16 MFMA ----
@@ -2766,7 +2773,28 @@ bool gemm_ext_kind(int kind) {
     return kind == FH_F16 || kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 || kind == FH_MXFP4 || kind == FH_Q2_K;
 }
 
+// Whether the ring kernel (gemm_ring.hip) takes the product: the formats other than Q2_K within its 32-bit offsets,
+// except where gemm_ext_kernel's tiles fill rounds of the chip better. Its time: two workgroups a CU, with 128-row
+// tiles 1.1 us a stage with one of them, 1.45 with both, with 64-row tiles 0.9, and 5 us of its own. Measured,
+// us, gemm_ext_kernel / ring: FP8 2048 x 11264 1024 rows 181 / 143, 2048 x 5632 2000 rows 173 / 146, 4096 rows 273 /
+// 283; 1024 x 2048 1024 rows 33 / 24, 4096 rows 58 / 67; F16 2048 x 5632 1024 rows 81 / 96, 700 rows 71 / 51.
+bool ext_ring(int kind, size_t rows, size_t k, size_t n) {
+    if (!ring_gguf_supported(kind, rows, k, n)) return false;
+    if (rows <= 32 || ext_splits(kind, rows, k, n) > 1) return true;
+    size_t bm, bn;
+    ext_tile(kind, rows, &bm, &bn);
+    const size_t tiles = (rows + bm - 1) / bm * ((n + bn - 1) / bn);
+    float stage = 0.9f * fmaxf((float)tiles / 512, 1.0f);  // a K step of all rounds
+    if (bm == 128) {
+        const float last = (float)(tiles % 512) / 256;
+        stage = 1.45f * (float)(tiles / 512) + (last > 0 ? 1.1f + 0.35f * fminf(fmaxf(last - 1, 0.0f), 1.0f) : 0.0f);
+        if (kind == FH_MXFP4) stage *= 0.95f;
+    }
+    return ring_us(kind, rows, k, n) <= stage * (float)(k / 32) + 5;
+}
+
 size_t gemm_ext_workspace_bytes(int kind, size_t rows, size_t k, size_t n) {
+    if (ext_ring(kind, rows, k, n)) return rows * k * 4;  // (its two K splits add into y)
     const uint32_t sp = ext_splits(kind, rows, k, n);
     return (rows * k * 4 + 255) / 256 * 256 + (sp > 1 ? (size_t)sp * rows * n * 4 : 0);
 }
@@ -2774,13 +2802,22 @@ size_t gemm_ext_workspace_bytes(int kind, size_t rows, size_t k, size_t n) {
 hipError_t launch_gemm_ext(hipStream_t s, int kind, const uint8_t *w, const float *x, float *y, size_t rows, size_t k,
                            size_t n, void *workspace) {
     _Float16 *xs = (_Float16 *)workspace;
+    const uint32_t M = (uint32_t)rows, K = (uint32_t)k, N = (uint32_t)n;
+    const size_t items = rows * (k / 32);
+    const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
+    if (ext_ring(kind, rows, k, n)) {
+        const uint32_t sp = ring_splits(kind, rows, k, n);
+        const size_t zeros = sp > 1 ? rows * n : 0;
+        if (kind == FH_MXFP4)
+            split_x_precise_kernel<FH_MXFP4><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+        else
+            split_x_precise_kernel<0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+        return launch_gemm_ring(s, kind, xs, w, nullptr, y, M, K, N, sp, sp > 1);
+    }
     float *partial = ext_splits(kind, rows, k, n) > 1
                          ? (float *)((uint8_t *)workspace + (rows * k * 4 + 255) / 256 * 256)
                          : nullptr;
-    const size_t items = rows * (k / 32);
-    const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
     split_x_precise_kernel<0><<<g, 256, 0, s>>>(x, xs, items, nullptr, 0);
-    const uint32_t M = (uint32_t)rows, K = (uint32_t)k, N = (uint32_t)n;
     switch (kind) {
     case FH_F16: return gemm_ext_dispatch<FH_F16>(s, xs, w, y, partial, M, K, N);
     case FH_FP8_E4M3: return gemm_ext_dispatch<FH_FP8_E4M3>(s, xs, w, y, partial, M, K, N);

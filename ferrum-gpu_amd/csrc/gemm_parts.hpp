@@ -16,6 +16,10 @@ __device__ __forceinline__ float half_to_float(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
 
+__device__ __forceinline__ float e8m0_half_scale(uint32_t e) {  // mxfp4.rs:26-33
+    return e < 2 ? __uint_as_float(0x00200000u << e) : __uint_as_float((e - 1) << 23);
+}
+
 __device__ __forceinline__ uint32_t f16x2_add(uint32_t w, _Float16 bias) {
     const f16x2 v = __builtin_bit_cast(f16x2, w) + f16x2{bias, bias};
     return __builtin_bit_cast(uint32_t, v);

@@ -22,14 +22,17 @@
 // loads, counted: loads complete in order) and the slot read in the stage before may be filled again.
 //
 // Measured (us, x split included, the 128 x 128 kernel and its reduction before / now, Q4_0): 512 rows 2048 x
-// 2560 35.8 / 28.1, 2048 x 2048 34.5 / 26.2, 2048 x 11264 99.8 / 71.0, 5632 x 2048 54.4 / 41.9, 896 x 1152
-// 28.0 / 15.3; 96 rows 2048 x 2560 27.2 / 16.2. A stage takes 0.99 us, 1,085 TFLOP/s of matrix-core work on
+// 2560 35.8 / 28.7, 2048 x 2048 34.5 / 26.2, 2048 x 11264 99.8 / 68.8, 5632 x 2048 54.4 / 41.2, 896 x 1152
+// 28.0 / 13.8; 96 rows 2048 x 2560 27.2 / 14.0. GGUF rows (gemm_ext_kernel, one stage ahead through registers,
+// before / now): FP8 2048 x 11264 300 rows 77 / 50, 1024 rows 181 / 144, 64 rows 30 / 23; MXFP4 69 / 47, 152 /
+// 131, 31 / 21; F16 69 / 47, 167 / 133, 28 / 18.5; 5632 x 2048 300 rows 52 / 40, 48 / 37, 48 / 38. A stage takes 0.99 us, 1,085 TFLOP/s of matrix-core work on
 // 256 CUs (a plain bf16 product reaches 1,210 on the card); what is left is a workgroup's own 6 us and the
 // last round.
 //
 // LDS: x row r of a slot keeps its 16-byte chunk c at c ^ ((r >> 1) & 7) (gemm.hip: the sixteen rows that
 // one cycle of a fragment read serves fall on sixteen different bank groups). Q8_0 quants are stored as
 // [half block][column][16 bytes], Q4_0 as [column][16 bytes].
+#include <algorithm>
 #include <cmath>
 
 #include "device_common.hpp"
@@ -39,17 +42,33 @@
 namespace fh {
 namespace {
 
+// The other formats' weights are GGUF rows (a block's scale and quants together, at 34- or 17-byte steps from any
+// byte; ds is null). A wavefront's part of a stage holds of each of its 64 columns the bytes from the block's
+// start, rounded down to a dword, on:
+//   FP8    [column][32 bytes], then [column][4]   F16 (a block is 64 codes' bytes, no scale) [column][64 bytes],
+//   MXFP4  [column][32 bytes]                     16-byte chunk c of a column at c ^ (column / 4) % 4
+// loaded 2 (F16: 4) lanes per column, since a load takes a cycle per cache line that it touches (a lane per column
+// would take 64 a load, 192 cycles of a stage's 2400 for each of eight wavefronts). In registers a lane shifts its
+// dwords to the byte with v_perm and the hardware converts the codes to f16, exactly.
+template <int KIND>
+constexpr bool kGguf = KIND != FH_Q8_0 && KIND != FH_Q4_0;
+template <int KIND>
+constexpr bool kFp8 = KIND == FH_FP8_E4M3 || KIND == FH_FP8_E5M2;
+template <int KIND>
+constexpr uint32_t kGgufBlock = kFp8<KIND> ? 34 : KIND == FH_MXFP4 ? 17 : 64;
+
 // KG groups of wavefronts share K (4 pairs and a 128-column tile, or 2 fours and a 256-column tile).
 template <int KIND, int MTW, int KG>
 struct Ring {
     static constexpr int WPG = 8 / KG, BN = 64 * WPG;  // wavefronts of a group
-    static constexpr uint32_t QB = KIND == FH_Q8_0 ? 32 : 16;
+    static constexpr uint32_t QB = KIND == FH_F16 ? 64 : KIND == FH_Q4_0 ? 16 : 32;
     static constexpr uint32_t X = 32 * MTW * 128;  // bytes of a group's stage: x,
     static constexpr uint32_t WQ = 64 * QB;        // a wavefront's quants
-    static constexpr uint32_t W = WQ + 256;        // and its scale dwords
+    static constexpr uint32_t D = KIND == FH_F16 || KIND == FH_MXFP4 ? 0 : 256;
+    static constexpr uint32_t W = WQ + D;          // and its scale (FP8: last) dwords
     static constexpr uint32_t GROUP = X + WPG * W, STAGE = KG * GROUP;
     static constexpr int XL = 4 * MTW / WPG;                         // x load instructions of a wavefront (1 KB each)
-    static constexpr int LOADS = XL + (KIND == FH_Q8_0 ? 2 : 1) + 1;  // load instructions per wavefront and stage
+    static constexpr int LOADS = XL + WQ / 1024 + D / 256;  // load instructions per wavefront and stage
     static constexpr int NS = 163840 / STAGE < 6 ? 163840 / STAGE : 6;
     static constexpr uint32_t SUMS = 8 * MTW * 8192;  // the wavefronts' sums (after the loop)
     static constexpr uint32_t LDS = NS * STAGE > SUMS ? NS * STAGE : SUMS;
@@ -89,9 +108,31 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
     const uint32_t woff = KIND == FH_Q8_0 ? g0 * nb * 1024 + (lane % 32) * 32 + (lane / 32) * 16
                                           : (g0 + lane / 32) * nb * 512 + (lane % 32) * 16;
     const uint32_t doff = (ncol >> 5) * nb8 * 512 + (ncol & 31) * 16;
+    // GGUF rows: the byte offset of what the lane loads (row, chunk), 64 / GL columns an instruction, and of its FP8
+    // last dword; columns past N read the last one (their outputs are dropped)
+    constexpr int GI = kGguf<KIND> ? R::WQ / 1024 : 1, GL = KIND == FH_F16 ? 4 : 2;  // instructions, lanes a column
+    constexpr uint32_t GB = kGgufBlock<KIND>;
+    uint32_t grow[GI] = {}, grow4 = 0, gsh = 0;
+    if constexpr (kGguf<KIND>) {
+        const uint32_t chunk = KIND == FH_F16 ? lane % 4 ^ lane / 16 : lane % 2;  // (lane / 16 = column / 4 % 4)
+#pragma unroll
+        for (int i = 0; i < GI; i++)
+            grow[i] = min(n0 + 64 * wn + 64 / GL * i + lane / GL, N - 1) * nb * GB + 16 * chunk;
+        grow4 = min(ncol, N - 1) * nb * GB + 32;
+        // the byte of block b's start in its first dword: (bits 16 j .. of gsh) + b GB, modulo 4
+        gsh = (min(n0 + 64 * wn + fr, N - 1) * nb * GB & 3) | (min(n0 + 64 * wn + 32 + fr, N - 1) * nb * GB & 3) << 16;
+    }
     auto dma = [&](uint32_t b, uint32_t slot, int part) {  // part 0: weights and scales; 1: x
         const bool live = b < st1;
         const uint32_t x0 = lds0 + slot * R::STAGE + kg * R::GROUP, w0 = x0 + R::X + wn * R::W;
+        if (part == 0 && kGguf<KIND>) {
+            const i32x4 rq = sgpr_rsrc(qs, live ? N * nb * GB + 64 : 0u);  // (the allocation has 256 bytes past it)
+#pragma unroll
+            for (int i = 0; i < GI; i++)
+                asm_load_lds16(rq, w0 + 1024 * i, (grow[i] + b * GB) & ~3u);
+            if constexpr (kFp8<KIND>) asm_load_lds4(rq, w0 + R::WQ, (grow4 + b * GB) & ~3u);
+            return;
+        }
         if (part == 0) {
             const i32x4 rq = sgpr_rsrc(qs, live ? (N + 31) / 32 * 32 * nb * R::QB : 0u);
             const i32x4 rd = sgpr_rsrc(ds, live ? (N + 31) / 32 * 512 * nb8 : 0u);
@@ -126,12 +167,31 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
     struct Frag {
         f16x8 h[MTW][2], l[MTW][2];
         u32x2 q[2][KIND == FH_Q8_0 ? 2 : 1];
-        uint32_t d[2];
+        u32x4 g[2][2];  // GGUF rows: the lane's dwords
+        uint32_t e[2], d[2];
     };
     auto read_w = [&](Frag &f, uint32_t slot) {
         const uint8_t *sw = arena + slot * R::STAGE + kg * R::GROUP + R::X + wn * R::W;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
+            const uint32_t c = j * 32 + fr;
+            if constexpr (kFp8<KIND>) {  // dwords 4 half .. + 4: codes 16 half .. + 15
+                f.g[j][0] = *(const u32x4 *)(sw + c * 32 + 16 * hf);
+                f.e[j] = *(const uint32_t *)(sw + (hf ? R::WQ + c * 4 : c * 32 + 16));
+                f.d[j] = *(const uint32_t *)(sw + c * 32);
+                continue;
+            }
+            if constexpr (KIND == FH_MXFP4) {  // dwords 2 half .. + 2: bytes 8 half .. + 7 of the nibbles
+                const u32x2 v = *(const u32x2 *)(sw + c * 32 + 8 * hf);
+                f.g[j][0] = u32x4{v[0], v[1], *(const uint32_t *)(sw + c * 32 + 8 * hf + 8), 0u};
+                f.d[j] = *(const uint32_t *)(sw + c * 32);
+                continue;
+            }
+            if constexpr (KIND == FH_F16) {
+#pragma unroll
+                for (int s = 0; s < 2; s++) f.g[j][s] = *(const u32x4 *)(sw + c * 64 + ((2 * hf + s) ^ (fr / 4 % 4)) * 16);
+                continue;
+            }
             if constexpr (KIND == FH_Q8_0) {
 #pragma unroll
                 for (int s = 0; s < 2; s++) f.q[j][s] = *(const u32x2 *)(sw + j * 1024 + s * 512 + fr * 16 + 8 * hf);
@@ -147,12 +207,64 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
         const uint8_t *row = arena + slot * R::STAGE + kg * R::GROUP + r * 128;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            f.h[i][s] = *(const f16x8 *)(row + (((hf + 2 * s) ^ ((r >> 1) & 7)) * 16));
-            f.l[i][s] = *(const f16x8 *)(row + (((4 + hf + 2 * s) ^ ((r >> 1) & 7)) * 16));
+            const uint32_t c = kGguf<KIND> ? 2 * hf + s : hf + 2 * s;  // (GGUF rows: a lane's codes are consecutive)
+            f.h[i][s] = *(const f16x8 *)(row + ((c ^ ((r >> 1) & 7)) * 16));
+            f.l[i][s] = *(const f16x8 *)(row + (((4 + c) ^ ((r >> 1) & 7)) * 16));
         }
     };
-    auto unpack = [&](const Frag &f, int j, f16x8 (&b)[2]) {  // exact f16 integers
-        if constexpr (KIND == FH_Q8_0) {
+    // Column tile j of block blk: exact f16 values; returns the block's scale. A block that holds an infinity or
+    // NaN has a NaN scale (an E4M3 NaN makes its outputs NaN by itself): the split x would otherwise meet an
+    // infinity with lo = 0 or of the other sign.
+    auto unpack = [&](const Frag &f, int j, uint32_t blk, f16x8 (&b)[2]) {
+        if constexpr (kFp8<KIND>) {
+            const uint32_t sh = ((gsh >> (16 * j)) + blk * GB) & 2, sel = sh ? 0x07060504u : 0x05040302u;
+            const u32x4 &w = f.g[j][0];
+            uint32_t bad = 0;
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                u32x4 o;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {  // codes 8 s + 4 i .. + 3
+                    const int at = 2 * s + i;
+                    const uint32_t v = __builtin_amdgcn_perm(at == 3 ? f.e[j] : w[(at + 1) % 4], w[at], sel);
+                    if constexpr (KIND == FH_FP8_E5M2) {  // the top byte of an f16
+                        o[2 * i] = __builtin_amdgcn_perm(v, 0u, 0x050c040cu);
+                        o[2 * i + 1] = __builtin_amdgcn_perm(v, 0u, 0x070c060cu);
+                        bad |= ((v & 0x7c7c7c7cu) + 0x04040404u) & 0x80808080u;
+                    } else {
+                        o[2 * i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 1.0f, false));
+                        o[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 1.0f, true));
+                    }
+                }
+                b[s] = __builtin_bit_cast(f16x8, o);
+            }
+            const float d = half_to_float((sh ? f.d[j] >> 16 : f.d[j]) & 0xffffu);
+            if constexpr (KIND == FH_FP8_E4M3) return d;
+            const auto r = __builtin_amdgcn_permlane32_swap(bad, bad, false, false);  // (both halves of the block)
+            return r[0] | r[1] ? __uint_as_float(0x7fc00000u) : d;
+        } else if constexpr (KIND == FH_MXFP4) {  // (values times two, 0 .. 12; x order: byte i's two elements side by side)
+            const uint32_t sh = ((gsh >> (16 * j)) + blk * GB) & 3, sel = 0x04030201u + 0x01010101u * sh;
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const uint32_t v = __builtin_amdgcn_perm(f.g[j][0][s + 1], f.g[j][0][s], sel);
+                b[s] = __builtin_bit_cast(
+                    f16x8, u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 0)),
+                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 1)),
+                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 2)),
+                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 3))});
+            }
+            return e8m0_half_scale((f.d[j] >> (8 * sh)) & 0xffu);
+        } else if constexpr (KIND == FH_F16) {
+            uint32_t bad = 0;
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                b[s] = __builtin_bit_cast(f16x8, f.g[j][s]);
+#pragma unroll
+                for (int c = 0; c < 4; c++) bad |= (f.g[j][s][c] & 0x7c007c00u) + 0x04000400u;
+            }
+            const auto r = __builtin_amdgcn_permlane32_swap(bad, bad, false, false);
+            return (r[0] | r[1]) & 0x80008000u ? __uint_as_float(0x7fc00000u) : 1.0f;
+        } else if constexpr (KIND == FH_Q8_0) {
 #pragma unroll
             for (int s = 0; s < 2; s++) {
                 const u32x2 q = f.q[j][s] ^ 0x80808080u;
@@ -173,6 +285,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
                                  f16x2_add(((q >> 12) & 0x000f000fu) | 0x64006400u, (_Float16)-1032.0f)});
             }
         }
+        if constexpr (!kGguf<KIND>) return half_to_float(blk & 1 ? f.d[j] >> 16 : f.d[j] & 0xffffu);
     };
     // Block b (fragments f): tile v's MFMAs (a dependent chain), each followed by a share of tile v - 1's scale
     // FMAs, or, in the first tile, of the second column tile's unpacking. The stage's other work, the
@@ -183,16 +296,14 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
         constexpr int V = 2 * MTW;
         f16x8 bq[2][2];
         float dq[2];
-        unpack(f, 0, bq[0]);
-#pragma unroll
-        for (int j = 0; j < 2; j++) dq[j] = half_to_float(b & 1 ? f.d[j] >> 16 : f.d[j] & 0xffffu);
+        dq[0] = unpack(f, 0, b, bq[0]);
         f32x16 pr[2];
 #pragma unroll
         for (int v = 0; v <= V; v++) {
             const int j = v / MTW, i = v % MTW, vp = v - 1, jp = vp / MTW, ip = vp % MTW;
             f32x16 q = {};
             if (v == 0) {
-                unpack(f, 1, bq[1]);
+                dq[1] = unpack(f, 1, b, bq[1]);
                 read_w(nxt, after);
             }
             if (v == 1) read_x(nxt, after, 0);
@@ -285,33 +396,44 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
 
 }  // namespace
 
-// The group count and K splits of a product, and its time in us: rounds of a workgroup per CU, each its stages
-// (0.99 us; measured 0.9 to 1.1) and a workgroup's own cost (first loads and epilogue, 6 us). Two splits only
-// where one leaves half of the CUs idle. (512 rows: 2048 x 2560 26 us with 128-column tiles, 42 with
-// 256-column ones; 896 x 9728 at 300 rows 29 and 26.)
+// The row tile, group count and K splits of a product, and its time in us: rounds of a workgroup per CU, each
+// its stages (64 rows: 0.99 us, measured 0.9 to 1.1; 32 rows: 0.5 us with few workgroups and 0.85 with one on
+// every CU, for twice the weight loads and unpacking per row) and a workgroup's own cost (first loads and epilogue, 7 and 4 us). Two splits only where one leaves half
+// of the CUs idle, at the cost of zeroing y and of two additions per output. GGUF rows cost a stage more by the factor f. (512 rows: 2048 x 2560 26 us with 128-column tiles, 42 with 256-column ones; 896 x 9728
+// at 300 rows 29 and 26. 32-row tiles where 64-row ones are few: Q8_0 5632 x 2048
+// 128 rows 29 with 64-row tiles, 23 with 32-row ones; 2048 x 11264 128 rows 25 and 29.)
 struct RingPlan {
-    uint32_t kg, splits;
+    uint32_t mtw, kg, splits;
     float us;
 };
-static RingPlan ring_plan(size_t rows, size_t k, size_t n) {
-    const size_t bm = rows <= 32 ? 32 : 64, mt = (rows + bm - 1) / bm, nb = k / 32;
-    RingPlan best{4, 1, INFINITY};
-    for (uint32_t kg : {4u, 2u})
-        for (uint32_t sp : {1u, 2u}) {
-            const uint64_t tiles = mt * ((n + 512 / kg - 1) / (512 / kg));
-            if (sp == 2 && (tiles > 128 || nb < 4 * kg)) continue;
-            const float us = (float)((tiles * sp + 255) / 256 * ((nb + sp * kg - 1) / (sp * kg) + 6) + (sp == 2 ? 2 : 0));
-            if (us < best.us) best = RingPlan{kg, sp, us};
-        }
+static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n) {
+    const size_t nb = k / 32;
+    const float f = kind == FH_F16 ? 1.3f : kind == FH_MXFP4 ? 1.15f : kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 ? 1.25f : 1.0f;
+    RingPlan best{1, 4, 1, INFINITY};
+    for (uint32_t mtw : {2u, 1u})
+        for (uint32_t kg : {4u, 2u})
+            for (uint32_t sp : {1u, 2u}) {
+                if (mtw == 2 && (rows <= 32 || (kind == FH_F16 && kg == 4))) continue;  // (that stage does not fit LDS three times)
+                const uint64_t tiles = (rows + 32 * mtw - 1) / (32 * mtw) * ((n + 512 / kg - 1) / (512 / kg));
+                if (sp == 2 && (tiles > 128 || nb < 4 * kg)) continue;
+                const float stages = (float)((nb + sp * kg - 1) / (sp * kg));
+                const float c32 = f * (0.45f + 0.4f * std::min((float)(tiles * sp) / 256, 1.0f)), c64 = f * 0.99f;
+                const float us = (float)((tiles * sp + 255) / 256) * (mtw == 2 ? c64 * stages + 7 : c32 * stages + 4) +
+                                 (sp == 2 ? 1.5f + 3e-6f * (float)rows * (float)n : 0);
+                if (us < best.us) best = RingPlan{mtw, kg, sp, us};
+            }
     return best;
 }
-uint32_t ring_splits(size_t rows, size_t k, size_t n) { return ring_plan(rows, k, n).splits; }
-float ring_us(size_t rows, size_t k, size_t n) { return ring_plan(rows, k, n).us; }
+uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n) { return ring_plan(kind, rows, k, n).splits; }
+float ring_us(int kind, size_t rows, size_t k, size_t n) { return ring_plan(kind, rows, k, n).us; }
 
 bool ring_supported(size_t rows, size_t k, size_t n) {
     // every byte offset a workgroup forms (rows and columns up to the last tile's end) fits in 32 bits
     const size_t lim = (size_t)1 << 31;
     return (rows + 63) * k * 4 < lim && (n + 255) * (k / 32 + 8) * 32 < lim && (rows + 63) / 32 * ((n + 127) / 128) < (1u << 26);
+}
+bool ring_gguf_supported(int kind, size_t rows, size_t k, size_t n) {
+    return kind != FH_Q2_K && ring_supported(rows, k, n) && n * (k / 32) * 64 + 128 < ((size_t)1 << 31);
 }
 
 template <int KIND, int MTW, int KG>
@@ -331,18 +453,26 @@ static hipError_t run_ring(hipStream_t s, const _Float16 *xs, const uint8_t *qs,
 template <int KIND>
 static hipError_t run_ring_kind(hipStream_t s, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
                                 uint32_t M, uint32_t K, uint32_t N, uint32_t sp, bool add) {
-    const uint32_t kg = ring_plan(M, K, N).kg;
-    if (M <= 32)
-        return kg == 4 ? run_ring<KIND, 1, 4>(s, xs, qs, ds, out, M, K, N, sp, add)
-                       : run_ring<KIND, 1, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
-    return kg == 4 ? run_ring<KIND, 2, 4>(s, xs, qs, ds, out, M, K, N, sp, add)
-                   : run_ring<KIND, 2, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
+    const RingPlan p = ring_plan(KIND, M, K, N);
+    if (p.mtw == 1)
+        return p.kg == 4 ? run_ring<KIND, 1, 4>(s, xs, qs, ds, out, M, K, N, sp, add)
+                         : run_ring<KIND, 1, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
+    if constexpr (KIND != FH_F16)
+        if (p.kg == 4) return run_ring<KIND, 2, 4>(s, xs, qs, ds, out, M, K, N, sp, add);
+    return run_ring<KIND, 2, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
 }
 
-hipError_t launch_gemm_ring(hipStream_t s, fh_kind kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds,
-                            float *out, uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add) {
-    return kind == FH_Q8_0 ? run_ring_kind<FH_Q8_0>(s, xs, qs, ds, out, M, K, N, splits, add)
-                           : run_ring_kind<FH_Q4_0>(s, xs, qs, ds, out, M, K, N, splits, add);
+hipError_t launch_gemm_ring(hipStream_t s, int kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
+                            uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add) {
+    switch (kind) {
+    case FH_Q8_0: return run_ring_kind<FH_Q8_0>(s, xs, qs, ds, out, M, K, N, splits, add);
+    case FH_Q4_0: return run_ring_kind<FH_Q4_0>(s, xs, qs, ds, out, M, K, N, splits, add);
+    case FH_F16: return run_ring_kind<FH_F16>(s, xs, qs, nullptr, out, M, K, N, splits, add);
+    case FH_FP8_E4M3: return run_ring_kind<FH_FP8_E4M3>(s, xs, qs, nullptr, out, M, K, N, splits, add);
+    case FH_FP8_E5M2: return run_ring_kind<FH_FP8_E5M2>(s, xs, qs, nullptr, out, M, K, N, splits, add);
+    case FH_MXFP4: return run_ring_kind<FH_MXFP4>(s, xs, qs, nullptr, out, M, K, N, splits, add);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace fh

@@ -313,13 +313,15 @@ hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, c
                                float *y, size_t rows, size_t k, size_t n, void *workspace,
                                SplitOut *defer = nullptr, float *partial = nullptr);
 size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n);
-// gemm_ring.hip: the precise product alone on split x: `splits` (1 or 2) partial products of M x N at out,
-// or (add) their sum added to zeros at out.
-uint32_t ring_splits(size_t rows, size_t k, size_t n);
-float ring_us(size_t rows, size_t k, size_t n);  // its time by the plan's model
+// gemm_ring.hip: the precise product alone on split x (of split_x_precise_kernel's order for the kind): `splits`
+// (1 or 2) partial products of M x N at out, or (add) their sum added to zeros at out. Kinds other than
+// Q8_0 and Q4_0 (ring_gguf_supported): qs is the GGUF rows.
+uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n);
+float ring_us(int kind, size_t rows, size_t k, size_t n);  // its time by the plan's model
 bool ring_supported(size_t rows, size_t k, size_t n);
-hipError_t launch_gemm_ring(hipStream_t s, fh_kind kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds,
-                            float *out, uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add);
+bool ring_gguf_supported(int kind, size_t rows, size_t k, size_t n);
+hipError_t launch_gemm_ring(hipStream_t s, int kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
+                            uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add);
 
 // prefill.hip: the GPT-2 prompt pass (one row per prompt token). prefill_row_kernel makes a row by mode
 // and writes it as a product's split x (launch_gemm_precise's), scaled by a power of two whose inverse

@@ -51,3 +51,29 @@ def test_ring_product(fh, g, orc, kind_name, k, n, rows):
         worst = float((err / np.maximum(bound, 1e-38)).max())
         print(f"{kind_name} {m} x {k} x {n}: {worst:.3f} of the bound", flush=True)
         assert np.all(err <= bound), (kind_name, k, n, m, worst)
+
+
+@pytest.mark.parametrize("kind_name", ["Fp8E4M3", "Fp8E5M2", "Fp4", "F16"])
+@pytest.mark.parametrize("k,n,rows", [(32, 1, (2, 33)), (96, 65, (31, 33, 65)), (160, 129, (64, 130)),
+                                      (1056, 257, (33, 200)), (4896, 127, (17, 100)), (896, 9728, (300,)),
+                                      (2048, 2560, (1024,))])
+def test_ring_product_of_gguf_rows(fh, g, orc, kind_name, k, n, rows):
+    """The formats kept as GGUF rows: odd block counts put a column's blocks at every byte offset."""
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(k + n)
+    raw = orc.encode(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32))
+    w = orc.decode(int(kind), raw, k * n).reshape(n, k).T.astype(np.float64)
+    qw = fh.upload_qweight(g, kind, raw, k, n)
+    for m in rows:
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        gx, gy = g.upload(x), g.upload(np.full(m * n, np.nan, np.float32))
+        fh.linear_q_with(g, gx, qw, gy, m, fh.QPath.Tiled)
+        first = g.read(gy)
+        fh.linear_q_with(g, gx, qw, gy, m, fh.QPath.Tiled)
+        got = g.read(gy)
+        assert np.array_equal(first.view(np.uint32), got.view(np.uint32)), (kind_name, k, n, m)
+        bound = (k + 8) * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(w))
+        err = np.abs(got.reshape(m, n) - x.astype(np.float64) @ w)
+        worst = float((err / np.maximum(bound, 1e-38)).max())
+        print(f"{kind_name} {m} x {k} x {n}: {worst:.3f} of the bound", flush=True)
+        assert np.all(err <= bound), (kind_name, k, n, m, worst)
