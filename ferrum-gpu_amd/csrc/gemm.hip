@@ -2742,8 +2742,10 @@ size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n) {
     return sp > 1 ? (size_t)sp * rows * n * 4 : 0;
 }
 
-// x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned)
-size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n) {
+// x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned; parts false: for a
+// call without `defer`, whose ring splits add into y)
+size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts) {
+    if (!parts && precise_plan(rows, k, n).kernel == PrecisePlan::RING) return rows * k * 4;
     return (rows * k * 4 + 255) / 256 * 256 + gemm_precise_partial_bytes(rows, k, n);
 }
 

@@ -5,7 +5,17 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/ferrum_hip.h"
+
 namespace fh {
+
+// Kinds kept as GGUF rows, and their bytes per 32 elements
+template <int KIND>
+constexpr bool kGguf = KIND != FH_Q8_0 && KIND != FH_Q4_0;
+template <int KIND>
+constexpr bool kFp8 = KIND == FH_FP8_E4M3 || KIND == FH_FP8_E5M2;
+template <int KIND>
+constexpr uint32_t kGgufBlock = kFp8<KIND> ? 34 : KIND == FH_MXFP4 ? 17 : 64;
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));

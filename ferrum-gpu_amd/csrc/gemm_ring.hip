@@ -50,13 +50,6 @@ namespace {
 // loaded 2 (F16: 4) lanes per column, since a load takes a cycle per cache line that it touches (a lane per column
 // would take 64 a load, 192 cycles of a stage's 2400 for each of eight wavefronts). In registers a lane shifts its
 // dwords to the byte with v_perm and the hardware converts the codes to f16, exactly.
-template <int KIND>
-constexpr bool kGguf = KIND != FH_Q8_0 && KIND != FH_Q4_0;
-template <int KIND>
-constexpr bool kFp8 = KIND == FH_FP8_E4M3 || KIND == FH_FP8_E5M2;
-template <int KIND>
-constexpr uint32_t kGgufBlock = kFp8<KIND> ? 34 : KIND == FH_MXFP4 ? 17 : 64;
-
 // KG groups of wavefronts share K (4 pairs and a 128-column tile, or 2 fours and a 256-column tile).
 template <int KIND, int MTW, int KG>
 struct Ring {

@@ -235,9 +235,9 @@ hipError_t launch_rows(hipStream_t s, fh_kind kind, const uint8_t *qs, const uin
 // One launch for one product of 2 to kRowsMax rows (fits: where it is the faster one); scratch holds
 // rows_call_scratch_bytes, tickets kTicketCount zeros (left zero).
 constexpr size_t kTicketCount = 8192;
-bool rows_call_fits(size_t rows, size_t k, size_t n, int cus);
+bool rows_call_fits(int kind, size_t rows, size_t k, size_t n, int cus);
 size_t rows_call_scratch_bytes(size_t rows, size_t k, size_t n, int cus);
-hipError_t launch_rows_call(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+hipError_t launch_rows_call(hipStream_t s, int kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
                             size_t rows, size_t k, size_t n, void *scratch, uint32_t *tickets, int cus);
 // Many products of one format: descs and map (device memory) as for launch_gemv_group; max_m the
 // most rows of any product, max_items the largest rows * k / 32.
@@ -300,7 +300,7 @@ bool gemm_f16_supported(size_t rows, size_t k, size_t n);
 hipError_t launch_gemm_f16(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
                            size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer = nullptr);
 // The precise MFMA GEMM (x as two f16 parts; split into workspace, then the product).
-size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n);
+size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts = true);
 // The MFMA GEMM on the GGUF rows of F16, FP8 E4M3 / E5M2, MXFP4 and Q2_K weights (rows >= 2) and
 // its workspace (x split, then the K-split partial products).
 bool gemm_ext_kind(int kind);

@@ -33,15 +33,11 @@
 #include <algorithm>
 
 #include "device_common.hpp"
+#include "gemm_parts.hpp"
 #include "internal.hpp"
 
 namespace fh {
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // blocks per batch (one LDS stage of x): eight for up to 8 rows, else four (measured: eight
 // blocks take more registers, and from 16 rows on the lost occupancy costs more than the fewer
@@ -79,10 +75,6 @@ static_assert(rows_order_is_a_permutation<FH_Q8_0>() && rows_order_is_a_permutat
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-
-__device__ __forceinline__ float half_to_float(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
 
 // A product's descriptor as wave-uniform values (every dword through readfirstlane): read from the
@@ -426,7 +418,7 @@ hipError_t launch_rows_mt(hipStream_t s, const RowsDesc *descs, const uint32_t *
 }
 
 
-// ---- one product per launch (linear_q, AUTO, 2 to 64 rows) ----
+// ---- one product per launch (linear_q, AUTO, 2 to 64 rows; every format but Q2_K) ----
 // A single few-row product is bound by latency, not by bytes or by the matrix cores: an 896 x 1152
 // Q8_0 product of 24 rows is 1.1 MB of weights (0.2 us at HBM speed), and the two kernels above took 14 us
 // for it (an x split, a launch boundary, then 9 workgroups that each walk all of K with one batch in
@@ -436,7 +428,8 @@ hipError_t launch_rows_mt(hipStream_t s, const RowsDesc *descs, const uint32_t *
 // meet in LDS in a fixed order. Deep products with few outputs also split K over S workgroups: each
 // writes its sums agent-coherent and takes a ticket, and the last to arrive adds them in split order
 // (reproducible) and returns the ticket to zero. Same operand order and numerics as rows_kernel.
-// Qwen2-0.5B layer, 24 rows, Q8_0, four calls: 70.3 -> 31.9 us.
+// Qwen2-0.5B layer, 24 rows, Q8_0, four calls: 70.3 -> 31.9 us. FP8 rows, one call of 24 rows, against the MFMA
+// GEMM and its split: 4864 x 896 33 -> 11.6 us, 1024 x 2048 13.7 -> 7.3, 2048 x 2560 22.6 -> 9.9.
 constexpr int kCallWaves = 8;
 constexpr int kCallKB = 2;  // blocks a wavefront takes at a time
 
@@ -448,9 +441,77 @@ __device__ __forceinline__ float agent_load(const float *p) {
     return __uint_as_float(__hip_atomic_load((gl_u32 *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
+// The formats kept as GGUF rows (FP8, MXFP4, F16; ds null) take the same kernel: a lane's share of a block (FP8 and
+// F16 elements 16 h .. + 15; MXFP4 nibble bytes 8 h .. + 7) comes straight from the row, at any byte, and the
+// hardware converts the codes to f16, exactly. Their operand order: FP8 and F16 position 16 s + 8 h + j is element
+// 16 h + 8 s + j; MXFP4 positions 2 i and 2 i + 1 are byte 8 h + 4 s + i's two elements. A block with an infinity
+// or NaN has a NaN scale (an E4M3 NaN makes its outputs NaN by itself): split x would meet an infinity with
+// lo = 0 or of the other sign.
+template <int KIND>
+struct GgufShare {
+    uint32_t q[KIND == FH_F16 ? 8 : kFp8<KIND> ? 4 : 2], d;
+    __device__ __forceinline__ void load(const uint8_t *blk, uint32_t h) {
+        if constexpr (KIND == FH_F16) {
+            __builtin_memcpy(q, blk + 32 * h, 32);
+        } else if constexpr (KIND == FH_MXFP4) {
+            __builtin_memcpy(q, blk + 1 + 8 * h, 8);
+            d = blk[0];
+        } else {
+            __builtin_memcpy(q, blk + 2 + 16 * h, 16);
+            uint16_t t;
+            __builtin_memcpy(&t, blk, 2);
+            d = t;
+        }
+    }
+    // The two k steps' fragments; returns the block's scale.
+    __device__ __forceinline__ float unpack(f16x8 (&b)[2]) const {
+        typedef decltype(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(0u, 1.0f, false)) pair;
+        const auto bits = [](pair v) { return __builtin_bit_cast(uint32_t, v); };
+        uint32_t bad = 0;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            uint32_t o[4];
+            if constexpr (KIND == FH_MXFP4) {  // (values times two, 0 .. 12)
+                o[0] = bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[s], 2.0f, 0));
+                o[1] = bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[s], 2.0f, 1));
+                o[2] = bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[s], 2.0f, 2));
+                o[3] = bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[s], 2.0f, 3));
+            } else if constexpr (KIND == FH_F16) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    o[c] = q[4 * s + c];
+                    bad |= (o[c] & 0x7c007c00u) + 0x04000400u;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const uint32_t v = q[2 * s + i];
+                    if constexpr (KIND == FH_FP8_E5M2) {  // the top byte of an f16
+                        o[2 * i] = __builtin_amdgcn_perm(v, 0u, 0x050c040cu);
+                        o[2 * i + 1] = __builtin_amdgcn_perm(v, 0u, 0x070c060cu);
+                        bad |= (v & 0x7c7c7c7cu) + 0x04040404u;
+                    } else {
+                        o[2 * i] = bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 1.0f, false));
+                        o[2 * i + 1] = bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 1.0f, true));
+                    }
+                }
+            }
+            b[s] = __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
+        }
+        if constexpr (KIND == FH_MXFP4) return e8m0_half_scale(d);
+        const float sc = KIND == FH_F16 ? 1.0f : half_to_float(d);
+        if constexpr (KIND == FH_FP8_E4M3) return sc;
+        const auto r = __builtin_amdgcn_permlane32_swap(bad, bad, false, false);  // (both halves of the block)
+        return (r[0] | r[1]) & (KIND == FH_F16 ? 0x80008000u : 0x80808080u) ? __uint_as_float(0x7fc00000u) : sc;
+    }
+};
+
 // Eight x values (two float4) -> their hi and lo parts in operand order.
+template <int KIND>
 __device__ __forceinline__ void split_frag(const f32x4 &a, const f32x4 &b, f16x8 &hi, f16x8 &lo) {
-    const float e[8] = {a.x, a.z, a.y, a.w, b.x, b.z, b.y, b.w};
+    constexpr bool MX = KIND == FH_MXFP4, NAT = kGguf<KIND> && !MX;
+    const float e[8] = {a.x, MX ? b.x : NAT ? a.y : a.z, MX || !NAT ? a.y : a.z, MX ? b.y : a.w,
+                        MX ? a.z : b.x, MX || !NAT ? b.z : b.y, MX ? a.w : NAT ? b.z : b.y, b.w};
 #pragma unroll
     for (int q = 0; q < 8; q++) {
         const _Float16 v = (_Float16)fminf(fmaxf(e[q], -65504.0f), 65504.0f);
@@ -460,7 +521,7 @@ __device__ __forceinline__ void split_frag(const f32x4 &a, const f32x4 &b, f16x8
 }
 
 template <int KIND, int MT, int TN>
-__global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void rows_call_kernel(
+__global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 && !kGguf<KIND> ? 4 : 2)) void rows_call_kernel(
     const uint8_t *__restrict__ qs, const uint16_t *__restrict__ ds, const float *__restrict__ x, float *__restrict__ y,
     uint32_t m, uint32_t nb, uint32_t n, uint32_t splits, float *__restrict__ part, uint32_t *__restrict__ tickets) {
     constexpr uint32_t QB = KIND == FH_Q8_0 ? 32 : 16;
@@ -475,13 +536,17 @@ __global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void
     const auto rx = make_rsrc(x, m * nb * 128);
     __amdgpu_buffer_rsrc_t rq[TN], rd[TN];
 #pragma unroll
-    for (int j = 0; j < TN; j++) {
+    for (int j = 0; j < TN && !kGguf<KIND>; j++) {
         const bool live = g0 + j < groups;  // a tile past the product: every load reads 0
         rq[j] = make_rsrc(qs + (size_t)(live ? g0 + j : 0) * nb * 32 * QB, live ? nb * 32 * QB : 0);
         rd[j] = make_rsrc(ds + (size_t)(live ? g0 + j : 0) * nb8 * 256, live ? nb8 * 512 : 0);
     }
+    const uint8_t *grow[TN] = {};  // GGUF rows: the lane's (an output past the product reads the last one)
+#pragma unroll
+    for (int j = 0; j < TN && kGguf<KIND>; j++) grow[j] = qs + (size_t)min((g0 + j) * 32 + r, n - 1) * nb * kGgufBlock<KIND>;
     struct Batch {
         f32x4 x[MT][kCallKB][2][2];            // [row tile][block][k step][half of eight]
+        GgufShare<KIND> g[TN][2];
         u32x4 q[TN][KIND == FH_Q8_0 ? 2 : 1];  // Q8_0: a block each; Q4_0: lane half h holds block h's
         uint32_t d[TN];                        // the two blocks' scales
     };
@@ -489,6 +554,11 @@ __global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void
         const uint32_t b0 = 2 * p;
 #pragma unroll
         for (int j = 0; j < TN; j++) {
+            if constexpr (kGguf<KIND>) {  // (a block past the row: the last one again, against x = 0)
+#pragma unroll
+                for (int i = 0; i < 2; i++) b.g[j][i].load(grow[j] + min(b0 + i, nb - 1) * kGgufBlock<KIND>, h);
+                continue;
+            }
             if constexpr (KIND == FH_Q8_0) {
 #pragma unroll
                 for (int i = 0; i < 2; i++)
@@ -506,14 +576,14 @@ __global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void
             for (int kb = 0; kb < kCallKB; kb++)
 #pragma unroll
                 for (int s = 0; s < 2; s++) {
-                    // element 16 s + 8 h (Q4_0) or 16 h + 8 s (Q8_0) of the block; rows past m and
-                    // blocks past the row read 0
-                    const uint32_t e = KIND == FH_Q4_0 ? 16 * s + 8 * h : 16 * h + 8 * s;
+                    // element 16 s + 8 h (Q4_0) or 16 h + 8 s of the block (MXFP4 8 h + 4 s, and 16 further);
+                    // rows past m and blocks past the row read 0
+                    const uint32_t e = KIND == FH_Q4_0 ? 16 * s + 8 * h : KIND == FH_MXFP4 ? 8 * h + 4 * s : 16 * h + 8 * s;
                     const uint32_t off = b0 + kb < nb ? (((i * 32 + r) * nb + b0 + kb) * 32 + e) * 4 : 0x80000000u;
 #pragma unroll
                     for (int c = 0; c < 2; c++)
                         b.x[i][kb][s][c] =
-                            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(off + 16 * c), 0, 0));
+                            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(off + (KIND == FH_MXFP4 ? 64 : 16) * c), 0, 0));
                 }
     };
     f32x16 acc[MT][TN];
@@ -530,6 +600,11 @@ __global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void
         float dv[TN][kCallKB];
 #pragma unroll
         for (int j = 0; j < TN; j++) {
+            if constexpr (kGguf<KIND>) {
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++) dv[j][kb] = b.g[j][kb].unpack(bf[j][kb]);
+                continue;
+            }
             if constexpr (KIND == FH_Q8_0) {
 #pragma unroll
                 for (int kb = 0; kb < 2; kb++) {
@@ -562,7 +637,7 @@ __global__ __launch_bounds__(64 * kCallWaves, (MT == 1 && TN == 1 ? 4 : 2)) void
             for (int i = 0; i < MT; i++) {
                 f16x8 hi[2], lo[2];
 #pragma unroll
-                for (int s = 0; s < 2; s++) split_frag(b.x[i][kb][s][0], b.x[i][kb][s][1], hi[s], lo[s]);
+                for (int s = 0; s < 2; s++) split_frag<KIND>(b.x[i][kb][s][0], b.x[i][kb][s][1], hi[s], lo[s]);
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
                     f32x16 p = {};
@@ -685,17 +760,24 @@ bool rows_supported(size_t rows, size_t k, size_t n) {
            nb * 32 * 32 < ((size_t)1 << 31) && (n + 31) / 32 * 32 <= ((size_t)1 << 30);
 }
 
-// Where the one-launch kernel is the faster one for a single product (us, Q4_0, this kernel / rows_kernel
-// and its split / the precise GEMM): up to 32 rows while its workgroups run at once (24 rows: 896 x 1152
-// 5.9 / 13.2 / 15.9, 4864 x 896 11.0 / 27.8 / 31.6, 2048 x 11264, 176 workgroups, 13.0 / 16.3 / 25.8; but
-// 2048 x 20000, 313 workgroups, 24.0 / 20.4 / 28.6); past 32 rows, with twice the x to split, also up to
-// 64 tile blocks per CU (48 rows: 896 x 9728 14.8 / 18.7 / 21.8, 5632 x 2048 20.1 / 45.2 / 31.1; but
-// 2048 x 11264 23.8 / 22.7 / 28.5). k <= 16384 keeps the K splits' scratch small.
-bool rows_call_fits(size_t rows, size_t k, size_t n, int cus) {
-    if (rows < 2 || rows > kRowsMax || !rows_supported(rows, k, n) || k > 16384) return false;
+// Where the one-launch kernel is the faster one for a single product (us, this kernel / the precise GEMM's ring
+// kernel and its x split): while its workgroups run at once, up to 32 rows (Q8_0, 8 and 32 rows: 896 x 1152 5.8 and
+// 7.2 / 10.1 and 10.5, 4864 x 896 10.6 and 11.7 / 16.6 and 17.6, 2048 x 11264 11.8 and 14.7 / 12.6 and 14.4); GGUF
+// rows, whose loads touch a cache line per output, while a workgroup has few blocks (FP8, 24 rows: 896 x 9728, 56
+// blocks, 9.2 / 12.5; 2048 x 5632, 64 blocks, 16.1 / 15.4, but 8 rows 13.3 / 14.9; 2048 x 11264, 128, 23.0 /
+// 16.6). Past 32 rows, with twice the x to split, up to 44 blocks (Q4_0, 48 rows: 5632 x 2048 20.0 / 22.9,
+// 896 x 1152 9.6 / 11.6; 896 x 9728, 56, 14.8 / 12.2); Q8_0 and F16, whose ring stages are cheaper, only
+// without K splits over workgroups (2048 x 2560, three splits, Q8_0 13.0 / 11.4), F16 up to 16 (896 x 1152,
+// 28, 10.3 / 8.9). k <= 16384 keeps the K splits' scratch small.
+bool rows_call_fits(int kind, size_t rows, size_t k, size_t n, int cus) {
+    if (kind == FH_Q2_K || rows < 2 || rows > kRowsMax || !rows_supported(rows, k, n) || k > 16384) return false;
     const size_t c = cus > 0 ? (size_t)cus : 256;
     const CallPlan p = call_plan(k, n, cus);
-    return p.wgs <= c && p.wgs <= kTicketCount && (rows <= 32 || k / 32 * ((n + 31) / 32) <= 64 * c);
+    if (p.wgs > c || p.wgs > kTicketCount) return false;
+    const size_t blocks = (k / 32 + p.splits - 1) / p.splits * p.tn;  // of a workgroup
+    if (rows <= 32) return kind == FH_Q8_0 || kind == FH_Q4_0 || blocks <= (rows <= 16 ? 64 : 56);
+    if (kind == FH_F16) return p.splits == 1 && blocks <= 16;
+    return blocks <= 44 && (kind != FH_Q8_0 || p.splits == 1);
 }
 
 size_t rows_call_scratch_bytes(size_t rows, size_t k, size_t n, int cus) {
@@ -703,14 +785,20 @@ size_t rows_call_scratch_bytes(size_t rows, size_t k, size_t n, int cus) {
     return p.splits > 1 ? (size_t)p.wgs * p.splits * p.tn * (rows > 32 ? 2 : 1) * 4096 : 0;
 }
 
-hipError_t launch_rows_call(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+hipError_t launch_rows_call(hipStream_t s, int kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
                             size_t rows, size_t k, size_t n, void *scratch, uint32_t *tickets, int cus) {
     const CallPlan p = call_plan(k, n, cus);
-    if (kind == FH_Q8_0)
-        return launch_rows_call_kind<FH_Q8_0>(s, qs, ds, x, y, (uint32_t)rows, (uint32_t)(k / 32), (uint32_t)n, p,
-                                              (float *)scratch, tickets);
-    return launch_rows_call_kind<FH_Q4_0>(s, qs, ds, x, y, (uint32_t)rows, (uint32_t)(k / 32), (uint32_t)n, p,
-                                          (float *)scratch, tickets);
+    const uint32_t m = (uint32_t)rows, nb = (uint32_t)(k / 32), N = (uint32_t)n;
+    float *part = (float *)scratch;
+    switch (kind) {
+    case FH_Q8_0: return launch_rows_call_kind<FH_Q8_0>(s, qs, ds, x, y, m, nb, N, p, part, tickets);
+    case FH_Q4_0: return launch_rows_call_kind<FH_Q4_0>(s, qs, ds, x, y, m, nb, N, p, part, tickets);
+    case FH_F16: return launch_rows_call_kind<FH_F16>(s, qs, ds, x, y, m, nb, N, p, part, tickets);
+    case FH_FP8_E4M3: return launch_rows_call_kind<FH_FP8_E4M3>(s, qs, ds, x, y, m, nb, N, p, part, tickets);
+    case FH_FP8_E5M2: return launch_rows_call_kind<FH_FP8_E5M2>(s, qs, ds, x, y, m, nb, N, p, part, tickets);
+    case FH_MXFP4: return launch_rows_call_kind<FH_MXFP4>(s, qs, ds, x, y, m, nb, N, p, part, tickets);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 size_t rows_xsplit_bytes(size_t rows, size_t k) { return rows * (k / 32) * 128; }

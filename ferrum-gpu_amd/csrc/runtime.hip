@@ -761,7 +761,7 @@ static fh_status command_scratch(fh_device *dev, void *fixed, size_t bytes, void
 static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, float *y, size_t rows,
                         fh_path path, void *fixed = nullptr) {
     fh_status st;
-    if (path == FH_PATH_AUTO && kind_ok(w->kind) && rows_call_fits(rows, w->k, w->n, dev->cus)) {  // one launch
+    if (path == FH_PATH_AUTO && rows_call_fits(w->kind, rows, w->k, w->n, dev->cus)) {  // one launch
         void *part = nullptr;
         const size_t bytes = rows_call_scratch_bytes(rows, w->k, w->n, dev->cus);
         if (bytes && (st = command_scratch(dev, fixed, bytes, &part))) return st;
@@ -769,6 +769,11 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         (void)launch_rows_call(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, part, dev->tickets, dev->cus);
         return end_command(dev, "linear_q");
     }
+    // Past 16 rows the precise GEMM's ring kernel beats the few-row kernel's two launches (us, Q8_0, few-row /
+    // ring: 2048 x 11264 33 rows 23.3 / 17.0, 64 rows 25.3 / 17.5; 2048 x 20000 32 rows 23.4 / 17.9, 16 rows 18.6 /
+    // 17.0 but Q4_0 17.3 / 18.4), with no more scratch.
+    if (path == FH_PATH_AUTO && rows > 16 && rows <= kRowsMax && kind_ok(w->kind) && ring_supported(rows, w->k, w->n))
+        path = FH_PATH_TILED;
     if (path == FH_PATH_AUTO) path = fh_choose(rows, w->kind, w->k, w->n);
     if (ext_kind(w->kind)) {  // decoded on the fly (formats.hip; the multi-row MFMA GEMM in gemm.hip)
         if (path != FH_PATH_NAIVE && path != FH_PATH_GEMV && path != FH_PATH_TILED)
@@ -822,7 +827,7 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         return end_command(dev, "linear_q");
     case FH_PATH_TILED: {
         void *ws = nullptr;
-        if (rows && (st = command_scratch(dev, fixed, gemm_precise_workspace_bytes(rows, w->k, w->n), &ws)))
+        if (rows && (st = command_scratch(dev, fixed, gemm_precise_workspace_bytes(rows, w->k, w->n, false), &ws)))
             return st;
         if ((st = begin_command(dev, "linear_q"))) return st;
         if (rows) (void)launch_gemm_precise(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws);

@@ -51,3 +51,39 @@ def test_one_launch_product(fh, g, orc, kind_name, k, n):
         err = np.abs(got.reshape(m, n) - x.astype(np.float64) @ w)
         assert np.all(err <= bound), (kind_name, k, n, m, float((err / np.maximum(bound, 1e-38)).max()))
         print(f"{kind_name} {k}x{n} rows {m}: {float((err / np.maximum(bound, 1e-38)).max()):.3f} of the bound", flush=True)
+
+
+@pytest.mark.parametrize("kind_name", ["Fp8E4M3", "Fp8E5M2", "Fp4", "F16"])
+@pytest.mark.parametrize("k,n", [(32, 1), (96, 33), (1056, 40), (4864, 100), (64, 16450)])
+def test_one_launch_product_of_gguf_rows(fh, g, orc, kind_name, k, n):
+    """The formats kept as GGUF rows. In the first output's last block and the last output's first one an
+    infinity or NaN makes that output NaN for every row of x, and no other."""
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(k + n)
+    raw = orc.encode(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32))
+    w = orc.decode(int(kind), raw, k * n).reshape(n, k).T.astype(np.float64)
+    qw = fh.upload_qweight(g, kind, raw, k, n)
+    for m in (2, 3, 31, 32, 33, 64):
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        gx, gy = g.upload(np.concatenate([[0.0], x.reshape(-1)])), g.zeros(m * n)
+        fh.linear_q_ptr(g, gx.device_ptr() + 4, qw, gy.device_ptr(), m)
+        first = g.read(gy)
+        fh.linear_q_ptr(g, gx.device_ptr() + 4, qw, gy.device_ptr(), m)
+        got = g.read(gy)
+        assert np.array_equal(first.view(np.uint32), got.view(np.uint32)), (kind_name, k, n, m)
+        bound = (k + 8) * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(w))
+        err = np.abs(got.reshape(m, n) - x.astype(np.float64) @ w)
+        assert np.all(err <= bound), (kind_name, k, n, m, float((err / np.maximum(bound, 1e-38)).max()))
+    bad = {"Fp8E4M3": [0xff], "Fp8E5M2": [0x7c], "F16": [0x00, 0xfc]}.get(kind_name)
+    if bad is None or n < 2:
+        return
+    nb = raw.size // (k // 32 * n)
+    codes = raw.copy().reshape(n, k // 32, nb)
+    codes[0, -1, nb - len(bad):] = bad
+    codes[-1, 0, nb - 32 if nb == 34 else 0:][: len(bad)] = bad
+    qw = fh.upload_qweight(g, kind, codes.reshape(-1), k, n)
+    m = 5
+    gx, gy = g.upload(rng.standard_normal(m * k).astype(np.float32)), g.zeros(m * n)
+    fh.linear_q_ptr(g, gx.device_ptr(), qw, gy.device_ptr(), m)
+    nan = np.isnan(g.read(gy).reshape(m, n))
+    assert nan[:, [0, -1]].all() and nan.sum() == 2 * m
