@@ -11,8 +11,8 @@
 //
 // The precise kernels (FH_PATH_TILED, within the reference's 1e-5 product tolerance,
 // ferrum_wgpu/src/tolerance.rs:7; gemm_stream_precise_kernel here and gemm_ring_kernel in
-// gemm_ring.hip, gemm_precise_kernel for what is too large for both): x = hi + lo, two f16 parts (about 22 bits), split once per
-// element by split_x_precise_kernel; per 32 x 32 tile and block four v_mfma_f32_32x32x16_f16.
+// gemm_ring.hip, gemm_precise_kernel for what is too large for both): x = hi + lo, two f16 parts (about
+// 22 bits), split once per element by split_x_precise_kernel; per 32 x 32 tile and block four v_mfma_f32_32x32x16_f16.
 //
 // gemm_kernel (FH_PATH_TILED_FAST, the scoring GEMM, within |g - w| <= 1e-3 + 2e-3 |w|): x = hi
 // + lo with hi in f16 and lo kept as e4m3 (about 15 bits in all). Per tile and block two f16
@@ -21,7 +21,8 @@
 // power-of-two scales (x lo: per row and 32-element block; the operand: per column) the
 // instruction applies itself, so the correction accumulates over all of K with no per-block work.
 // That is 1.5 f16-equivalent passes instead of 2. split_x_kernel prepares hi, lo and the scales
-// (the layouts are in xsplit.hpp).
+// (the layouts are in xsplit.hpp). A single product whose ring kernel's workgroups run at once takes
+// the precise product instead.
 //
 // k order inside a block (f16 operands): fast_elem_of_pos (xsplit.hpp), the order the quant
 // unpack produces. The MFMA sums over k, so x is laid out in that same order and no shuffle is
@@ -151,14 +152,16 @@ __global__ __launch_bounds__(256) void make_b8_kernel(const uint8_t *__restrict_
 
 // ---- x -> (hi, lo) f16, per block in operand order: xs[m][b] = 32 hi halves then 32 lo ----
 // Eight lanes per (row, block), lane j loading elements 4j..4j+3 (a wavefront reads 1 KiB of
-// contiguous x per instruction). |x| beyond the f16 range saturates hi (|x| < 65504 is exact). zero: floats
-// a product with two K splits adds into.
+// contiguous x per instruction). |x| beyond the f16 range saturates hi (|x| < 65504 is exact), and lo too with SAT
+// (the fast path's products, which stay finite for any x). zero: floats a product with two K splits adds into.
+template <bool SAT>
 __device__ __forceinline__ void split1(float e, _Float16 &h, _Float16 &l) {
     h = (_Float16)fminf(fmaxf(e, -65504.0f), 65504.0f);
-    l = (_Float16)(e - (float)h);
+    const float r = e - (float)h;
+    l = (_Float16)(SAT ? fminf(fmaxf(r, -65504.0f), 65504.0f) : r);
 }
 
-template <int KIND>
+template <int KIND, bool SAT = false>
 __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__restrict__ x, _Float16 *__restrict__ xs,
                                                       size_t items, float *__restrict__ zero, size_t zeros) {
     const int j = threadIdx.x % 8;
@@ -173,7 +176,7 @@ __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__res
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 _Float16 h, l;
-                split1(e[q], h, l);
+                split1<SAT>(e[q], h, l);
                 hi[q] = h;
                 lo[q] = l;
             }
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__res
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 _Float16 h, l;
-                split1(e[q], h, l);
+                split1<SAT>(e[q], h, l);
                 hi[q] = h;
                 lo[q] = l;
             }
@@ -213,7 +216,7 @@ __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__res
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 _Float16 h, l;
-                split1(e[q], h, l);
+                split1<SAT>(e[q], h, l);
                 part[q] = j < 4 ? h : l;
             }
             *(f16x8 *)(out + (j < 4 ? 0 : 32) + 8 * (j % 4)) = part;
@@ -2141,11 +2144,15 @@ hipError_t gemm_ext_dispatch(hipStream_t s, const _Float16 *xs, const uint8_t *w
 }
 
 // ---- the dequant-f16 GEMM (FH_PATH_TILED_F16): weights dequantised into LDS, plain f16 MFMA ----
+// (Smaller products take the ring kernel with the same x and exact quants, by f16_ring.)
 // x -> f16 of x 2^-s per row (2^s puts the row's largest |x| in [2^14, 2^15), so no element
-// overflows and every one keeps f16's 11 bits), in operand order, and xs[m] = 2^s.
+// overflows and every one keeps f16's 11 bits), in operand order, and xs[m] = 2^s. zero: rows of `zeros` floats that a
+// product with two K splits adds into.
 template <int KIND>
 __global__ __launch_bounds__(256) void split_x_f16_kernel(const float *__restrict__ x, _Float16 *__restrict__ xh,
-                                                          float *__restrict__ xs, uint32_t K) {
+                                                          float *__restrict__ xs, uint32_t K, float *__restrict__ zero,
+                                                          uint32_t zeros) {
+    for (uint32_t i = threadIdx.x; i < zeros; i += 256) zero[(size_t)blockIdx.x * zeros + i] = 0.0f;
     // The row is read once: thread t keeps float4 t + 256 i for i < kKeep in registers (rows up to
     // 8192 wide; wider rows read the rest twice). Float4 q is elements 4 (q % 8) .. + 3 of block
     // q / 8, so eight consecutive lanes hold one block.
@@ -2627,12 +2634,6 @@ hipError_t run_gemm_f16(hipStream_t s, const GemmF16Args &g) {
     return hipGetLastError();
 }
 
-// tile shape by rows
-void f16_tile(size_t rows, size_t *bm, size_t *bn) {
-    *bm = rows <= 32 ? 32 : rows <= 64 ? 64 : 128;
-    *bn = 256;
-}
-
 // The 256 x 256 kernel's plan: taken when the product has at least 128 such tiles; the K split
 // (at most 4, at least 8 stages per split) that best fills whole rounds of one CTA per CU.
 bool f16_big_plan(size_t rows, size_t k, size_t n, uint32_t *splits) {
@@ -2682,8 +2683,6 @@ template <int KIND>
 hipError_t gemm_f16_dispatch(hipStream_t s, const GemmF16Args &g) {
     uint32_t sp = 1;
     if (f16_big_plan(g.M, g.K, g.N, &sp)) return run_gemm_f16_big<KIND>(s, g, sp);
-    if (g.M <= 32) return run_gemm_f16<KIND, 32, 256>(s, g);
-    if (g.M <= 64) return run_gemm_f16<KIND, 64, 256>(s, g);
     return run_gemm_f16<KIND, 128, 256>(s, g);
 }
 
@@ -2742,6 +2741,8 @@ size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n) {
     return sp > 1 ? (size_t)sp * rows * n * 4 : 0;
 }
 
+bool gemm_precise_ring(size_t rows, size_t k, size_t n) { return precise_plan(rows, k, n).kernel == PrecisePlan::RING; }
+
 // x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned; parts false: for a
 // call without `defer`, whose ring splits add into y)
 size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts) {
@@ -2751,7 +2752,7 @@ size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts)
 
 hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x,
                                float *y, size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer,
-                               float *partial) {
+                               float *partial, bool saturate) {
     _Float16 *xs = (_Float16 *)workspace;
     if (!gemm_precise_partial_bytes(rows, k, n))
         partial = nullptr;
@@ -2762,11 +2763,17 @@ hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, c
     const PrecisePlan plan = precise_plan(rows, k, n);  // two ring splits add into y, zeroed by the x split
     const size_t zeros = plan.kernel == PrecisePlan::RING && plan.splits > 1 && !defer ? rows * n : 0;
     if (kind == FH_Q8_0) {
-        if (x) split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+        if (x && saturate)
+            split_x_precise_kernel<FH_Q8_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+        else if (x)
+            split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
         return gemm_precise_dispatch<FH_Q8_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                               defer);
     }
-    if (x) split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    if (x && saturate)
+        split_x_precise_kernel<FH_Q4_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    else if (x)
+        split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
     return gemm_precise_dispatch<FH_Q4_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                           defer);
 }
@@ -2912,15 +2919,26 @@ hipError_t launch_gemm_swiglu(hipStream_t s, fh_kind kind, const uint8_t *qs, co
 }
 
 // x as f16 (2 bytes per element), the row scales, then the K-split partials, each 256-aligned
+// Whether the ring kernel (gemm_ring.hip, x in one part) takes an f16 product: within its 32-bit offsets, but not
+// where the 256 x 256 kernel fills rounds of the chip better: 2.2 us a stage of 64 k and round, 6 us of its own,
+// and the reduction pass when K is split (4 bytes per output and part at 4 TB/s). Measured, us, Q8_0, 128 x 256 tiles
+// or 256 x 256 / ring: 100 rows 2048 x 2560 38 / 14, 300 rows 5632 x 2048 51 / 32, 1024 rows 2048 x 11264 126 / 100,
+// 2048 rows 5632 x 2048 100 / 85; 2048 rows 2048 x 11264 176 / 197, 1024 rows 896 x 9728 41 / 60, 4096 rows 217 / 367.
+static bool f16_ring(size_t rows, size_t k, size_t n) {
+    if (!ring_supported(rows, k, n)) return false;
+    uint32_t sp = 1;
+    if (!f16_big_plan(rows, k, n, &sp)) return true;
+    const uint64_t tiles = (uint64_t)((rows + 255) / 256) * ((n + 255) / 256), rounds = (tiles * sp + 255) / 256;
+    const uint64_t per = (((k / 32 + 1) / 2 + sp - 1) / sp + 1) & ~1ull;
+    const float us = 2.2f * (float)(rounds * per) + 6.0f + (sp > 1 ? (float)(sp + 1) * (float)rows * (float)n * 1e-6f : 0.0f);
+    return ring_f16_us(rows, k, n) < us;
+}
+
 size_t gemm_f16_workspace_bytes(size_t rows, size_t k, size_t n) {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     uint32_t sp = 1;
-    if (!f16_big_plan(rows, k, n, &sp)) {
-        size_t bm, bn;
-        f16_tile(rows, &bm, &bn);
-        const uint64_t tiles = (uint64_t)((rows + bm - 1) / bm) * ((n + bn - 1) / bn);
-        sp = gemm_splits(tiles, (uint32_t)((k / 32 + 1) / 2));
-    }
+    if (!f16_ring(rows, k, n) && !f16_big_plan(rows, k, n, &sp))
+        sp = gemm_splits((uint64_t)((rows + 127) / 128) * ((n + 255) / 256), (uint32_t)((k / 32 + 1) / 2));
     return up(rows * k * 2) + up(rows * 4) + (sp > 1 ? (size_t)sp * rows * n * 4 : 0);
 }
 
@@ -2946,12 +2964,17 @@ hipError_t launch_gemm_f16(hipStream_t s, fh_kind kind, const uint8_t *qs, const
     g.K = (uint32_t)k;
     g.N = (uint32_t)n;
     g.defer = defer;
-    if (kind == FH_Q8_0) {
-        split_x_f16_kernel<FH_Q8_0><<<(unsigned)rows, 256, 0, s>>>(x, (_Float16 *)g.xh, (float *)g.xs, g.K);
-        return gemm_f16_dispatch<FH_Q8_0>(s, g);
+    const bool ring = f16_ring(rows, k, n);
+    const uint32_t zeros = ring && ring_f16_splits(rows, k, n) > 1 ? g.N : 0;
+    if (kind == FH_Q8_0)
+        split_x_f16_kernel<FH_Q8_0><<<(unsigned)rows, 256, 0, s>>>(x, (_Float16 *)g.xh, (float *)g.xs, g.K, y, zeros);
+    else
+        split_x_f16_kernel<FH_Q4_0><<<(unsigned)rows, 256, 0, s>>>(x, (_Float16 *)g.xh, (float *)g.xs, g.K, y, zeros);
+    if (ring) {
+        if (defer) *defer = SplitOut{y, 1u};
+        return launch_gemm_ring_f16(s, kind, g.xh, g.xs, qs, ds, y, g.M, g.K, g.N);
     }
-    split_x_f16_kernel<FH_Q4_0><<<(unsigned)rows, 256, 0, s>>>(x, (_Float16 *)g.xh, (float *)g.xs, g.K);
-    return gemm_f16_dispatch<FH_Q4_0>(s, g);
+    return kind == FH_Q8_0 ? gemm_f16_dispatch<FH_Q8_0>(s, g) : gemm_f16_dispatch<FH_Q4_0>(s, g);
 }
 
 bool gemm_score_supported(fh_path path, size_t rows, size_t k, size_t n) {

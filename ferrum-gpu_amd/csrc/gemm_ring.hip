@@ -21,6 +21,9 @@
 // stage: behind it the stage's x has landed for everybody (each wavefront first waits for its own
 // loads, counted: loads complete in order) and the slot read in the stage before may be filled again.
 //
+// The f16 product (FH_PATH_TILED_F16) runs here too, with x in one part (64 bytes per row and block, two MFMAs
+// per tile and block: 0.8 us a stage) and a row scale at the end.
+//
 // Measured (us, x split included, the 128 x 128 kernel and its reduction before / now, Q4_0): 512 rows 2048 x
 // 2560 35.8 / 28.7, 2048 x 2048 34.5 / 26.2, 2048 x 11264 99.8 / 68.8, 5632 x 2048 54.4 / 41.2, 896 x 1152
 // 28.0 / 13.8; 96 rows 2048 x 2560 27.2 / 14.0. GGUF rows (gemm_ext_kernel, one stage ahead through registers,
@@ -51,31 +54,33 @@ namespace {
 // would take 64 a load, 192 cycles of a stage's 2400 for each of eight wavefronts). In registers a lane shifts its
 // dwords to the byte with v_perm and the hardware converts the codes to f16, exactly.
 // KG groups of wavefronts share K (4 pairs and a 128-column tile, or 2 fours and a 256-column tile).
-template <int KIND, int MTW, int KG>
+template <int KIND, int MTW, int KG, int XP = 2>
 struct Ring {
     static constexpr int WPG = 8 / KG, BN = 64 * WPG;  // wavefronts of a group
     static constexpr uint32_t QB = KIND == FH_F16 ? 64 : KIND == FH_Q4_0 ? 16 : 32;
-    static constexpr uint32_t X = 32 * MTW * 128;  // bytes of a group's stage: x,
+    static constexpr uint32_t XB = 64 * XP;         // bytes of an x row and block
+    static constexpr uint32_t X = 32 * MTW * XB;   // bytes of a group's stage: x,
     static constexpr uint32_t WQ = 64 * QB;        // a wavefront's quants
     static constexpr uint32_t D = KIND == FH_F16 || KIND == FH_MXFP4 ? 0 : 256;
     static constexpr uint32_t W = WQ + D;          // and its scale (FP8: last) dwords
     static constexpr uint32_t GROUP = X + WPG * W, STAGE = KG * GROUP;
-    static constexpr int XL = 4 * MTW / WPG;                         // x load instructions of a wavefront (1 KB each)
+    static constexpr int XL = X / 1024 / WPG;                        // x load instructions of a wavefront (1 KB each)
     static constexpr int LOADS = XL + WQ / 1024 + D / 256;  // load instructions per wavefront and stage
     static constexpr int NS = 163840 / STAGE < 6 ? 163840 / STAGE : 6;
     static constexpr uint32_t SUMS = 8 * MTW * 8192;  // the wavefronts' sums (after the loop)
     static constexpr uint32_t LDS = NS * STAGE > SUMS ? NS * STAGE : SUMS;
-    static_assert(NS >= 3 && (NS - 1) * LOADS < 64 && LDS <= 163840, "ring size");
+    static_assert(XL >= 1 && NS >= 3 && (NS - 1) * LOADS < 64 && LDS <= 163840, "ring size");
 };
 
 // ADD: the workgroup's sums are added into y (two K splits onto zeros); else stored, split blockIdx.y at
 // y + blockIdx.y M N.
-template <int KIND, int MTW, int KG, bool ADD>
+// XP: x parts, 2 (the precise product) or 1 (the f16 product: rows of x scaled to f16, output rows times rs).
+template <int KIND, int MTW, int KG, bool ADD, int XP = 2>
 __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__restrict__ xs, const uint8_t *__restrict__ qs,
                                                            const uint16_t *__restrict__ ds, float *__restrict__ y,
                                                            uint32_t M, uint32_t K, uint32_t N, uint32_t mt, uint32_t nt,
-                                                           uint32_t split_stages) {
-    using R = Ring<KIND, MTW, KG>;
+                                                           uint32_t split_stages, const float *__restrict__ rs) {
+    using R = Ring<KIND, MTW, KG, XP>;
     constexpr int BM = 32 * MTW, NS = R::NS;
     __shared__ __attribute__((aligned(1024))) uint8_t arena[R::LDS];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t *)arena;
@@ -95,9 +100,10 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
     // Loads of block b into ring slot `slot`. Rows past M and columns past the padded weight rows fall past
     // their resource's end by their offsets alone and read 0; a block past the split reads 0 through empty
     // resources (the count of loads in flight stays the same).
-    const uint32_t xrow = 8 * R::XL * wn + lane / 8;  // instruction i: rows 8 i further
+    constexpr uint32_t XR = 1024 / R::XB, XC = R::XB / 16;  // rows of an x instruction, 16-byte chunks of a row
+    const uint32_t xrow = XR * R::XL * wn + lane / XC;      // instruction i: rows XR i further
     const uint32_t g0 = n0 / 32 + 2 * wn;            // the wavefront's first group of 32 columns
-    const uint32_t xoff = (m0 + xrow) * nb * 128, ncol = n0 + 64 * wn + lane;
+    const uint32_t xoff = (m0 + xrow) * nb * R::XB, ncol = n0 + 64 * wn + lane;
     const uint32_t woff = KIND == FH_Q8_0 ? g0 * nb * 1024 + (lane % 32) * 32 + (lane / 32) * 16
                                           : (g0 + lane / 32) * nb * 512 + (lane % 32) * 16;
     const uint32_t doff = (ncol >> 5) * nb8 * 512 + (ncol & 31) * 16;
@@ -115,6 +121,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
         // the byte of block b's start in its first dword: (bits 16 j .. of gsh) + b GB, modulo 4
         gsh = (min(n0 + 64 * wn + fr, N - 1) * nb * GB & 3) | (min(n0 + 64 * wn + 32 + fr, N - 1) * nb * GB & 3) << 16;
     }
+    auto xswap = [](uint32_t r) { return XP == 2 ? (r >> 1) & 7 : (r >> 2) & 3; };
     auto dma = [&](uint32_t b, uint32_t slot, int part) {  // part 0: weights and scales; 1: x
         const bool live = b < st1;
         const uint32_t x0 = lds0 + slot * R::STAGE + kg * R::GROUP, w0 = x0 + R::X + wn * R::W;
@@ -138,13 +145,11 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
             asm_load_lds4(rd, w0 + R::WQ, doff + (b / 8) * 512 + (b % 8) / 2 * 4);
             return;
         }
-        const i32x4 rx = sgpr_rsrc(xs, live ? M * nb * 128 : 0u);
+        const i32x4 rx = sgpr_rsrc(xs, live ? M * nb * R::XB : 0u);
 #pragma unroll
-        for (int i = 0; i < R::XL; i++) {
-            const uint32_t r = xrow + 8 * i;
-            asm_load_lds16(rx, x0 + 8 * (R::XL * wn + i) * 128,
-                           xoff + 8 * i * nb * 128 + b * 128 + ((lane % 8) ^ ((r >> 1) & 7)) * 16);
-        }
+        for (int i = 0; i < R::XL; i++)
+            asm_load_lds16(rx, x0 + 1024 * (R::XL * wn + i),
+                           xoff + XR * i * nb * R::XB + b * R::XB + ((lane % XC) ^ xswap(xrow + XR * i)) * 16);
     };
 
     f32x16 acc[MTW][2];
@@ -158,7 +163,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
     // One stage's operands in registers: x fragments (hi and lo, k16 steps 0 and 1), the packed quants of the
     // lane's share of the two column tiles, their scale dwords (blocks b & ~1 and b | 1).
     struct Frag {
-        f16x8 h[MTW][2], l[MTW][2];
+        f16x8 h[MTW][2], l[MTW][XP == 2 ? 2 : 1];
         u32x2 q[2][KIND == FH_Q8_0 ? 2 : 1];
         u32x4 g[2][2];  // GGUF rows: the lane's dwords
         uint32_t e[2], d[2];
@@ -197,12 +202,12 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
     };
     auto read_x = [&](Frag &f, uint32_t slot, int i) {
         const uint32_t r = i * 32 + fr;
-        const uint8_t *row = arena + slot * R::STAGE + kg * R::GROUP + r * 128;
+        const uint8_t *row = arena + slot * R::STAGE + kg * R::GROUP + r * R::XB;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             const uint32_t c = kGguf<KIND> ? 2 * hf + s : hf + 2 * s;  // (GGUF rows: a lane's codes are consecutive)
-            f.h[i][s] = *(const f16x8 *)(row + ((c ^ ((r >> 1) & 7)) * 16));
-            f.l[i][s] = *(const f16x8 *)(row + (((4 + c) ^ ((r >> 1) & 7)) * 16));
+            f.h[i][s] = *(const f16x8 *)(row + (c ^ xswap(r)) * 16);
+            if constexpr (XP == 2) f.l[i][s] = *(const f16x8 *)(row + ((4 + c) ^ xswap(r)) * 16);
         }
     };
     // Column tile j of block blk: exact f16 values; returns the block's scale. A block that holds an infinity or
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
             if (v == V) dma(b + KG * NS, slot, 1);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                if (v < V)
+                if (v < V && s < 2 * XP)
                     q = __builtin_amdgcn_mfma_f32_32x32x16_f16(s < 2 ? f.h[i][s] : f.l[i][s - 2], bq[j][s % 2], q, 0, 0, 0);
                 if (v > 0) {
 #pragma unroll
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
             if (v > 0) asm volatile("" : "+v"(acc[ip][jp]));  // the FMAs stay here
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                if (v < V) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (v < V && s < 2 * XP) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 if (v == 0)
                     __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
                 else if (v < V)
@@ -379,6 +384,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
         for (int p = 1; p < KG; p++) v += sums[p * PART + e * 64 + lane];
         const uint32_t row = m0 + i * 32 + 8 * (r / 4) + 4 * hf + r % 4, col = n0 + 64 * h + j * 32 + fr;
         if (row < M && col < N) {
+            if constexpr (XP == 1) v *= rs[row];
             if (ADD)
                 unsafeAtomicAdd(y + (size_t)row * N + col, v);
             else
@@ -399,13 +405,14 @@ struct RingPlan {
     uint32_t mtw, kg, splits;
     float us;
 };
-static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n) {
+static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n, int xp = 2) {
     const size_t nb = k / 32;
-    const float f = kind == FH_F16 ? 1.3f : kind == FH_MXFP4 ? 1.15f : kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 ? 1.25f : 1.0f;
+    const float f = kind == FH_F16 ? 1.3f : kind == FH_MXFP4 ? 1.15f : kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 ? 1.25f : xp == 1 ? 0.8f : 1.0f;
     RingPlan best{1, 4, 1, INFINITY};
     for (uint32_t mtw : {2u, 1u})
         for (uint32_t kg : {4u, 2u})
             for (uint32_t sp : {1u, 2u}) {
+                if (xp == 1 && mtw == 1 && kg == 2) continue;
                 if (mtw == 2 && (rows <= 32 || (kind == FH_F16 && kg == 4))) continue;  // (that stage does not fit LDS three times)
                 const uint64_t tiles = (rows + 32 * mtw - 1) / (32 * mtw) * ((n + 512 / kg - 1) / (512 / kg));
                 if (sp == 2 && (tiles > 128 || nb < 4 * kg)) continue;
@@ -420,6 +427,11 @@ static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n) {
 uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n) { return ring_plan(kind, rows, k, n).splits; }
 float ring_us(int kind, size_t rows, size_t k, size_t n) { return ring_plan(kind, rows, k, n).us; }
 
+bool ring_one_round(size_t rows, size_t k, size_t n) {
+    const RingPlan p = ring_plan(FH_Q8_0, rows, k, n);
+    return (rows + 32 * p.mtw - 1) / (32 * p.mtw) * ((n + 512 / p.kg - 1) / (512 / p.kg)) * p.splits <= 256;
+}
+
 bool ring_supported(size_t rows, size_t k, size_t n) {
     // every byte offset a workgroup forms (rows and columns up to the last tile's end) fits in 32 bits
     const size_t lim = (size_t)1 << 31;
@@ -429,17 +441,17 @@ bool ring_gguf_supported(int kind, size_t rows, size_t k, size_t n) {
     return kind != FH_Q2_K && ring_supported(rows, k, n) && n * (k / 32) * 64 + 128 < ((size_t)1 << 31);
 }
 
-template <int KIND, int MTW, int KG>
+template <int KIND, int MTW, int KG, int XP = 2>
 static hipError_t run_ring(hipStream_t s, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out, uint32_t M,
-                           uint32_t K, uint32_t N, uint32_t sp, bool add) {
-    constexpr uint32_t BN = Ring<KIND, MTW, KG>::BN;
+                           uint32_t K, uint32_t N, uint32_t sp, bool add, const float *rs = nullptr) {
+    constexpr uint32_t BN = Ring<KIND, MTW, KG, XP>::BN;
     const uint32_t mt = (M + 32 * MTW - 1) / (32 * MTW), nt = (N + BN - 1) / BN, nb = K / 32;
     const dim3 grid((mt * nt + 7) / 8 * 8, sp);
     const uint32_t per = ((nb + sp - 1) / sp + KG - 1) / KG * KG;
     if (add)
-        gemm_ring_kernel<KIND, MTW, KG, true><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per);
+        gemm_ring_kernel<KIND, MTW, KG, true, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, rs);
     else
-        gemm_ring_kernel<KIND, MTW, KG, false><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per);
+        gemm_ring_kernel<KIND, MTW, KG, false, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, rs);
     return hipGetLastError();
 }
 
@@ -453,6 +465,23 @@ static hipError_t run_ring_kind(hipStream_t s, const _Float16 *xs, const uint8_t
     if constexpr (KIND != FH_F16)
         if (p.kg == 4) return run_ring<KIND, 2, 4>(s, xs, qs, ds, out, M, K, N, sp, add);
     return run_ring<KIND, 2, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
+}
+
+template <int KIND>
+static hipError_t run_ring_f16(hipStream_t s, const _Float16 *xs, const float *rs, const uint8_t *qs, const uint16_t *ds,
+                               float *out, uint32_t M, uint32_t K, uint32_t N) {
+    const RingPlan p = ring_plan(KIND, M, K, N, 1);
+    const bool add = p.splits > 1;
+    if (p.mtw == 1) return run_ring<KIND, 1, 4, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, rs);
+    if (p.kg == 4) return run_ring<KIND, 2, 4, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, rs);
+    return run_ring<KIND, 2, 2, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, rs);
+}
+float ring_f16_us(size_t rows, size_t k, size_t n) { return ring_plan(FH_Q8_0, rows, k, n, 1).us; }
+uint32_t ring_f16_splits(size_t rows, size_t k, size_t n) { return ring_plan(FH_Q8_0, rows, k, n, 1).splits; }
+hipError_t launch_gemm_ring_f16(hipStream_t s, int kind, const _Float16 *xs, const float *rs, const uint8_t *qs,
+                                const uint16_t *ds, float *out, uint32_t M, uint32_t K, uint32_t N) {
+    return kind == FH_Q8_0 ? run_ring_f16<FH_Q8_0>(s, xs, rs, qs, ds, out, M, K, N)
+                           : run_ring_f16<FH_Q4_0>(s, xs, rs, qs, ds, out, M, K, N);
 }
 
 hipError_t launch_gemm_ring(hipStream_t s, int kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,

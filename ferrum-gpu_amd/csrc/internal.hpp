@@ -301,6 +301,7 @@ hipError_t launch_gemm_f16(hipStream_t s, fh_kind kind, const uint8_t *qs, const
                            size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer = nullptr);
 // The precise MFMA GEMM (x as two f16 parts; split into workspace, then the product).
 size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts = true);
+bool gemm_precise_ring(size_t rows, size_t k, size_t n);  // whether the ring kernel takes the precise product
 // The MFMA GEMM on the GGUF rows of F16, FP8 E4M3 / E5M2, MXFP4 and Q2_K weights (rows >= 2) and
 // its workspace (x split, then the K-split partial products).
 bool gemm_ext_kind(int kind);
@@ -311,15 +312,21 @@ hipError_t launch_gemm_ext(hipStream_t s, int kind, const uint8_t *w, const floa
 // partial != nullptr: the K-split partial products go there (as launch_gemm's).
 hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x,
                                float *y, size_t rows, size_t k, size_t n, void *workspace,
-                               SplitOut *defer = nullptr, float *partial = nullptr);
+                               SplitOut *defer = nullptr, float *partial = nullptr, bool saturate = false);
 size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n);
 // gemm_ring.hip: the precise product alone on split x (of split_x_precise_kernel's order for the kind): `splits`
 // (1 or 2) partial products of M x N at out, or (add) their sum added to zeros at out. Kinds other than
 // Q8_0 and Q4_0 (ring_gguf_supported): qs is the GGUF rows.
 uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n);
 float ring_us(int kind, size_t rows, size_t k, size_t n);  // its time by the plan's model
+bool ring_one_round(size_t rows, size_t k, size_t n);  // no more workgroups than CUs
 bool ring_supported(size_t rows, size_t k, size_t n);
 bool ring_gguf_supported(int kind, size_t rows, size_t k, size_t n);
+// The f16 product: x in one f16 part, its rows scaled; output rows times rs; added to zeros at out where K is split.
+float ring_f16_us(size_t rows, size_t k, size_t n);
+uint32_t ring_f16_splits(size_t rows, size_t k, size_t n);
+hipError_t launch_gemm_ring_f16(hipStream_t s, int kind, const _Float16 *xs, const float *rs, const uint8_t *qs,
+                                const uint16_t *ds, float *out, uint32_t M, uint32_t K, uint32_t N);
 hipError_t launch_gemm_ring(hipStream_t s, int kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
                             uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add);
 

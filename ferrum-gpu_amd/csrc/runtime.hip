@@ -840,8 +840,16 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         if (fixed && rows && !w->b8)
             return fail(FH_ERR_INVALID, "linear_q_noalloc: the fast GEMM needs the weight's correction operand, "
                                         "which its first multi-row FH_PATH_TILED_FAST linear_q builds");
+        // The precise product where its ring kernel's workgroups run at once: the faster one there, and closer (us, Q8_0 and
+        // Q4_0, fast / ring: 100 rows 2048 x 2560 25.5 and 25.2 / 13.3 and 13.8, 300 rows 2048 x 11264 53 and 51 / 43 and
+        // 45, 1024 rows 5632 x 2048 79 and 79 / 64 and 63, 2048 rows 1024 x 2048 38.5 and 37.9 / 32.5 and 33.5; past one
+        // round 1024 rows 2048 x 5632 81 and 68 / 75 and 76). Its scratch must fit where the fast one's does.
+        const size_t pbytes = gemm_precise_workspace_bytes(rows, w->k, w->n, false);
+        const bool precise = rows && rows <= 2048 && gemm_precise_ring(rows, w->k, w->n) && ring_one_round(rows, w->k, w->n) &&
+                             (!fixed || pbytes <= FH_NOALLOC_SCRATCH_BYTES);
         void *ws = nullptr;
-        if (rows && (st = command_scratch(dev, fixed, gemm_workspace_bytes(rows, w->k, w->n), &ws))) return st;
+        if (rows && (st = command_scratch(dev, fixed, precise ? pbytes : gemm_workspace_bytes(rows, w->k, w->n), &ws)))
+            return st;
         void *fresh = nullptr;  // the correction operand, built within the weight's first multi-row command
         if (rows && !w->b8 && (st = alloc_bytes(dev, gemm_b8_bytes(w->k, w->n), &fresh))) return st;
         if ((st = begin_command(dev, "linear_q"))) {
@@ -852,7 +860,10 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
             (void)launch_make_b8(dev->stream, w->kind, w->qs, w->ds, (uint8_t *)fresh, w->k, w->n);
             w->b8 = (uint8_t *)fresh;
         }
-        if (rows) (void)launch_gemm(dev->stream, w->kind, w->qs, w->ds, w->b8, x, y, rows, w->k, w->n, ws);
+        if (precise)
+            (void)launch_gemm_precise(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws, nullptr, nullptr, true);
+        else if (rows)
+            (void)launch_gemm(dev->stream, w->kind, w->qs, w->ds, w->b8, x, y, rows, w->k, w->n, ws);
         return end_command(dev, "linear_q");
     }
     case FH_PATH_TILED_F16: {

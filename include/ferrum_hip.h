@@ -82,10 +82,11 @@ typedef enum fh_kind {
  * row), TILED = the LDS-staged MFMA dequant-GEMM (any rows; x carried to about 22 bits, within the
  * reference's 1e-5 product tolerance), AUTO = fh_choose. No counterpart in the reference:
  * TILED_FAST = the scoring GEMM (x as f16 plus an fp8 correction on the fp8 matrix cores; within
- * the MFMA-GEMM tolerance |g - w| <= 1e-3 + 2e-3 |w|, about 5e-5 absolute at the scoring shapes);
+ * the MFMA-GEMM tolerance |g - w| <= 1e-3 + 2e-3 |w|, about 5e-5 absolute at the scoring shapes;
+ * a single product of up to some hundreds of rows runs TILED's kernel, which is faster there);
  * TILED_F16 = the dequant-f16 GEMM (weights dequantised to f16 d*q in LDS, x as f16 with a
  * power-of-two row scale, plain f16 MFMA with f32 accumulation; each product rounds both operands
- * to f16, so |g - w| <= 2^-10 sum_k |x_k w_k| roughly: it does NOT meet the MFMA-GEMM tolerance
+ * to f16, or x alone where the product is small enough for the ring kernel, so |g - w| <= 2^-10 sum_k |x_k w_k| roughly: it does NOT meet the MFMA-GEMM tolerance
  * per output; measured at the TinyLlama-1.1B shapes, M = 4096, 5.4e-5 (Q4_0) and 1.1e-4 (Q8_0)
  * of the outputs fall outside it, the worst at 1.8 to 2.0 times the bound);
  * ROWS = the few-row kernel for 2..64 rows (the weights streamed once from HBM into registers for

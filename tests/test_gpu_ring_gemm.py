@@ -77,3 +77,32 @@ def test_ring_product_of_gguf_rows(fh, g, orc, kind_name, k, n, rows):
         worst = float((err / np.maximum(bound, 1e-38)).max())
         print(f"{kind_name} {m} x {k} x {n}: {worst:.3f} of the bound", flush=True)
         assert np.all(err <= bound), (kind_name, k, n, m, worst)
+
+
+@pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
+@pytest.mark.parametrize("k,n,rows", [(32, 1, (2, 33)), (96, 65, (31, 33, 65)), (160, 129, (64, 130)),
+                                      (1056, 257, (33, 200)), (4896, 127, (17, 100)), (896, 9728, (300,)),
+                                      (2048, 2560, (1024,))])
+def test_ring_product_of_the_other_paths(fh, g, orc, kind_name, k, n, rows):
+    """TiledF16 (x in one f16 part, 11 bits of each element on its row's power-of-two scale: 2^-11 sum_k |x_k w_k|
+    beside the summation error; rows up to 1e8) and TiledFast, which takes the precise product here."""
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(k + n)
+    b = orc.quantise_matrix(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32), k, n)
+    w = orc.dequantised_in_out(int(kind), b, k, n).reshape(k, n).astype(np.float64)
+    qw = fh.upload_qweight(g, kind, b, k, n)
+    for m in rows:
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        for path, x, eps in ((fh.QPath.TiledFast, x, 0.0),
+                             (fh.QPath.TiledF16, x * (10.0 ** rng.integers(-6, 9, (m, 1))).astype(np.float32), 2.0**-11)):
+            gx, gy = g.upload(x), g.upload(np.full(m * n, np.nan, np.float32))
+            fh.linear_q_with(g, gx, qw, gy, m, path)
+            first = g.read(gy)
+            fh.linear_q_with(g, gx, qw, gy, m, path)
+            got = g.read(gy)
+            assert np.array_equal(first.view(np.uint32), got.view(np.uint32)), (kind_name, path, k, n, m)
+            bound = (eps + (k + 8) * 2.0**-24) * (np.abs(x).astype(np.float64) @ np.abs(w))
+            err = np.abs(got.reshape(m, n) - x.astype(np.float64) @ w)
+            worst = float((err / np.maximum(bound, 1e-38)).max())
+            print(f"{kind_name} {path.name} {m} x {k} x {n}: {worst:.3f} of the bound", flush=True)
+            assert np.all(err <= bound), (kind_name, path, k, n, m, worst)
