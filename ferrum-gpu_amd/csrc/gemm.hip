@@ -1669,6 +1669,7 @@ struct PrecisePlan {
     uint32_t splits;
 };
 PrecisePlan precise_plan(size_t rows, size_t k, size_t n) {
+    rows = (rows + 31) / 32 * 32;  // one plan for the rows of a 32-row tile (llama.hip sizes its workspace by them)
     const bool ring = ring_supported(rows, k, n);
     uint32_t sp = 1;
     if (stream_plan(rows, k, n, &sp) && stream_supported(rows, k, n)) {
@@ -2925,6 +2926,7 @@ hipError_t launch_gemm_swiglu(hipStream_t s, fh_kind kind, const uint8_t *qs, co
 // or 256 x 256 / ring: 100 rows 2048 x 2560 38 / 14, 300 rows 5632 x 2048 51 / 32, 1024 rows 2048 x 11264 126 / 100,
 // 2048 rows 5632 x 2048 100 / 85; 2048 rows 2048 x 11264 176 / 197, 1024 rows 896 x 9728 41 / 60, 4096 rows 217 / 367.
 static bool f16_ring(size_t rows, size_t k, size_t n) {
+    rows = (rows + 31) / 32 * 32;  // (as precise_plan)
     if (!ring_supported(rows, k, n)) return false;
     uint32_t sp = 1;
     if (!f16_big_plan(rows, k, n, &sp)) return true;

@@ -407,6 +407,7 @@ struct RingPlan {
 };
 static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n, int xp = 2) {
     const size_t nb = k / 32;
+    rows = (rows + 31) / 32 * 32;  // (one plan for the rows of a 32-row tile)
     const float f = kind == FH_F16 ? 1.3f : kind == FH_MXFP4 ? 1.15f : kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 ? 1.25f : xp == 1 ? 0.8f : 1.0f;
     RingPlan best{1, 4, 1, INFINITY};
     for (uint32_t mtw : {2u, 1u})

@@ -1310,13 +1310,22 @@ fh_status ensure_rows(fh_llama *m, size_t t) {
     const bool fast = m->path == FH_PATH_TILED_FAST;
     const std::pair<size_t, size_t> prods[] = {{t, d}, {t, qd}, {t, hid}, {chunk, d}};
     const std::pair<size_t, size_t> kns[] = {{d, w}, {qd, d}, {d, 2 * hid}, {hid, d}};
+    // The arena serves every later call of up to t rows, and fewer rows may split K more ways: the largest need of
+    // any row count (the plans change at multiples of 32 rows).
+    auto most = [](size_t rows, auto &&bytes) {
+        size_t b = bytes(rows);
+        for (size_t r = 32; r < rows; r += 32) b = std::max(b, bytes(r));
+        return b;
+    };
     if (fast) {
         for (auto rk : prods) ws = std::max(ws, gemm_xsplit_bytes(rk.first, rk.second));
-        for (auto kn : kns) part = std::max(part, gemm_partial_bytes(t, kn.first, kn.second));
-        part = std::max(part, gemm_partial_bytes(chunk, d, m->vocab));
+        for (auto kn : kns)
+            part = std::max(part, most(t, [&](size_t r) { return gemm_partial_bytes(r, kn.first, kn.second); }));
+        part = std::max(part, most(chunk, [&](size_t r) { return gemm_partial_bytes(r, d, m->vocab); }));
     } else {
-        for (auto kn : kns) ws = std::max(ws, linear_ws(m, t, kn.first, kn.second));
-        ws = std::max(ws, linear_ws(m, chunk, d, m->vocab));
+        for (auto kn : kns)
+            ws = std::max(ws, most(t, [&](size_t r) { return linear_ws(m, r, kn.first, kn.second); }));
+        ws = std::max(ws, most(chunk, [&](size_t r) { return linear_ws(m, r, d, m->vocab); }));
     }
     const size_t tp = (t + 31) / 32 * 32, kvd = m->kv_dim();
     const size_t split = split_attention(m) ? 2 * up256(tp * qd * 2) + 4 * up256(tp * kvd * 2) + up256(tp * m->heads) +
