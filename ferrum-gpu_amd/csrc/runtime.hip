@@ -843,10 +843,11 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         // The precise product where its ring kernel's workgroups run at once: the faster one there, and closer (us, Q8_0 and
         // Q4_0, fast / ring: 100 rows 2048 x 2560 25.5 and 25.2 / 13.3 and 13.8, 300 rows 2048 x 11264 53 and 51 / 43 and
         // 45, 1024 rows 5632 x 2048 79 and 79 / 64 and 63, 2048 rows 1024 x 2048 38.5 and 37.9 / 32.5 and 33.5; past one
-        // round 1024 rows 2048 x 5632 81 and 68 / 75 and 76). Its scratch must fit where the fast one's does.
+        // round 1024 rows 2048 x 5632 81 and 68 / 75 and 76), while its scratch, the larger one, fits the static array
+        // too (both entry points give the same bits).
         const size_t pbytes = gemm_precise_workspace_bytes(rows, w->k, w->n, false);
         const bool precise = rows && rows <= 2048 && gemm_precise_ring(rows, w->k, w->n) && ring_one_round(rows, w->k, w->n) &&
-                             (!fixed || pbytes <= FH_NOALLOC_SCRATCH_BYTES);
+                             pbytes <= FH_NOALLOC_SCRATCH_BYTES;
         void *ws = nullptr;
         if (rows && (st = command_scratch(dev, fixed, precise ? pbytes : gemm_workspace_bytes(rows, w->k, w->n), &ws)))
             return st;
