@@ -414,8 +414,8 @@ GPT2_SMALL = {"vocab": 50257, "ctx": 1024, "dim": 768, "heads": 12, "layers": 12
 def bench_decode(fh, g, n_prompt=32, n_new=256, reps=3, cpu=True):
     """GPT-2-small (GPT-2 initialisation, tied head) with Q8_0 weights, KV-cached
     greedy decode of n_new tokens from an n_prompt-token seeded uniform-random prompt. One rep is one
-    fh_gpt2_generate call from position 0 (the prompt is fed token by token, so a rep is
-    n_prompt + n_new - 1 decode steps); the median rep is reported."""
+    fh_gpt2_generate call from position 0 (the prompt's tokens but the last run as one pass, so a
+    rep is that pass and n_new decode steps, over which its time is spread); the median rep is reported."""
     from ferrum_hip.gguf import Gguf
     from ferrum_hip.gpt2 import GpuGpt2, gpt2_init, to_gguf
 
@@ -432,7 +432,7 @@ def bench_decode(fh, g, n_prompt=32, n_new=256, reps=3, cpu=True):
         toks = model.generate(prompt, n_new)
         times.append(time.perf_counter() - t0)
     t = float(np.median(times))
-    steps = n_prompt + n_new - 1
+    steps = n_new
     out = {"tok_s": n_new / t, "steps_per_s": steps / t, "ms_per_step": t / steps * 1e3,
            "weight_gbs": model.step_bytes() * steps / t / 1e9, "step_bytes": model.step_bytes(),
            "first_tokens": toks[:8], "reps": reps, "launches_per_step": model.step_launches()}
