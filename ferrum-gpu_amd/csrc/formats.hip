@@ -361,7 +361,7 @@ __global__ __launch_bounds__(256) void encode_blocks_kernel(const float *__restr
     }
 }
 
-// q2k.rs:16-150, one thread per super-block
+// q2k.rs:16-150
 __device__ __forceinline__ int32_t nearest_int(float x) {
     const float t = x + 12582912.0f;
     return (int32_t)(__float_as_uint(t) & 0x007fffffu) - 0x00400000;

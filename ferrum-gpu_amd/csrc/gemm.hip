@@ -1774,7 +1774,8 @@ hipError_t run_gemm_score(hipStream_t s, fh_path path, const void *xa, const uin
     return hipGetLastError();
 }
 
-// ---- the MFMA GEMM on the other weight formats' GGUF rows (F16, FP8 E4M3 / E5M2, MXFP4) ----
+// ---- the MFMA GEMM on the other weight formats' GGUF rows (F16, FP8 E4M3 / E5M2, MXFP4, Q2_K) ----
+// (All but Q2_K come here only where ext_ring says so; the ring kernel takes the rest.)
 // Every element of these formats is an f16-exact value times a per-32-block f32 scale: F16 its
 // own value (scale 1), E5M2 code c the f16 with bits c << 8 (fp8.rs:34-63), E4M3 code c the f16
 // with bits (c & 0x7f) << 7 | (c & 0x80) << 8 times 2^8 (normal and subnormal alike), MXFP4

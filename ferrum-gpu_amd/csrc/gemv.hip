@@ -315,7 +315,10 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
 // launch with few wavefronts, each a chain of many batches: 24 products of 4864 x 896 are 672 tasks of 19
 // batches for the chip's 2048 wavefronts (20.7 -> 14.1 us, 2.9 -> 4.2 TB/s). Every wavefront streams its batches of
 // the workgroup's tasks as gemv_kernel does, the next one in flight across task boundaries and across
-// the barrier that ends each task.
+// the barrier that ends each task. (us, a wavefront per task / this: 16 products of 5632 x 2048 Q4_0 26.7 / 21.2, Q8_0
+// 31.4 / 30.9; 195 of 4864 x 896 88.7 / 88.6. It loses where the tasks just fill the wavefronts of one round: 60 of
+// 4864 x 896 30.4 / 35.1, 4 of 8192 x 8192 Q8_0 44.4 / 53.4; a rule on the task count would break that
+// a grouped launch equals a launch of one product bit for bit.)
 template <int KIND>
 __global__ __launch_bounds__(256) void gemv_wide_kernel(const GemvDesc *__restrict__ descs,
                                                         const uint32_t *__restrict__ map, GemvDesc one, uint32_t count,
