@@ -880,7 +880,7 @@ def main():
         eg = bench_ext_gemm(fh, g, ev, ext_kinds(fh), EXT_GEMM_CASES)
         log("other formats, MFMA GEMM:", eg)
         extra["ext_formats_gemm"] = {
-            "kernel": "gemm_ext_kernel: x as two f16 parts, f16-exact decoded values times per-block f32 scales "
+            "kernel": "gemm_ring_kernel or gemm_ext_kernel: x as two f16 parts, f16-exact decoded values times per-block f32 scales "
                       "(Q2_K: per 16-element sub-block, minus dmin times the x sums) on f16 MFMA; x split included",
             "by_format": eg}
         codec = bench_codec(fh, g, ev)
