@@ -34,9 +34,10 @@ struct Fmt<FH_Q4_0> {
 };
 
 // The snap's quantisation step: from this lane's 4 values of a block held by 8 lanes, the 4 Q8_0 codes and the
-// f16 scale bits.
+// f16 scale bits. The maximum starts from 0, so a block of NaN alone has scale 0, as in the encode.
 __device__ __forceinline__ void quantise4(const f32x4 v, int32_t (&q)[4], uint32_t &h) {
-    const float amax = group_reduce<8>(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))), MaxOp());
+    const float m = fmaxf(fmaxf(fmaxf(0.0f, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w));
+    const float amax = group_reduce<8>(m, MaxOp());
     const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
     h = float_to_half_bits(d);
 #pragma unroll

@@ -1,6 +1,7 @@
 """The two-lanes-per-block encoders and the four-per-thread decoder against the oracle, byte for byte: part-filled
 workgroups (one block, one short of and one past a workgroup's 128), values at the midpoints of the code
-tables and one unit to either side, signed zeros, subnormal and huge scales, NaN and infinities."""
+tables and one unit to either side, signed zeros, subnormal and huge scales, NaN and infinities. The snap (decode of
+encode) of blocks with NaN and infinities likewise, by rows, by columns and in a plan."""
 import numpy as np
 import pytest
 
@@ -71,3 +72,49 @@ def test_encode_of_nan_and_infinity(fh, g, orc, kind):
     want = orc.encode(int(kind), x.reshape(-1))
     got = g.read_bytes(fh.encode(g, kind, g.upload(x.reshape(-1)), x.size))[: want.size]
     assert np.array_equal(got, want), np.flatnonzero(got != want)[:8] // (want.size // 160)
+
+
+def nonfinite():
+    """160 blocks: all NaN, NaN in some lanes' or one lane's values only, infinities, both, and finite ones between."""
+    x = blocks(160, 11)
+    x[0], x[63], x[127], x[128], x[159] = np.nan, -np.nan, np.nan, np.nan, np.nan
+    x[2, :4], x[3, 4:], x[64, ::2], x[65, 31], x[66, :16], x[67, 16:] = (np.nan,) * 6
+    x[9, 0], x[77, 16], x[78, 1] = np.inf, -np.inf, -np.inf
+    x[78, 2], x[79, 3] = np.nan, np.inf
+    x[79, 4:] = np.nan
+    return x
+
+
+def same(got, want, what):
+    """The bits of every value that is not NaN, and NaN where it is."""
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan), (what, np.flatnonzero(np.isnan(got) != nan)[:8])
+    assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32)), what
+
+
+@pytest.mark.parametrize("kind", ("Q8_0", "Q4_0"))
+def test_encode_of_nan_and_infinity_q8_0_q4_0(fh, g, orc, kind):
+    kind = getattr(fh.QKind, kind)
+    x = nonfinite().reshape(-1)
+    want = orc.encode(int(kind), x)
+    got = g.read_bytes(fh.encode(g, kind, g.upload(x), x.size))[: want.size]
+    assert np.array_equal(got, want), np.flatnonzero(got != want)[:8] // (want.size // 160)
+
+
+def test_snap_of_nan_and_infinity(fh, g, orc):
+    x = nonfinite()
+    rows = x.reshape(-1)
+    cols = np.ascontiguousarray(x.T)  # a block down each of the 160 columns
+    src, csrc = g.upload(rows), g.upload(cols.reshape(-1))
+    want = orc.snap_rows(rows, 32)
+    dst, cdst = g.zeros(rows.size), g.zeros(rows.size)
+    fh.q8_snap_rows(g, src, dst, 32)
+    same(g.read(dst), want, "rows")
+    cwant = np.ascontiguousarray(want.reshape(160, 32).T).reshape(-1)
+    fh.q8_snap_cols(g, csrc, cdst, (32, 160))
+    same(g.read(cdst), cwant, "cols")
+    pdst, pcdst = g.zeros(rows.size), g.zeros(rows.size)
+    plan = fh.SnapPlan(g, [(fh.SNAP_ROWS, src, pdst, 32), (fh.SNAP_COLS, csrc, pcdst, (32, 160))])
+    plan.run()
+    same(g.read(pdst), want, "plan, rows")
+    same(g.read(pcdst), cwant, "plan, cols")
