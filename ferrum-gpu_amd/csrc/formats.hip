@@ -262,7 +262,7 @@ __device__ __forceinline__ uint32_t fp8_encode4(const f32x4 v) {
     return r;
 }
 
-// mxfp4.rs:60-83: the code nearest x of the sixteen, the first of equally near ones. With the block's scale
+// mxfp4.rs:60-83: the code nearest x of the sixteen, the first of equally near ones. Where every code's value is finite,
 // every difference that decides is exact in f32, so this is a comparison with the midpoints (the
 // smaller magnitude at a tie; zero has one code).
 __device__ __forceinline__ uint32_t mx_nearest(float x, float d) {
@@ -272,7 +272,8 @@ __device__ __forceinline__ uint32_t mx_nearest(float x, float d) {
     return q && x < 0.0f ? q | 8u : q;
 }
 // The search itself, for blocks that hold an infinity (their scale byte is 0, and the differences of finite
-// values against it round).
+// values against it round), and for those whose codes 6 and 7 (8 d and 12 d) are infinite and so never the nearest: scale
+// byte 253, from a maximum that the f32 logarithm rounds up to 2^128 (the 44 floats at the top).
 __device__ uint32_t mx_search(float x, float d) {
     uint32_t best = 0;
     float best_err = fabsf(mx_value(0) * d - x);
@@ -322,11 +323,12 @@ __global__ __launch_bounds__(256) void encode_blocks_kernel(const float *__restr
             uint32_t e = 0;
             if (amax > 0.0f && finite) e = (uint32_t)min(max(mx_floor_log2(amax) - 2 + 127, 0), 254);
             const float d = mx_half_scale(e);
+            const bool near = finite && e < 253;
             uint32_t w[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 w[i] = 0;
-                for (int c = 0; c < 4; c++) w[i] |= (finite ? mx_nearest(v[i][c], d) : mx_search(v[i][c], d)) << (8 * c);
+                for (int c = 0; c < 4; c++) w[i] |= (near ? mx_nearest(v[i][c], d) : mx_search(v[i][c], d)) << (8 * c);
             }
             // lane 0 holds the low nibbles of the sixteen bytes, lane 1 the high ones; each writes eight bytes
 #pragma unroll

@@ -118,3 +118,20 @@ def test_snap_of_nan_and_infinity(fh, g, orc):
     plan.run()
     same(g.read(pdst), want, "plan, rows")
     same(g.read(pcdst), cwant, "plan, cols")
+
+
+def test_mxfp4_encode_of_the_largest_floats(fh, g, orc):
+    """A block maximum within a few units of the largest float rounds to the next power of two in f32's log2: the codes
+    for 8 and 12 then decode to infinity, and the nearest code is the one for 6. Maxima at the largest float, at and
+    around the unit where the logarithm rounds up, at the start of the top binade and below it; the other values from
+    tiny to the maximum, those past 7/8 of it and the code midpoints among them."""
+    tops = np.uint32([0x7f7fffff, 0x7f7ffffe, 0x7f7fffd4, 0x7f7fffd3, 0x7f7fffd2, 0x7f7fff01, 0x7f7fff00, 0x7f7ffeff,
+                      0x7f600000, 0x7f000000, 0x7effffff, 0x7effffd4]).view(np.float32)
+    rng = np.random.default_rng(8)
+    share = np.concatenate([rng.uniform(-1, 1, 19), [1, -1, 0.95, -0.95, 0.875, 0.8750001, 0.75, 0.625, 0.5, 0.4375, 1e-3,
+                                                     1e-30, -0.0]]).astype(np.float32)
+    x = np.concatenate([np.roll(share, s)[None] * t for t in tops for s in (0, 7)]).reshape(-1).astype(np.float32)
+    assert np.isfinite(x).all()
+    want = orc.encode(int(fh.QKind.Fp4), x)
+    got = g.read_bytes(fh.encode(g, fh.QKind.Fp4, g.upload(x), x.size))[: want.size]
+    assert np.array_equal(got, want), np.flatnonzero(got != want)[:8] // 17
