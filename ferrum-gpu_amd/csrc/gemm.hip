@@ -1668,7 +1668,7 @@ struct PrecisePlan {
     enum { STREAM, RING, TILES } kernel;
     uint32_t splits;
 };
-PrecisePlan precise_plan(size_t rows, size_t k, size_t n) {
+PrecisePlan precise_plan(size_t rows, size_t k, size_t n, bool close = true) {
     rows = (rows + 31) / 32 * 32;  // one plan for the rows of a 32-row tile (llama.hip sizes its workspace by them)
     const bool ring = ring_supported(rows, k, n);
     uint32_t sp = 1;
@@ -1676,9 +1676,9 @@ PrecisePlan precise_plan(size_t rows, size_t k, size_t n) {
         const uint64_t tiles = (uint64_t)((rows + 255) / 256) * ((n + 255) / 256), rounds = (tiles * sp + 255) / 256;
         const float us = 1.75f * (float)rounds * (float)((k / 32 + sp - 1) / sp) + 6.0f +
                          (sp > 1 ? (float)(sp + 1) * (float)rows * (float)n * 1e-6f : 0.0f);
-        if (!ring || ring_us(FH_Q8_0, rows, k, n) > 0.98f * us) return {PrecisePlan::STREAM, sp};
+        if (!ring || ring_us(FH_Q8_0, rows, k, n, close) > 0.98f * us) return {PrecisePlan::STREAM, sp};
     }
-    if (ring) return {PrecisePlan::RING, ring_splits(FH_Q8_0, rows, k, n)};
+    if (ring) return {PrecisePlan::RING, ring_splits(FH_Q8_0, rows, k, n, close)};
     return {PrecisePlan::TILES, precise_splits(rows, k, n)};
 }
 
@@ -2737,13 +2737,40 @@ hipError_t launch_make_b8(hipStream_t s, fh_kind kind, const uint8_t *qs, const 
     return hipGetLastError();
 }
 
+// The partial sums of an output that K splits make here: of the streaming kernel, or of tiles of 32 x 256 (up to 32
+// rows), 64 x 128 (up to 64; other formats than Q8_0 and Q4_0 up to 1024) and 128 x 128. The ring kernel's plan
+// keeps its error no larger than with these.
+uint32_t gemm_sum_parts(int kind, size_t rows, size_t k, size_t n) {
+    const bool planes = kind == FH_Q8_0 || kind == FH_Q4_0;
+    uint32_t sp = 1;
+    if (planes && stream_plan(rows, k, n, &sp) && stream_supported(rows, k, n)) return sp;
+    const size_t bm = rows <= 32 ? 32 : rows <= (planes ? 64 : kMidRows) ? 64 : 128, bn = bm == 32 ? 256 : 128;
+    return gemm_splits((uint64_t)((rows + bm - 1) / bm) * ((n + bn - 1) / bn), (uint32_t)(k / 32));
+}
+
 // (Sized for a consumer that takes the ring kernel's two parts, which otherwise add into y.)
 size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n) {
     const uint32_t sp = precise_plan(rows, k, n).splits;
     return sp > 1 ? (size_t)sp * rows * n * 4 : 0;
 }
 
-bool gemm_precise_ring(size_t rows, size_t k, size_t n) { return precise_plan(rows, k, n).kernel == PrecisePlan::RING; }
+bool gemm_fast_ring(size_t rows, size_t k, size_t n) {
+    return precise_plan(rows, k, n, false).kernel == PrecisePlan::RING && ring_one_round(rows, k, n, false);
+}
+
+hipError_t launch_gemm_fast_ring(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                                 size_t rows, size_t k, size_t n, void *workspace) {
+    _Float16 *xs = (_Float16 *)workspace;
+    const size_t items = rows * (k / 32);
+    const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
+    const uint32_t sp = ring_splits(kind, rows, k, n, false);
+    const size_t zeros = sp > 1 ? rows * n : 0;
+    if (kind == FH_Q8_0)
+        split_x_precise_kernel<FH_Q8_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    else
+        split_x_precise_kernel<FH_Q4_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    return launch_gemm_ring(s, kind, xs, qs, ds, y, (uint32_t)rows, (uint32_t)k, (uint32_t)n, sp, sp > 1, false);
+}
 
 // x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned; parts false: for a
 // call without `defer`, whose ring splits add into y)
@@ -2754,7 +2781,7 @@ size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts)
 
 hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x,
                                float *y, size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer,
-                               float *partial, bool saturate) {
+                               float *partial) {
     _Float16 *xs = (_Float16 *)workspace;
     if (!gemm_precise_partial_bytes(rows, k, n))
         partial = nullptr;
@@ -2765,17 +2792,11 @@ hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, c
     const PrecisePlan plan = precise_plan(rows, k, n);  // two ring splits add into y, zeroed by the x split
     const size_t zeros = plan.kernel == PrecisePlan::RING && plan.splits > 1 && !defer ? rows * n : 0;
     if (kind == FH_Q8_0) {
-        if (x && saturate)
-            split_x_precise_kernel<FH_Q8_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
-        else if (x)
-            split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+        if (x) split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
         return gemm_precise_dispatch<FH_Q8_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                               defer);
     }
-    if (x && saturate)
-        split_x_precise_kernel<FH_Q4_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
-    else if (x)
-        split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    if (x) split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
     return gemm_precise_dispatch<FH_Q4_0>(s, xs, qs, ds, y, partial, (uint32_t)rows, (uint32_t)k, (uint32_t)n,
                                           defer);
 }
@@ -2786,22 +2807,24 @@ bool gemm_ext_kind(int kind) {
 
 // Whether the ring kernel (gemm_ring.hip) takes the product: the formats other than Q2_K within its 32-bit offsets,
 // except where gemm_ext_kernel's tiles fill rounds of the chip better. Its time: two workgroups a CU, with 128-row
-// tiles 1.1 us a stage with one of them, 1.45 with both, with 64-row tiles 0.9, and 5 us of its own. Measured,
+// tiles 1.1 us a stage with one of them, 1.45 with both, with 64-row tiles 1.06 up to 600 of them, 0.9 a round past that, 5 us of its own, and for K splits 2 us and
+// 0.6 us per 10^6 partial products and outputs. Measured,
 // us, gemm_ext_kernel / ring: FP8 2048 x 11264 1024 rows 181 / 143, 2048 x 5632 2000 rows 173 / 146, 4096 rows 273 /
 // 283; 1024 x 2048 1024 rows 33 / 24, 4096 rows 58 / 67; F16 2048 x 5632 1024 rows 81 / 96, 700 rows 71 / 51.
 bool ext_ring(int kind, size_t rows, size_t k, size_t n) {
     if (!ring_gguf_supported(kind, rows, k, n)) return false;
-    if (rows <= 32 || ext_splits(kind, rows, k, n) > 1) return true;
+    if (rows <= 32) return true;
     size_t bm, bn;
     ext_tile(kind, rows, &bm, &bn);
-    const size_t tiles = (rows + bm - 1) / bm * ((n + bn - 1) / bn);
-    float stage = 0.9f * fmaxf((float)tiles / 512, 1.0f);  // a K step of all rounds
+    const size_t sp = ext_splits(kind, rows, k, n), tiles = (rows + bm - 1) / bm * ((n + bn - 1) / bn) * sp;
+    float stage = fmaxf(0.9f * (float)tiles / 512, 1.06f);  // a K step of all rounds
     if (bm == 128) {
         const float last = (float)(tiles % 512) / 256;
         stage = 1.45f * (float)(tiles / 512) + (last > 0 ? 1.1f + 0.35f * fminf(fmaxf(last - 1, 0.0f), 1.0f) : 0.0f);
         if (kind == FH_MXFP4) stage *= 0.95f;
     }
-    return ring_us(kind, rows, k, n) <= stage * (float)(k / 32) + 5;
+    const float own = 5 + (sp > 1 ? 2 + 0.6e-6f * (float)(sp + 1) * (float)rows * (float)n : 0);
+    return ring_us(kind, rows, k, n) <= stage * (float)((k / 32 + sp - 1) / sp) + own;
 }
 
 size_t gemm_ext_workspace_bytes(int kind, size_t rows, size_t k, size_t n) {

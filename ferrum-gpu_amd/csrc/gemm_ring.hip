@@ -7,14 +7,16 @@
 // workgroups on the chip a stage of 32 k is 0.25 us of MFMAs per wavefront pair, a load from L2 or HBM
 // takes 0.5 to 1 us, and one stage of lookahead through registers therefore ran at a quarter of the matrix
 // cores' rate (512 x 2048 x 2560, Q4_0: 1.8 us a stage). So every operand goes from memory straight into
-// LDS (buffer loads with an LDS destination, no registers) through a ring of NS stages, NS - 1 stages ahead.
+// LDS (buffer loads with an LDS destination, no registers) through a ring of NS stages (a stage's loads go out while
+// the stage NS before it is computed).
 //
 // A workgroup is eight wavefronts on one CU: a 32 MTW x 128 tile, the blocks of K dealt to four pairs of
 // wavefronts (each pair its own ring), whose sums meet in LDS in order at the end. So a few hundred tiles
 // fill the chip without partial products in memory (the K splits of 128 x 128 tiles before wrote and
 // read up to 64 MB for a 4 MB output). Where even then half the CUs would idle, K is split over two
 // workgroups, which add into y (zeroed by the x split; two addends onto +0 give the same bits in either
-// order) or leave two parts for the consumer.
+// order) or leave two parts for the consumer. Where its sums would be longer chains than the tiled kernels' K splits
+// make, a workgroup does K in phases or keeps totals (ring_plan).
 //
 // A wavefront owns 64 columns: their packed quants and scales are its own part of the ring and are unpacked
 // in its registers, and the x rows (128 bytes per row and block) are shared by the pair. One barrier a
@@ -25,12 +27,12 @@
 // per tile and block: 0.8 us a stage) and a row scale at the end.
 //
 // Measured (us, x split included, the 128 x 128 kernel and its reduction before / now, Q4_0): 512 rows 2048 x
-// 2560 35.8 / 28.7, 2048 x 2048 34.5 / 26.2, 2048 x 11264 99.8 / 68.8, 5632 x 2048 54.4 / 41.2, 896 x 1152
-// 28.0 / 13.8; 96 rows 2048 x 2560 27.2 / 14.0. GGUF rows (gemm_ext_kernel, one stage ahead through registers,
-// before / now): FP8 2048 x 11264 300 rows 77 / 50, 1024 rows 181 / 144, 64 rows 30 / 23; MXFP4 69 / 47, 152 /
-// 131, 31 / 21; F16 69 / 47, 167 / 133, 28 / 18.5; 5632 x 2048 300 rows 52 / 40, 48 / 37, 48 / 38. A stage takes 0.99 us, 1,085 TFLOP/s of matrix-core work on
-// 256 CUs (a plain bf16 product reaches 1,210 on the card); what is left is a workgroup's own 6 us and the
-// last round.
+// 2560 34.5 / 32.7 (in two phases, by ring_plan's rounding), 2048 x 2048 33.9 / 22.7, 2048 x 11264 98.8 / 67.2, 5632 x
+// 2048 52.5 / 40.0; 200 rows 896 x 1152 22.5 / 12.3; 128 rows 2048 x 2560 28.8 / 14.7. GGUF rows (gemm_ext_kernel, one
+// stage ahead through registers, before / now): FP8 2048 x 11264 300 rows 77 / 50, 1024 rows 181 / 144, 64 rows 30 /
+// 23; MXFP4 69 / 47, 152 / 131, 31 / 21; F16 69 / 47, 167 / 133, 28 / 18.5; 5632 x 2048 300 rows 50 / 39, 46 / 34,
+// 46 / 38. A stage takes 0.99 us, 1,085 TFLOP/s of matrix-core work on 256 CUs (a plain bf16 product reaches 1,210 on
+// the card); what is left is a workgroup's own 6 us and the last round.
 //
 // LDS: x row r of a slot keeps its 16-byte chunk c at c ^ ((r >> 1) & 7) (gemm.hip: the sixteen rows that
 // one cycle of a fragment read serves fall on sixteen different bank groups). Q8_0 quants are stored as
@@ -72,33 +74,26 @@ struct Ring {
     static_assert(XL >= 1 && NS >= 3 && (NS - 1) * LOADS < 64 && LDS <= 163840, "ring size");
 };
 
-// ADD: the workgroup's sums are added into y (two K splits onto zeros); else stored, split blockIdx.y at
-// y + blockIdx.y M N.
+constexpr uint32_t kFlush = 8;
+
+// Blocks st0 .. st1 - 1 of the tile at (m0, n0). ADD: its sums are added into y (two K splits onto zeros); else stored
+// or (again) added to what this workgroup's last phase stored.
 // XP: x parts, 2 (the precise product) or 1 (the f16 product: rows of x scaled to f16, output rows times rs).
-template <int KIND, int MTW, int KG, bool ADD, int XP = 2>
-__global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__restrict__ xs, const uint8_t *__restrict__ qs,
-                                                           const uint16_t *__restrict__ ds, float *__restrict__ y,
-                                                           uint32_t M, uint32_t K, uint32_t N, uint32_t mt, uint32_t nt,
-                                                           uint32_t split_stages, const float *__restrict__ rs) {
+template <int KIND, int MTW, int KG, bool ADD, bool PHASED, int XP>
+__device__ __forceinline__ void ring_phase(uint8_t *arena, const _Float16 *__restrict__ xs, const uint8_t *__restrict__ qs,
+                                           const uint16_t *__restrict__ ds, float *__restrict__ y, uint32_t M, uint32_t nb,
+                                           uint32_t N, uint32_t m0, uint32_t n0, uint32_t st0, uint32_t st1, bool again,
+                                           uint32_t wave, const float *__restrict__ rs) {
     using R = Ring<KIND, MTW, KG, XP>;
-    constexpr int BM = 32 * MTW, NS = R::NS;
-    __shared__ __attribute__((aligned(1024))) uint8_t arena[R::LDS];
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t *)arena;
-
-    // XCD x (workgroups x, x + 8, ...) owns the x-th equal run of the tiles, column by column: its
-    // workgroups share weight columns (read once from HBM) and x rows in its L2
-    const uint32_t tiles = mt * nt, per_xcd = (tiles + 7) / 8, t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= per_xcd || t >= tiles) return;  // whole workgroup: no barrier is left waiting
-    const uint32_t m0 = t % mt * BM, n0 = t / mt * R::BN;
-    const uint32_t nb = K / 32, nb8 = (nb + 7) / 8;
-    const uint32_t st0 = blockIdx.y * split_stages, st1 = min(nb, st0 + split_stages);
-    if (!ADD) y += (size_t)blockIdx.y * M * N;
-
-    const uint32_t tid = threadIdx.x, lane = tid % 64, fr = lane % 32, hf = lane / 32;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64), wn = wave % R::WPG, kg = wave / R::WPG;
+    constexpr int NS = R::NS;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t *)arena, nb8 = (nb + 7) / 8;
+    uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(lane));  // (a phase makes its own offsets: none is kept in registers through the stages)
+    const uint32_t fr = lane % 32, hf = lane / 32;
+    const uint32_t wn = wave % R::WPG, kg = wave / R::WPG;
 
     // Loads of block b into ring slot `slot`. Rows past M and columns past the padded weight rows fall past
-    // their resource's end by their offsets alone and read 0; a block past the split reads 0 through empty
+    // their resource's end by their offsets alone and read 0; a block past the phase reads 0 through empty
     // resources (the count of loads in flight stays the same).
     constexpr uint32_t XR = 1024 / R::XB, XC = R::XB / 16;  // rows of an x instruction, 16-byte chunks of a row
     const uint32_t xrow = XR * R::XL * wn + lane / XC;      // instruction i: rows XR i further
@@ -152,13 +147,15 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
                            xoff + XR * i * nb * R::XB + b * R::XB + ((lane % XC) ^ xswap(xrow + XR * i)) * 16);
     };
 
-    f32x16 acc[MTW][2];
+    // The sums; those of 32-row tiles go into a total every kFlush blocks, an even number, (64-row tiles leave no registers for it).
+    constexpr bool TOTALS = MTW == 1 && XP == 2;
+    f32x16 acc[MTW][2], total[TOTALS ? MTW : 1][2];
 #pragma unroll
     for (int i = 0; i < MTW; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; r++) acc[i][j][r] = total[TOTALS ? i : 0][j][r] = 0.0f;
 
     // One stage's operands in registers: x fragments (hi and lo, k16 steps 0 and 1), the packed quants of the
     // lane's share of the two column tiles, their scale dwords (blocks b & ~1 and b | 1).
@@ -357,12 +354,26 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
         compute(cur, nxt, b, slot, after);
         slot = after;
     };
-    for (uint32_t b = st0 + kg; b < st1 + kg; b += 2 * KG) {  // (b - kg: uniform over the workgroup)
-        stage(fa, fb, b);
-        if (b - kg + KG >= st1) break;
-        stage(fb, fa, b + KG);
+    // (b0: the blocks of a total's next chain; without totals all of them)
+    for (uint32_t b0 = st0, b1; b0 < st1; b0 = b1) {
+        b1 = TOTALS ? min(st1, b0 + KG * kFlush) : st1;
+        for (uint32_t b = b0 + kg; b < b1 + kg; b += 2 * KG) {  // (b - kg: uniform over the workgroup)
+            stage(fa, fb, b);
+            if (b - kg + KG >= b1) break;
+            stage(fb, fa, b + KG);
+        }
+        if constexpr (TOTALS)
+#pragma unroll
+            for (int i = 0; i < MTW; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        total[i][j][r] += acc[i][j][r];
+                        acc[i][j][r] = 0.0f;
+                    }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the last loads, past the split, write zeros into LDS)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the last loads, past the phase, write zeros into LDS)
     __syncthreads();
     // the groups' sums in order. D layout of a 32 x 32 tile: register r of lane l is row 8 (r / 4) +
     // 4 (l / 32) + r % 4, column l % 32
@@ -373,43 +384,107 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__res
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) sums[kg * PART + (((wn * MTW + i) * 2 + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+            for (int r = 0; r < 16; r++) sums[kg * PART + (((wn * MTW + i) * 2 + j) * 16 + r) * 64 + lane] = TOTALS ? total[TOTALS ? i : 0][j][r] : acc[i][j][r];
+    // output c of this thread: element (64 columns, i, j, register) c * 8 + wave of lane `lane`
+    constexpr int OUT = 4 * MTW * R::WPG;
+    auto place = [&](int c, uint32_t &row, uint32_t &col) {
+        const uint32_t e = c * 8 + wave, r = e % 16, j = e / 16 % 2, i = e / 32 % MTW, h = e / (32 * MTW);
+        row = m0 + i * 32 + 8 * (r / 4) + 4 * hf + r % 4;
+        col = n0 + 64 * h + j * 32 + fr;
+    };
+    float last[OUT];  // what this thread stored in the phase before (all loads in flight together)
+#pragma unroll
+    for (int c = 0; c < OUT; c++) last[c] = 0.0f;
+    if (PHASED && again) {
+#pragma unroll
+        for (int c = 0; c < OUT; c++) {
+            uint32_t row, col;
+            place(c, row, col);
+            last[c] = y[(size_t)min(row, M - 1) * N + min(col, N - 1)];
+        }
+    }
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 4 * MTW * R::WPG; c++) {
-        const uint32_t e = c * 8 + wave;  // (64 columns, i, j, register)
-        const uint32_t r = e % 16, j = e / 16 % 2, i = e / 32 % MTW, h = e / (32 * MTW);
+    for (int c = 0; c < OUT; c++) {
+        const uint32_t e = c * 8 + wave;
         float v = sums[e * 64 + lane];
 #pragma unroll
         for (int p = 1; p < KG; p++) v += sums[p * PART + e * 64 + lane];
-        const uint32_t row = m0 + i * 32 + 8 * (r / 4) + 4 * hf + r % 4, col = n0 + 64 * h + j * 32 + fr;
+        uint32_t row, col;
+        place(c, row, col);
         if (row < M && col < N) {
             if constexpr (XP == 1) v *= rs[row];
             if (ADD)
                 unsafeAtomicAdd(y + (size_t)row * N + col, v);
             else
-                y[(size_t)row * N + col] = v;
+                y[(size_t)row * N + col] = PHASED && again ? last[c] + v : v;
         }
+    }
+}
+
+// A tile, split blockIdx.y of K (its sums at y + blockIdx.y M N, or ADD), in phases of `phase` blocks.
+template <int KIND, int MTW, int KG, bool ADD, bool PHASED, int XP = 2>
+__global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const _Float16 *__restrict__ xs, const uint8_t *__restrict__ qs,
+                                                           const uint16_t *__restrict__ ds, float *__restrict__ y,
+                                                           uint32_t M, uint32_t K, uint32_t N, uint32_t mt, uint32_t nt,
+                                                           uint32_t split_stages, uint32_t phase,
+                                                           const float *__restrict__ rs) {
+    using R = Ring<KIND, MTW, KG, XP>;
+    __shared__ __attribute__((aligned(1024))) uint8_t arena[R::LDS];
+    // XCD x (workgroups x, x + 8, ...) owns the x-th equal run of the tiles, column by column: its
+    // workgroups share weight columns (read once from HBM) and x rows in its L2
+    const uint32_t tiles = mt * nt, per_xcd = (tiles + 7) / 8, t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per_xcd || t >= tiles) return;  // whole workgroup: no barrier is left waiting
+    const uint32_t m0 = t % mt * 32 * MTW, n0 = t / mt * R::BN, nb = K / 32;
+    const uint32_t st0 = blockIdx.y * split_stages, st1 = min(nb, st0 + split_stages);
+    if (!ADD) y += (size_t)blockIdx.y * M * N;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    for (uint32_t p0 = st0;;) {
+        const uint32_t p1 = PHASED ? min(st1, p0 + phase) : st1;
+        ring_phase<KIND, MTW, KG, ADD, PHASED, XP>(arena, xs, qs, ds, y, M, nb, N, m0, n0, p0, p1, p0 != st0, wave, rs);
+        if (!PHASED || (p0 = p1) >= st1) return;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores are out of the next phase's load counts,
+        __syncthreads();                                  // and its loads may overwrite the sums
     }
 }
 
 }  // namespace
 
-// The row tile, group count and K splits of a product, and its time in us: rounds of a workgroup per CU, each
+// The row tile, group count, K splits and phases of a product, and its time in us: rounds of a workgroup per CU, each
 // its stages (64 rows: 0.99 us, measured 0.9 to 1.1; 32 rows: 0.5 us with few workgroups and 0.85 with one on
-// every CU, for twice the weight loads and unpacking per row) and a workgroup's own cost (first loads and epilogue, 7 and 4 us). Two splits only where one leaves half
-// of the CUs idle, at the cost of zeroing y and of two additions per output. GGUF rows cost a stage more by the factor f. (512 rows: 2048 x 2560 26 us with 128-column tiles, 42 with 256-column ones; 896 x 9728
-// at 300 rows 29 and 26. 32-row tiles where 64-row ones are few: Q8_0 5632 x 2048
+// every CU, for twice the weight loads and unpacking per row) and a workgroup's own cost (first loads and epilogue,
+// 7 and 4 us). Two splits only where one leaves half of the CUs idle, at the cost of zeroing y and of two additions
+// per output. GGUF rows cost a stage more by the factor f. (512 rows: 2048 x 2560 26 us with 128-column tiles, 42 with
+// 256-column ones; 896 x 9728 at 300 rows 29 and 26. 32-row tiles where 64-row ones are few: Q8_0 5632 x 2048
 // 128 rows 29 with 64-row tiles, 23 with 32-row ones; 2048 x 11264 128 rows 25 and 29.)
+//
+// Rounding. The variance of an output's relative error is 0.064 v + 0.58 in units of (1e-7)^2 (F16 0.80; fitted to 20
+// products of 896 to 11008 inputs), v being the roundings of f32 sums in units of the last one: chains of l of nb
+// equal addends give l / 2, n partial sums one after the other (n + 1) / 2 - 1 / n. The plan keeps v no larger than
+// the K splits of the tiled kernels (gemm_sum_parts) make it: by more groups or splits, by 32-row tiles, whose chains
+// are kFlush blocks, or with K in 2 to 4 phases of a workgroup, each added to the one before in y (6.5 us a turn: the
+// sums' way through LDS, their stores and the first loads of a phase). Relative error (1e-7) and us of Q8_0, fastest
+// plan / this one / 128 x 128 tiles: 3600 rows 3808 x 736 1.59 / 1.13 / 1.16 and 77 / 102 / 116; 300 rows 2048 x 11264
+// 1.28 / 1.04 / 1.08 and 42 / 53 / 79; 975 rows 1344 x 3052 1.14 / 1.02 / 1.02 and 32 / 40 / 56; 512 rows 2048 x 2560
+// 1.11 / 1.02 / 1.07 and 25 / 30 / 34; 975 rows 6912 x 1344 1.56 / 1.29 / 1.46 and 65 / 71 / 81.
 struct RingPlan {
-    uint32_t mtw, kg, splits;
+    uint32_t mtw, kg, splits, phases;
     float us;
 };
-static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n, int xp = 2) {
+static float added_in_turn(uint32_t n) { return (float)(n + 1) / 2 - 1 / (float)n; }
+static float sum_roundings(size_t nb, uint32_t mtw, uint32_t kg, uint32_t outer) {
+    kg = (uint32_t)std::min<size_t>(kg, nb);
+    const float chain = (float)nb / (float)(kg * outer), flush = (float)kFlush;
+    const float one = mtw == 1 && chain > flush ? (flush + chain / flush) / 2 : chain / 2;
+    return one + added_in_turn(kg) + added_in_turn(outer);
+}
+static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n, bool close = true, int xp = 2) {
     const size_t nb = k / 32;
     rows = (rows + 31) / 32 * 32;  // (one plan for the rows of a 32-row tile)
-    const float f = kind == FH_F16 ? 1.3f : kind == FH_MXFP4 ? 1.15f : kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 ? 1.25f : xp == 1 ? 0.8f : 1.0f;
-    RingPlan best{1, 4, 1, INFINITY};
+    const float f = kind == FH_MXFP4 ? 1.15f : kind == FH_FP8_E4M3 || kind == FH_FP8_E5M2 ? 1.25f : xp == 1 ? 0.8f : 1.0f;
+    const uint32_t parts = close ? gemm_sum_parts(kind, rows, k, n) : 1;
+    const float most = close ? 1.02f * ((float)nb / (float)(2 * parts) + added_in_turn(parts)) + 0.17f : INFINITY;  // (+ 1%)
+    RingPlan best{1, 4, 1, 1, INFINITY};
     for (uint32_t mtw : {2u, 1u})
         for (uint32_t kg : {4u, 2u})
             for (uint32_t sp : {1u, 2u}) {
@@ -417,19 +492,24 @@ static RingPlan ring_plan(int kind, size_t rows, size_t k, size_t n, int xp = 2)
                 if (mtw == 2 && (rows <= 32 || (kind == FH_F16 && kg == 4))) continue;  // (that stage does not fit LDS three times)
                 const uint64_t tiles = (rows + 32 * mtw - 1) / (32 * mtw) * ((n + 512 / kg - 1) / (512 / kg));
                 if (sp == 2 && (tiles > 128 || nb < 4 * kg)) continue;
-                const float stages = (float)((nb + sp * kg - 1) / (sp * kg));
-                const float c32 = f * (0.45f + 0.4f * std::min((float)(tiles * sp) / 256, 1.0f)), c64 = f * 0.99f;
-                const float us = (float)((tiles * sp + 255) / 256) * (mtw == 2 ? c64 * stages + 7 : c32 * stages + 4) +
+                uint32_t ph = 1;
+                while (ph < 4 && sp == 1 && mtw == 2 && sum_roundings(nb, mtw, kg, ph) > most) ph++;
+                if (sum_roundings(nb, mtw, kg, sp * ph) > most) continue;
+                const float fk = kind == FH_F16 ? (mtw == 2 ? 1.15f : 0.97f) : f;
+                const float stages = (float)((nb + sp * kg - 1) / (sp * kg)), turn = 6.5f * (float)(ph - 1);
+                const float c32 = fk * (0.45f + 0.4f * std::min((float)(tiles * sp) / 256, 1.0f)), c64 = fk * 0.99f;
+                const float us = (float)((tiles * sp + 255) / 256) * ((mtw == 2 ? c64 * stages + 7 : c32 * stages + 4) + turn) +
                                  (sp == 2 ? 1.5f + 3e-6f * (float)rows * (float)n : 0);
-                if (us < best.us) best = RingPlan{mtw, kg, sp, us};
+                if (us < best.us) best = RingPlan{mtw, kg, sp, ph, us};
             }
-    return best;
+    // (two or three blocks: every plan has a rounding more than one chain, 1 to 2.6% of the error)
+    return best.us < INFINITY ? best : ring_plan(kind, rows, k, n, false, xp);
 }
-uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n) { return ring_plan(kind, rows, k, n).splits; }
-float ring_us(int kind, size_t rows, size_t k, size_t n) { return ring_plan(kind, rows, k, n).us; }
+uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n, bool close) { return ring_plan(kind, rows, k, n, close).splits; }
+float ring_us(int kind, size_t rows, size_t k, size_t n, bool close) { return ring_plan(kind, rows, k, n, close).us; }
 
-bool ring_one_round(size_t rows, size_t k, size_t n) {
-    const RingPlan p = ring_plan(FH_Q8_0, rows, k, n);
+bool ring_one_round(size_t rows, size_t k, size_t n, bool close) {
+    const RingPlan p = ring_plan(FH_Q8_0, rows, k, n, close);
     return (rows + 32 * p.mtw - 1) / (32 * p.mtw) * ((n + 512 / p.kg - 1) / (512 / p.kg)) * p.splits <= 256;
 }
 
@@ -444,41 +524,44 @@ bool ring_gguf_supported(int kind, size_t rows, size_t k, size_t n) {
 
 template <int KIND, int MTW, int KG, int XP = 2>
 static hipError_t run_ring(hipStream_t s, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out, uint32_t M,
-                           uint32_t K, uint32_t N, uint32_t sp, bool add, const float *rs = nullptr) {
+                           uint32_t K, uint32_t N, uint32_t sp, bool add, uint32_t phases, const float *rs = nullptr) {
     constexpr uint32_t BN = Ring<KIND, MTW, KG, XP>::BN;
     const uint32_t mt = (M + 32 * MTW - 1) / (32 * MTW), nt = (N + BN - 1) / BN, nb = K / 32;
     const dim3 grid((mt * nt + 7) / 8 * 8, sp);
-    const uint32_t per = ((nb + sp - 1) / sp + KG - 1) / KG * KG;
+    const uint32_t per = ((nb + sp - 1) / sp + KG - 1) / KG * KG, phase = ((per + phases - 1) / phases + KG - 1) / KG * KG;
     if (add)
-        gemm_ring_kernel<KIND, MTW, KG, true, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, rs);
+        gemm_ring_kernel<KIND, MTW, KG, true, false, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, phase, rs);
+    else if (MTW == 2 && XP == 2 && phases > 1)
+        gemm_ring_kernel<KIND, MTW, KG, false, MTW == 2 && XP == 2, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per,
+                                                                                           phase, rs);
     else
-        gemm_ring_kernel<KIND, MTW, KG, false, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, rs);
+        gemm_ring_kernel<KIND, MTW, KG, false, false, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, phase, rs);
     return hipGetLastError();
 }
 
 template <int KIND>
 static hipError_t run_ring_kind(hipStream_t s, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
-                                uint32_t M, uint32_t K, uint32_t N, uint32_t sp, bool add) {
-    const RingPlan p = ring_plan(KIND, M, K, N);
+                                uint32_t M, uint32_t K, uint32_t N, uint32_t sp, bool add, bool close) {
+    const RingPlan p = ring_plan(KIND, M, K, N, close);
     if (p.mtw == 1)
-        return p.kg == 4 ? run_ring<KIND, 1, 4>(s, xs, qs, ds, out, M, K, N, sp, add)
-                         : run_ring<KIND, 1, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
+        return p.kg == 4 ? run_ring<KIND, 1, 4>(s, xs, qs, ds, out, M, K, N, sp, add, p.phases)
+                         : run_ring<KIND, 1, 2>(s, xs, qs, ds, out, M, K, N, sp, add, p.phases);
     if constexpr (KIND != FH_F16)
-        if (p.kg == 4) return run_ring<KIND, 2, 4>(s, xs, qs, ds, out, M, K, N, sp, add);
-    return run_ring<KIND, 2, 2>(s, xs, qs, ds, out, M, K, N, sp, add);
+        if (p.kg == 4) return run_ring<KIND, 2, 4>(s, xs, qs, ds, out, M, K, N, sp, add, p.phases);
+    return run_ring<KIND, 2, 2>(s, xs, qs, ds, out, M, K, N, sp, add, p.phases);
 }
 
 template <int KIND>
 static hipError_t run_ring_f16(hipStream_t s, const _Float16 *xs, const float *rs, const uint8_t *qs, const uint16_t *ds,
                                float *out, uint32_t M, uint32_t K, uint32_t N) {
-    const RingPlan p = ring_plan(KIND, M, K, N, 1);
+    const RingPlan p = ring_plan(KIND, M, K, N, false, 1);
     const bool add = p.splits > 1;
-    if (p.mtw == 1) return run_ring<KIND, 1, 4, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, rs);
-    if (p.kg == 4) return run_ring<KIND, 2, 4, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, rs);
-    return run_ring<KIND, 2, 2, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, rs);
+    if (p.mtw == 1) return run_ring<KIND, 1, 4, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, 1, rs);
+    if (p.kg == 4) return run_ring<KIND, 2, 4, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, 1, rs);
+    return run_ring<KIND, 2, 2, 1>(s, xs, qs, ds, out, M, K, N, p.splits, add, 1, rs);
 }
-float ring_f16_us(size_t rows, size_t k, size_t n) { return ring_plan(FH_Q8_0, rows, k, n, 1).us; }
-uint32_t ring_f16_splits(size_t rows, size_t k, size_t n) { return ring_plan(FH_Q8_0, rows, k, n, 1).splits; }
+float ring_f16_us(size_t rows, size_t k, size_t n) { return ring_plan(FH_Q8_0, rows, k, n, false, 1).us; }
+uint32_t ring_f16_splits(size_t rows, size_t k, size_t n) { return ring_plan(FH_Q8_0, rows, k, n, false, 1).splits; }
 hipError_t launch_gemm_ring_f16(hipStream_t s, int kind, const _Float16 *xs, const float *rs, const uint8_t *qs,
                                 const uint16_t *ds, float *out, uint32_t M, uint32_t K, uint32_t N) {
     return kind == FH_Q8_0 ? run_ring_f16<FH_Q8_0>(s, xs, rs, qs, ds, out, M, K, N)
@@ -486,14 +569,14 @@ hipError_t launch_gemm_ring_f16(hipStream_t s, int kind, const _Float16 *xs, con
 }
 
 hipError_t launch_gemm_ring(hipStream_t s, int kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
-                            uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add) {
+                            uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add, bool close) {
     switch (kind) {
-    case FH_Q8_0: return run_ring_kind<FH_Q8_0>(s, xs, qs, ds, out, M, K, N, splits, add);
-    case FH_Q4_0: return run_ring_kind<FH_Q4_0>(s, xs, qs, ds, out, M, K, N, splits, add);
-    case FH_F16: return run_ring_kind<FH_F16>(s, xs, qs, nullptr, out, M, K, N, splits, add);
-    case FH_FP8_E4M3: return run_ring_kind<FH_FP8_E4M3>(s, xs, qs, nullptr, out, M, K, N, splits, add);
-    case FH_FP8_E5M2: return run_ring_kind<FH_FP8_E5M2>(s, xs, qs, nullptr, out, M, K, N, splits, add);
-    case FH_MXFP4: return run_ring_kind<FH_MXFP4>(s, xs, qs, nullptr, out, M, K, N, splits, add);
+    case FH_Q8_0: return run_ring_kind<FH_Q8_0>(s, xs, qs, ds, out, M, K, N, splits, add, close);
+    case FH_Q4_0: return run_ring_kind<FH_Q4_0>(s, xs, qs, ds, out, M, K, N, splits, add, close);
+    case FH_F16: return run_ring_kind<FH_F16>(s, xs, qs, nullptr, out, M, K, N, splits, add, close);
+    case FH_FP8_E4M3: return run_ring_kind<FH_FP8_E4M3>(s, xs, qs, nullptr, out, M, K, N, splits, add, close);
+    case FH_FP8_E5M2: return run_ring_kind<FH_FP8_E5M2>(s, xs, qs, nullptr, out, M, K, N, splits, add, close);
+    case FH_MXFP4: return run_ring_kind<FH_MXFP4>(s, xs, qs, nullptr, out, M, K, N, splits, add, close);
     default: return hipErrorInvalidValue;
     }
 }

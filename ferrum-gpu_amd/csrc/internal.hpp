@@ -301,7 +301,6 @@ hipError_t launch_gemm_f16(hipStream_t s, fh_kind kind, const uint8_t *qs, const
                            size_t rows, size_t k, size_t n, void *workspace, SplitOut *defer = nullptr);
 // The precise MFMA GEMM (x as two f16 parts; split into workspace, then the product).
 size_t gemm_precise_workspace_bytes(size_t rows, size_t k, size_t n, bool parts = true);
-bool gemm_precise_ring(size_t rows, size_t k, size_t n);  // whether the ring kernel takes the precise product
 // The MFMA GEMM on the GGUF rows of F16, FP8 E4M3 / E5M2, MXFP4 and Q2_K weights (rows >= 2) and
 // its workspace (x split, then the K-split partial products).
 bool gemm_ext_kind(int kind);
@@ -312,14 +311,21 @@ hipError_t launch_gemm_ext(hipStream_t s, int kind, const uint8_t *w, const floa
 // partial != nullptr: the K-split partial products go there (as launch_gemm's).
 hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x,
                                float *y, size_t rows, size_t k, size_t n, void *workspace,
-                               SplitOut *defer = nullptr, float *partial = nullptr, bool saturate = false);
+                               SplitOut *defer = nullptr, float *partial = nullptr);
 size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n);
+// Whether a single fast product takes the precise product's ring kernel (by its fastest plan), and that product: x
+// split into workspace (rows k floats), finite for any finite x.
+bool gemm_fast_ring(size_t rows, size_t k, size_t n);
+hipError_t launch_gemm_fast_ring(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                                 size_t rows, size_t k, size_t n, void *workspace);
 // gemm_ring.hip: the precise product alone on split x (of split_x_precise_kernel's order for the kind): `splits`
 // (1 or 2) partial products of M x N at out, or (add) their sum added to zeros at out. Kinds other than
 // Q8_0 and Q4_0 (ring_gguf_supported): qs is the GGUF rows.
-uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n);
-float ring_us(int kind, size_t rows, size_t k, size_t n);  // its time by the plan's model
-bool ring_one_round(size_t rows, size_t k, size_t n);  // no more workgroups than CUs
+uint32_t gemm_sum_parts(int kind, size_t rows, size_t k, size_t n);  // (gemm.hip) of an output in its kernels
+// close: by a plan whose rounding is no larger than gemm_sum_parts' (else the fastest).
+uint32_t ring_splits(int kind, size_t rows, size_t k, size_t n, bool close = true);
+float ring_us(int kind, size_t rows, size_t k, size_t n, bool close = true);  // its time by the plan's model
+bool ring_one_round(size_t rows, size_t k, size_t n, bool close = true);      // no more workgroups than CUs
 bool ring_supported(size_t rows, size_t k, size_t n);
 bool ring_gguf_supported(int kind, size_t rows, size_t k, size_t n);
 // The f16 product: x in one f16 part, its rows scaled; output rows times rs; added to zeros at out where K is split.
@@ -328,7 +334,7 @@ uint32_t ring_f16_splits(size_t rows, size_t k, size_t n);
 hipError_t launch_gemm_ring_f16(hipStream_t s, int kind, const _Float16 *xs, const float *rs, const uint8_t *qs,
                                 const uint16_t *ds, float *out, uint32_t M, uint32_t K, uint32_t N);
 hipError_t launch_gemm_ring(hipStream_t s, int kind, const _Float16 *xs, const uint8_t *qs, const uint16_t *ds, float *out,
-                            uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add);
+                            uint32_t M, uint32_t K, uint32_t N, uint32_t splits, bool add, bool close = true);
 
 // prefill.hip: the GPT-2 prompt pass (one row per prompt token). prefill_row_kernel makes a row by mode
 // and writes it as a product's split x (launch_gemm_precise's), scaled by a power of two whose inverse

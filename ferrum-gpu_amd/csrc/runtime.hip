@@ -845,9 +845,8 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         // 45, 1024 rows 5632 x 2048 79 and 79 / 64 and 63, 2048 rows 1024 x 2048 38.5 and 37.9 / 32.5 and 33.5; past one
         // round 1024 rows 2048 x 5632 81 and 68 / 75 and 76), while its scratch, the larger one, fits the static array
         // too (both entry points give the same bits).
-        const size_t pbytes = gemm_precise_workspace_bytes(rows, w->k, w->n, false);
-        const bool precise = rows && rows <= 2048 && gemm_precise_ring(rows, w->k, w->n) && ring_one_round(rows, w->k, w->n) &&
-                             pbytes <= FH_NOALLOC_SCRATCH_BYTES;
+        const size_t pbytes = rows * w->k * 4;
+        const bool precise = rows && rows <= 2048 && gemm_fast_ring(rows, w->k, w->n) && pbytes <= FH_NOALLOC_SCRATCH_BYTES;
         void *ws = nullptr;
         if (rows && (st = command_scratch(dev, fixed, precise ? pbytes : gemm_workspace_bytes(rows, w->k, w->n), &ws)))
             return st;
@@ -862,7 +861,7 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
             w->b8 = (uint8_t *)fresh;
         }
         if (precise)
-            (void)launch_gemm_precise(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws, nullptr, nullptr, true);
+            (void)launch_gemm_fast_ring(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws);
         else if (rows)
             (void)launch_gemm(dev->stream, w->kind, w->qs, w->ds, w->b8, x, y, rows, w->k, w->n, ws);
         return end_command(dev, "linear_q");
