@@ -31,11 +31,13 @@ struct fh_device {
     void *ws = nullptr;
     size_t ws_bytes = 0;
     // kTicketCount zeros: arrival counters of launches that split a product's K over workgroups; every
-    // such launch leaves them zero, and launches on the one stream use them in order.
+    // such launch leaves them zero, and launches on the one stream use them in order (the no-allocation
+    // entry point's launches, which a caller may replay on another stream, use scratch_tickets).
     uint32_t *tickets = nullptr;
     // This GPU's copy of the no-allocation entry point's static scratch array (its device
     // address, taken when the device is opened).
     void *scratch = nullptr;
+    uint32_t *scratch_tickets = nullptr;  // and of its arrival counters
 };
 
 struct fh_buffer {

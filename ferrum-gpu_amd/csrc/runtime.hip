@@ -16,6 +16,9 @@
 // uses this name as an address: fh_device_open takes this GPU's device address of it with
 // hipGetSymbolAddress, and every launch gets that pointer.
 static __device__ __align__(256) uint8_t scratch[FH_NOALLOC_SCRATCH_BYTES];
+// Its arrival counters (fh_device::tickets' counterpart): apart from every handle's, since a captured call may run on
+// another stream while the handle's own calls use those.
+static __device__ uint32_t scratch_tickets[fh::kTicketCount];
 
 namespace fh {
 
@@ -351,7 +354,8 @@ fh_status fh_device_open(int ordinal, fh_device **out) {
     d->name = prop.name[0] ? prop.name : prop.gcnArchName;
     // this GPU's copy of the no-allocation scratch (the device is current), and the event that
     // orders the calls using it
-    if ((e = hipGetSymbolAddress(&d->scratch, HIP_SYMBOL(scratch))) != hipSuccess) {
+    if ((e = hipGetSymbolAddress(&d->scratch, HIP_SYMBOL(scratch))) != hipSuccess ||
+        (e = hipGetSymbolAddress((void **)&d->scratch_tickets, HIP_SYMBOL(scratch_tickets))) != hipSuccess) {
         delete d;
         return hip_fail(nullptr, e, "scratch address");
     }
@@ -766,7 +770,8 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         const size_t bytes = rows_call_scratch_bytes(rows, w->k, w->n, dev->cus);
         if (bytes && (st = command_scratch(dev, fixed, bytes, &part))) return st;
         if ((st = begin_command(dev, "linear_q"))) return st;
-        (void)launch_rows_call(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, part, dev->tickets, dev->cus);
+        uint32_t *tickets = fixed ? dev->scratch_tickets : dev->tickets;
+        (void)launch_rows_call(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, part, tickets, dev->cus);
         return end_command(dev, "linear_q");
     }
     // Past 16 rows the precise GEMM's ring kernel beats the few-row kernel's two launches (us, Q8_0, few-row /

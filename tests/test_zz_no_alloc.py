@@ -134,3 +134,66 @@ def test_noalloc_refuses_overlapping_x_and_y(fh, g, orc):
     qw, gx, ya, yb, _ = case(fh, g, orc, fh.QKind.Q8_0, 8, 256, 256, 9, cpu=False)
     with pytest.raises(fh.GpuError, match="overlap"):
         fh.linear_q_noalloc(g, gx.device_ptr(), qw, gx.device_ptr() + 4 * 256, 8, fh.QPath.Rows)
+
+
+# K-split one-launch products (eight splits each), then one with a single split
+FEW = [(24, 4864, 896), (8, 5632, 1024), (5, 896, 300)]
+
+
+@pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0", "Fp8E4M3", "Fp8E5M2", "Fp4", "F16"])
+def test_noalloc_few_row_products_equal_linear_q(fh, g, orc, kind_name):
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(12)
+    for rows, k, n in FEW + [(48, 896, 1152), (200, 1056, 257)]:
+        raw = orc.encode(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32))
+        qw, gx = fh.upload_qweight(g, kind, raw, k, n), g.upload(rng.standard_normal(rows * k).astype(np.float32))
+        ya, yb = g.zeros(rows * n), g.zeros(rows * n)
+        fh.linear_q_ptr(g, gx.device_ptr(), qw, ya.device_ptr(), rows)
+        for _ in range(2):
+            fh.linear_q_noalloc(g, gx.device_ptr(), qw, yb.device_ptr(), rows)
+            assert np.array_equal(g.read(ya).view(np.uint32), g.read(yb).view(np.uint32)), (rows, k, n)
+
+
+def test_captured_noalloc_products_beside_ordinary_ones(fh, g, orc):
+    """A graph of no-allocation K-split products, replayed on a stream of its own while ordinary K-split products
+    run on the handle's: neither touches the other's scratch or arrival counters, so both keep their bits."""
+    hip = ctypes.CDLL("libamdhip64.so.7", mode=__import__("os").RTLD_NOLOAD | ctypes.RTLD_GLOBAL)
+    P = ctypes.c_void_p
+
+    def call(name, *a):
+        assert getattr(hip, name)(*a) == 0, name
+
+    work = []
+    for kind_name in ("Q8_0", "Fp8E4M3"):
+        for i, (rows, k, n) in enumerate(FEW):
+            kind, rng = fh.QKind[kind_name], np.random.default_rng(30 + i)
+            raw = orc.encode(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32))
+            x = rng.standard_normal(rows * k).astype(np.float32)
+            work.append((rows, fh.upload_qweight(g, kind, raw, k, n), g.upload(x), g.zeros(rows * n), g.zeros(rows * n)))
+    for rows, qw, gx, ya, _ in work:
+        fh.linear_q_ptr(g, gx.device_ptr(), qw, ya.device_ptr(), rows)
+    want = [g.read(ya).copy() for *_, ya, _ in work]
+    stream, graph, run = P(g.stream()), P(), P()
+    call("hipStreamBeginCapture", stream, 2)  # relaxed
+    for rows, qw, gx, _, yb in work:
+        fh.linear_q_noalloc(g, gx.device_ptr(), qw, yb.device_ptr(), rows)
+    call("hipStreamEndCapture", stream, ctypes.byref(graph))
+    call("hipGraphInstantiate", ctypes.byref(run), graph, None, None, ctypes.c_size_t(0))
+    other = P()
+    call("hipStreamCreateWithFlags", ctypes.byref(other), 1)
+    try:
+        for rep in range(20):
+            for _ in range(4):
+                call("hipGraphLaunch", run, other)
+            for _ in range(8):
+                for rows, qw, gx, ya, _ in work:
+                    fh.linear_q_ptr(g, gx.device_ptr(), qw, ya.device_ptr(), rows)
+            call("hipStreamSynchronize", other)
+            g.sync()
+            for (rows, qw, gx, ya, yb), w in zip(work, want):
+                assert np.array_equal(g.read(ya).view(np.uint32), w.view(np.uint32)), (rep, rows, "ordinary")
+                assert np.array_equal(g.read(yb).view(np.uint32), w.view(np.uint32)), (rep, rows, "captured")
+    finally:
+        call("hipGraphExecDestroy", run)
+        call("hipGraphDestroy", graph)
+        call("hipStreamDestroy", other)
