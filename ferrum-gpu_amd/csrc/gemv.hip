@@ -172,7 +172,9 @@ struct PrepJobs {
     uint32_t count, py;
 };
 
-template <int KIND, bool LDSX>
+// WIDE: products past kGemvLdsBlocks blocks, whose batches go to four sums in turn, added as gemv_wide_kernel's
+// wavefronts' are, so the two give the same bits.
+template <int KIND, bool LDSX, bool WIDE>
 __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ descs,
                                                    const uint32_t *__restrict__ map, GemvDesc one, uint32_t count,
                                                    uint32_t tasks, uint32_t tasks_per_wave, uint32_t lds_blocks,
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
                 }
             }
         };
-        float acc = 0.0f;
+        float acc[WIDE ? 4 : 1] = {};  // (WIDE: acc[0] is the next batch's sum)
         __shared__ float stage_rows[4][kStage][32];
         __shared__ StageMeta stage_meta[4][kStage];
         const uint32_t wv = threadIdx.x / 64;
@@ -261,12 +263,29 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
         // After computing batch cp: on a task's last batch, add the row's odd blocks (lane 32 + r) to
         // its even ones (lane r) and stage the row.
         auto finish = [&](const Pos &cp) {
+            if constexpr (WIDE) {
+                const float last = acc[0];
+                acc[0] = acc[1];
+                acc[1] = acc[2];
+                acc[2] = acc[3];
+                acc[3] = last;
+            }
             if (cp.b + kBatch >= cp.nb) {
-                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
-                const float sum = acc + __uint_as_float(upper ? sw[0] : sw[1]);
+                float sum = 0.0f, part[WIDE ? 4 : 1];
+#pragma unroll
+                for (int i = 0; i < (WIDE ? 4 : 1); i++) {
+                    const uint32_t a = __float_as_uint(acc[i]);
+                    const auto sw = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+                    part[i] = acc[i] + __uint_as_float(upper ? sw[0] : sw[1]);
+                    acc[i] = 0.0f;
+                }
+                if constexpr (WIDE)  // after an odd number of batches the first is in part[3] (or part[1])
+                    sum = (cp.b / kBatch) % 2 == 0 ? (part[3] + part[0]) + (part[1] + part[2])
+                                                   : (part[0] + part[1]) + (part[2] + part[3]);
+                else
+                    sum = part[0];
                 if (!upper) stage_rows[wv][staged][r] = sum;
                 if (lane == 0) stage_meta[wv][staged] = StageMeta{cp.y, cp.g * 32, cp.n};
-                acc = 0.0f;
                 if (++staged == kStage) flush();
             }
         };
@@ -279,9 +298,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
             load_batch<KIND, LDSX>(b1, ltk, lp.b, o, lds_base);
             __builtin_amdgcn_sched_barrier(0);
             if (cp.b + kBatch / 2 >= cp.nb)
-                compute_batch<KIND, kBatch / 4>(b0, upper, acc);  // a task's last half batch
+                compute_batch<KIND, kBatch / 4>(b0, upper, acc[0]);  // a task's last half batch
             else
-                compute_batch<KIND>(b0, upper, acc);
+                compute_batch<KIND>(b0, upper, acc[0]);
             __builtin_amdgcn_sched_barrier(0);
             finish(cp);
             if (lp.t >= t1) break;
@@ -290,9 +309,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
             load_batch<KIND, LDSX>(b0, ltk, lp.b, o, lds_base);
             __builtin_amdgcn_sched_barrier(0);
             if (cp.b + kBatch / 2 >= cp.nb)
-                compute_batch<KIND, kBatch / 4>(b1, upper, acc);
+                compute_batch<KIND, kBatch / 4>(b1, upper, acc[0]);
             else
-                compute_batch<KIND>(b1, upper, acc);
+                compute_batch<KIND>(b1, upper, acc[0]);
             __builtin_amdgcn_sched_barrier(0);
             finish(cp);
             if (lp.t >= t1) break;
@@ -311,14 +330,11 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvDesc *__restrict__ 
 }
 
 // Products too wide for the LDS records (nb > kGemvLdsBlocks): a task's batches are dealt to the four
-// wavefronts of a workgroup, whose row sums meet in LDS in a fixed order. A wavefront per task left such a
-// launch with few wavefronts, each a chain of many batches: 24 products of 4864 x 896 are 672 tasks of 19
-// batches for the chip's 2048 wavefronts (20.7 -> 14.1 us, 2.9 -> 4.2 TB/s). Every wavefront streams its batches of
-// the workgroup's tasks as gemv_kernel does, the next one in flight across task boundaries and across
-// the barrier that ends each task. (us, a wavefront per task / this: 16 products of 5632 x 2048 Q4_0 26.7 / 21.2, Q8_0
-// 31.4 / 30.9; 195 of 4864 x 896 88.7 / 88.6. It loses where the tasks just fill the wavefronts of one round: 60 of
-// 4864 x 896 30.4 / 35.1, 4 of 8192 x 8192 Q8_0 44.4 / 53.4; a rule on the task count would break that
-// a grouped launch equals a launch of one product bit for bit.)
+// wavefronts of a workgroup, whose row sums meet in LDS in a fixed order. A wavefront per task leaves a launch of few
+// tasks with few wavefronts, each a chain of many batches: 24 products of 4864 x 896 are 672 tasks of 19 batches for
+// the chip's 2048 wavefronts (19.0 -> 12.2 us). Every wavefront streams its batches of the workgroup's tasks as
+// gemv_kernel does, the next one in flight across task boundaries and across the barrier that ends each task. That
+// barrier and a store per task cost 10 to 15% where gemv_kernel's wavefronts are all at work, so wide_fills decides.
 template <int KIND>
 __global__ __launch_bounds__(256) void gemv_wide_kernel(const GemvDesc *__restrict__ descs,
                                                         const uint32_t *__restrict__ map, GemvDesc one, uint32_t count,
@@ -412,17 +428,32 @@ constexpr uint32_t kMaxLdsBlocks = kGemvLdsBlocks;  // per wavefront: 17.5 KiB o
 constexpr uint32_t kMinLdsTasks = 8;     // tasks per wavefront below which x is prepared once, globally
 
 // Resident workgroups per CU for a kernel and its dynamic LDS (cached per LDS size).
-template <int KIND, bool LDSX>
+template <int KIND, bool LDSX, bool WIDE>
 int resident_groups(uint32_t lds_bytes) {
     static int cache[kMaxLdsBlocks / 8 + 1] = {};
     const uint32_t key = lds_bytes / (4 * 8 * kPrepBytes);
     if (key <= kMaxLdsBlocks / 8 && cache[key] > 0) return cache[key];
     int b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, gemv_kernel<KIND, LDSX>, 256, lds_bytes) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, gemv_kernel<KIND, LDSX, WIDE>, 256, lds_bytes) != hipSuccess ||
         b < 1)
         b = 1;
     if (key <= kMaxLdsBlocks / 8) cache[key] = b;
     return b;
+}
+
+// Whether gemv_wide_kernel takes a launch of `tasks` (on `groups` workgroups a CU) and not gemv_kernel (`waves` wavefronts
+// of `per` tasks each): where its fullest CU has a tenth fewer tasks, and for Q4_0 while gemv_kernel would have at most
+// one wavefront a SIMD (Q8_0's quants, twice the bytes, keep that one busy). Measured, us, wide / gemv_kernel, 4864 inputs,
+// Q4_0 and Q8_0: 700 tasks 12.3 / 19.3 and 17.1 / 18.8; 1024 15.8 / 20.2 and 24.2 / 25.0; 1400 21.5 / 23.9 and 33.9 /
+// 39.3; 2000 30.7 / 26.7 and 50.1 / 48.1; 2300 32.5 / 38.4 and 55.1 / 74.2; 4000 58.9 / 52.6 and 98.8 / 96.8; 4600 62.1 /
+// 67.4 and 109 / 120; Q4_0 5460 (195 products of 896 outputs) 78.8 / 74.7. Of 220 such pairs (3616 to 16384 inputs, 64 to
+// 8000 tasks) the rule takes the better one or one within 5% of it.
+bool wide_fills(bool q4, uint32_t tasks, uint32_t cus, uint32_t groups, uint32_t waves, uint32_t per) {
+    if (q4 && tasks <= 4 * cus) return true;
+    const uint32_t wper = (tasks + cus * groups - 1) / (cus * groups), wgs = (tasks + wper - 1) / wper;
+    const uint64_t wide = (uint64_t)((wgs + cus - 1) / cus) * wper;
+    const uint64_t narrow = (uint64_t)((waves + 4 * cus - 1) / (4 * cus)) * 4 * per;
+    return 11 * wide < 10 * narrow;
 }
 
 // other: the products of another launch whose prepared x this launch may write (other->count 0:
@@ -436,7 +467,7 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
     // product it touches); otherwise a separate preparation kernel (a row of workgroups per
     // product, 32 blocks per workgroup) writes it to global memory once.
     const uint32_t nb8 = (max_nb + 7) / 8 * 8;
-    const uint32_t waves_est = (uint32_t)(cus > 0 ? cus : 256) * min(4u * resident_groups<KIND, false>(0), waves_per_cu());
+    const uint32_t waves_est = (uint32_t)(cus > 0 ? cus : 256) * min(4u * resident_groups<KIND, false, false>(0), waves_per_cu());
     const bool ldsx = nb8 <= kMaxLdsBlocks && (tasks + waves_est - 1) / waves_est >= kMinLdsTasks;
     const uint32_t lds_bytes = ldsx ? 4 * nb8 * kPrepBytes : 0;
     PrepJobs jobs{other.descs, 0, (other.max_nb + 31) / 32};
@@ -455,26 +486,19 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
             jobs.count = other.count;
             *other_done = true;
         }
-        static const hipError_t attr = hipFuncSetAttribute((const void *)gemv_kernel<KIND, true>,
+        static const hipError_t attr = hipFuncSetAttribute((const void *)gemv_kernel<KIND, true, false>,
                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                                            (int)(4 * kMaxLdsBlocks * kPrepBytes));
         (void)attr;
     }
     const uint32_t ncus = (uint32_t)(cus > 0 ? cus : 256);
-    if (max_nb > kMaxLdsBlocks) {  // (a launch of a plan holds only such products, or none)
-        static const int groups = [] {
-            int b = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, gemv_wide_kernel<KIND>, 256, 0) != hipSuccess || b < 1) b = 1;
-            return b;
-        }();
-        const uint32_t wper = (tasks + ncus * (uint32_t)groups - 1) / (ncus * (uint32_t)groups);
-        gemv_wide_kernel<KIND><<<(tasks + wper - 1) / wper, 256, 0, s>>>(descs, map, one, count, tasks, wper);
-        return hipGetLastError();
-    }
+    const bool wide = max_nb > kMaxLdsBlocks;  // (a launch of a plan holds only such products, or none)
     // as many wavefronts as fit on the chip at once (or the requested per-CU count), each an
     // equal share of the tasks; past the requested count, up to what fits, where that leaves less of the
     // last round idle (8832 tasks: 5 each for 1767 of 2048 wavefronts, 3 each for 2944 of 3072)
-    const uint32_t resident = 4u * (uint32_t)(ldsx ? resident_groups<KIND, true>(lds_bytes) : resident_groups<KIND, false>(0));
+    const uint32_t resident = 4u * (uint32_t)(ldsx   ? resident_groups<KIND, true, false>(lds_bytes)
+                                              : wide ? resident_groups<KIND, false, true>(0)
+                                                     : resident_groups<KIND, false, false>(0));
     uint32_t max_waves = 0;
     float best = 0.0f;
     for (uint32_t w = min(resident, waves_per_cu()); w <= resident; w += 4) {
@@ -487,11 +511,23 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
     }
     const uint32_t per = (tasks + max_waves - 1) / max_waves;
     const uint32_t waves = (tasks + per - 1) / per;
-    if (ldsx)
-        gemv_kernel<KIND, true><<<(waves + 3) / 4, 256, lds_bytes, s>>>(descs, map, one, count, tasks, per, nb8, jobs);
-    else
-        gemv_kernel<KIND, false><<<(waves + 3) / 4, 256, 0, s>>>(descs, map, one, count, tasks, per, 0,
-                                                                 PrepJobs{nullptr, 0, 1});
+    static const uint32_t groups = [] {
+        int b = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, gemv_wide_kernel<KIND>, 256, 0) != hipSuccess || b < 1) b = 1;
+        return (uint32_t)b;
+    }();
+    if (wide && wide_fills(KIND == FH_Q4_0, tasks, ncus, groups, waves, per)) {
+        const uint32_t wper = (tasks + ncus * groups - 1) / (ncus * groups);
+        gemv_wide_kernel<KIND><<<(tasks + wper - 1) / wper, 256, 0, s>>>(descs, map, one, count, tasks, wper);
+    } else if (wide) {
+        gemv_kernel<KIND, false, true><<<(waves + 3) / 4, 256, 0, s>>>(descs, map, one, count, tasks, per, 0,
+                                                                       PrepJobs{nullptr, 0, 1});
+    } else if (ldsx) {
+        gemv_kernel<KIND, true, false><<<(waves + 3) / 4, 256, lds_bytes, s>>>(descs, map, one, count, tasks, per, nb8, jobs);
+    } else {
+        gemv_kernel<KIND, false, false><<<(waves + 3) / 4, 256, 0, s>>>(descs, map, one, count, tasks, per, 0,
+                                                                        PrepJobs{nullptr, 0, 1});
+    }
     return hipGetLastError();
 }
 
