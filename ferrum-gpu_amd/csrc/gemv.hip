@@ -413,16 +413,18 @@ __global__ __launch_bounds__(256) void gemv_wide_kernel(const GemvDesc *__restri
     }
 }
 
-// Wavefronts per CU a launch aims for (FERRUM_HIP_GEMV_WAVES_PER_CU overrides, 1..32), at most
-// what fits.
-uint32_t waves_per_cu() {
+// Wavefronts per CU that FERRUM_HIP_GEMV_WAVES_PER_CU asks for (1..32; 0: not set), of gemv_kernel, which then takes
+// every launch.
+uint32_t waves_asked() {
     static const uint32_t w = [] {
         const char *e = getenv("FERRUM_HIP_GEMV_WAVES_PER_CU");
         const long v = e ? strtol(e, nullptr, 10) : 0;
-        return (uint32_t)(v >= 1 && v <= 32 ? v : 8);
+        return (uint32_t)(v >= 1 && v <= 32 ? v : 0);
     }();
     return w;
 }
+// Wavefronts per CU a launch of gemv_kernel aims for, at most what fits.
+uint32_t waves_per_cu() { return waves_asked() ? waves_asked() : 8; }
 
 constexpr uint32_t kMaxLdsBlocks = kGemvLdsBlocks;  // per wavefront: 17.5 KiB of prepared x, 70 KiB per workgroup (two fit a CU)
 constexpr uint32_t kMinLdsTasks = 8;     // tasks per wavefront below which x is prepared once, globally
@@ -493,9 +495,10 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
     }
     const uint32_t ncus = (uint32_t)(cus > 0 ? cus : 256);
     const bool wide = max_nb > kMaxLdsBlocks;  // (a launch of a plan holds only such products, or none)
-    // as many wavefronts as fit on the chip at once (or the requested per-CU count), each an
-    // equal share of the tasks; past the requested count, up to what fits, where that leaves less of the
-    // last round idle (8832 tasks: 5 each for 1767 of 2048 wavefronts, 3 each for 2944 of 3072)
+    // as many wavefronts as fit on the chip at once (or the per-CU count), each an equal share of the
+    // tasks; past that count, unless it was asked for, up to what fits, where that leaves less of the last round
+    // idle (8832 tasks: 5 each for 1767 of 2048 wavefronts, 3 each for 2944 of 3072) and, with x prepared in
+    // LDS, a share still pays for that
     const uint32_t resident = 4u * (uint32_t)(ldsx   ? resident_groups<KIND, true, false>(lds_bytes)
                                               : wide ? resident_groups<KIND, false, true>(0)
                                                      : resident_groups<KIND, false, false>(0));
@@ -503,6 +506,7 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
     float best = 0.0f;
     for (uint32_t w = min(resident, waves_per_cu()); w <= resident; w += 4) {
         const uint32_t waves = ncus * w, per = (tasks + waves - 1) / waves;
+        if (max_waves && (waves_asked() || (ldsx && per < kMinLdsTasks))) break;
         const float used = (float)tasks / (float)(per * waves);
         if (used > 1.05f * best) {
             best = used;
@@ -516,7 +520,7 @@ hipError_t launch_kind(hipStream_t s, const GemvDesc *descs, const uint32_t *map
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, gemv_wide_kernel<KIND>, 256, 0) != hipSuccess || b < 1) b = 1;
         return (uint32_t)b;
     }();
-    if (wide && wide_fills(KIND == FH_Q4_0, tasks, ncus, groups, waves, per)) {
+    if (wide && !waves_asked() && wide_fills(KIND == FH_Q4_0, tasks, ncus, groups, waves, per)) {
         const uint32_t wper = (tasks + ncus * groups - 1) / (ncus * groups);
         gemv_wide_kernel<KIND><<<(tasks + wper - 1) / wper, 256, 0, s>>>(descs, map, one, count, tasks, wper);
     } else if (wide) {
