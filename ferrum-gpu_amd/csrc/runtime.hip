@@ -776,8 +776,13 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
     }
     // Past 16 rows the precise GEMM's ring kernel beats the few-row kernel's two launches (us, Q8_0, few-row /
     // ring: 2048 x 11264 33 rows 23.3 / 17.0, 64 rows 25.3 / 17.5; 2048 x 20000 32 rows 23.4 / 17.9, 16 rows 18.6 /
-    // 17.0 but Q4_0 17.3 / 18.4), with no more scratch.
-    if (path == FH_PATH_AUTO && rows > 16 && rows <= kRowsMax && kind_ok(w->kind) && ring_supported(rows, w->k, w->n))
+    // 17.0 but Q4_0 17.3 / 18.4), with no more scratch. But where its 128-column tiles make more than two rounds (n past
+    // 65536: vocabulary heads) of short K, a workgroup's own 4 us count more than its stages (few-row / ring, Q4_0
+    // and Q8_0: 896 x 151936 24 rows 32 / 42 and 39 / 44, 48 rows 54 / 62 and 61 / 63; 1536 x 151936 17 rows 0.80 and 0.96 of
+    // the ring's time, 33 rows 1.02 and 1.13; 2048 x 128256 24 rows 61 / 53 and 71 / 62; 896 x 65536 24 rows 17 / 17).
+    const bool head = w->n > 65536 && w->k <= (rows <= 32 ? 1536u : w->kind == FH_Q4_0 ? 896u : 512u);
+    if (path == FH_PATH_AUTO && rows > 16 && rows <= kRowsMax && kind_ok(w->kind) && !head &&
+        ring_supported(rows, w->k, w->n))
         path = FH_PATH_TILED;
     if (path == FH_PATH_AUTO) path = fh_choose(rows, w->kind, w->k, w->n);
     if (ext_kind(w->kind)) {  // decoded on the fly (formats.hip; the multi-row MFMA GEMM in gemm.hip)

@@ -186,7 +186,8 @@ FH_API fh_status fh_qweight_dequantise(fh_device *dev, const fh_qweight *w, fh_b
 /* ---- quantized linear layers (ferrum_wgpu/src/ops/quant.rs:306-381) ---- */
 /* choose (quant.rs:306-323): the path AUTO picks for rows x (k, n), from MI355X measurements. For one
  * product of 2 to 64 rows AUTO itself takes a one-launch form of the few-row kernel where that is
- * faster (every format but Q2_K), and the TILED kernel for the other products of more than 16 rows. */
+ * faster (every format but Q2_K), and the TILED kernel for the other products of more than 16 rows (but the path named
+ * here for the short K of vocabulary heads, n past 65536). */
 FH_API fh_path fh_choose(size_t rows, fh_kind kind, size_t k, size_t n);
 /* linear_q / linear_q_with: y[rows, n] = x[rows, k] * W, W dequantized in the kernel, no bias.
  * x must hold exactly rows*k floats ("linear_q x"), y exactly rows*n ("linear_q y"); y is

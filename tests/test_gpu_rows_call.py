@@ -87,3 +87,23 @@ def test_one_launch_product_of_gguf_rows(fh, g, orc, kind_name, k, n):
     fh.linear_q_ptr(g, gx.device_ptr(), qw, gy.device_ptr(), m)
     nan = np.isnan(g.read(gy).reshape(m, n))
     assert nan[:, [0, -1]].all() and nan.sum() == 2 * m
+
+
+@pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
+def test_wide_heads_take_the_few_row_kernel(fh, g, orc, kind_name):
+    """Products of 17 to 64 rows past 65536 outputs: the few-row kernel's bits for a short K, the ring kernel's for a
+    longer one and for one output tile less."""
+    kind = fh.QKind[kind_name]
+    rng = np.random.default_rng(6)
+    for k, n, rows, path in ((64, 65537, 17, "Rows"), (64, 65537, 64, "Rows"), (1536, 65540, 32, "Rows"), (64, 65536, 17, "Tiled"),
+                             (1568, 65540, 32, "Tiled"), (928, 65540, 33, "Tiled")):
+        base = rng.standard_normal((500, k)).astype(np.float32) * np.float32(0.02)
+        raw = orc.encode(int(kind), base.reshape(-1)).reshape(500, -1)[np.arange(n) % 500]
+        qw, gx = fh.upload_qweight(g, kind, raw.reshape(-1), k, n), g.upload(rng.standard_normal(rows * k).astype(np.float32))
+        ya, yb, yc = g.zeros(rows * n), g.zeros(rows * n), g.zeros(rows * n)
+        fh.linear_q(g, gx, qw, ya, rows)
+        fh.linear_q_with(g, gx, qw, yb, rows, fh.QPath[path])
+        fh.linear_q_with(g, gx, qw, yc, rows, fh.QPath["Tiled" if path == "Rows" else "Rows"])
+        a, b, c = (g.read(y).view(np.uint32) for y in (ya, yb, yc))
+        assert np.array_equal(a, b), (k, n, rows)
+        assert not np.array_equal(a, c), (k, n, rows)  # (the other kernel sums in another order)
