@@ -4,12 +4,23 @@ test_gpu_rows.py: (k + 8) 2^-24 sum_k |x_k w_k|).
 
 Sizes: one block of K and block counts that are not a multiple of the wavefront groups (some groups then
 add zeros), fewer than the ring's depth, and deep enough for two K splits that add into y (run twice:
-the same bits whichever lands first); row tiles of 32 and 64 and their edges; columns below, at and past a
-wavefront's 64 and the two tile widths; shapes whose plan takes the 256-column tiles."""
+the same bits whichever lands first); 32-row tiles and their edges; columns below, at and past a
+wavefront's 64 and the tile's 128; shapes whose plan takes the 64 x 256 tiles. RAGGED: each tile (rows x columns), with
+part-filled row and column tiles and odd block counts, by ring_plan on 256 CUs (planes, GGUF rows where another)."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
+
+RAGGED = [
+    (896, 4865, (300,)),    # 64 x 128 (F16 32 x 256)
+    (5664, 2047, (290,)),   # 64 x 128, two K splits into y (F16 32 x 128)
+    (2080, 11261, (300,)),  # 64 x 256 in three phases, GGUF rows in one
+    (1376, 3053, (975,)),   # 64 x 256 in two phases
+    (2080, 2563, (513,)),   # 64 x 128, FP8 in two phases (MXFP4 and F16 32 x 256)
+    (4896, 897, (1025,)),   # 64 x 128 in two phases (GGUF rows: gemm_ext_kernel)
+    (992, 33001, (20,)),    # 32 x 256
+]
 
 
 @pytest.fixture(scope="module")
@@ -31,7 +42,7 @@ def g(fh):
 @pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
 @pytest.mark.parametrize("k,n,rows", [(32, 1, (2, 33)), (96, 65, (31, 32, 33, 65)), (160, 129, (64, 130)),
                                       (512, 300, (5, 40, 129)), (1056, 257, (33, 64, 200)), (4896, 127, (17, 100)),
-                                      (896, 9728, (300,)), (2048, 2560, (1024,))])
+                                      (896, 9728, (300,)), (2048, 2560, (1024,))] + RAGGED)
 def test_ring_product(fh, g, orc, kind_name, k, n, rows):
     kind = fh.QKind[kind_name]
     rng = np.random.default_rng(k + n)
@@ -56,7 +67,7 @@ def test_ring_product(fh, g, orc, kind_name, k, n, rows):
 @pytest.mark.parametrize("kind_name", ["Fp8E4M3", "Fp8E5M2", "Fp4", "F16"])
 @pytest.mark.parametrize("k,n,rows", [(32, 1, (2, 33)), (96, 65, (31, 33, 65)), (160, 129, (64, 130)),
                                       (1056, 257, (33, 200)), (4896, 127, (17, 100)), (896, 9728, (300,)),
-                                      (2048, 2560, (1024,))])
+                                      (2048, 2560, (1024,))] + RAGGED)
 def test_ring_product_of_gguf_rows(fh, g, orc, kind_name, k, n, rows):
     """The formats kept as GGUF rows: odd block counts put a column's blocks at every byte offset."""
     kind = fh.QKind[kind_name]
@@ -82,7 +93,7 @@ def test_ring_product_of_gguf_rows(fh, g, orc, kind_name, k, n, rows):
 @pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
 @pytest.mark.parametrize("k,n,rows", [(32, 1, (2, 33)), (96, 65, (31, 33, 65)), (160, 129, (64, 130)),
                                       (1056, 257, (33, 200)), (4896, 127, (17, 100)), (896, 9728, (300,)),
-                                      (2048, 2560, (1024,))])
+                                      (2048, 2560, (1024,))] + RAGGED)
 def test_ring_product_of_the_other_paths(fh, g, orc, kind_name, k, n, rows):
     """TiledF16 (x in one f16 part, 11 bits of each element on its row's power-of-two scale: 2^-11 sum_k |x_k w_k|
     beside the summation error; rows up to 1e8) and TiledFast, which takes the precise product here."""

@@ -4,8 +4,9 @@ test_gpu_rows.py: (k + 8) 2^-24 sum_k |x_k w_k|).
 
 Sizes: one and two 32-row tiles and their edges; block counts below a wavefront's pair, odd, not a
 multiple of the eight wavefronts' pairs, and deep enough to split K over workgroups (with a remainder);
-outputs that are not whole tiles, one and two tiles per workgroup (past 512 tiles); x at a 4-byte
-offset. Each product runs twice with another between them: the K splits' tickets must be left at zero
+outputs that are not whole tiles, one and two tiles per workgroup (257 to 512 tiles: an odd count, whose
+last workgroup has one tile, with a last tile of 5 outputs), and a count past that, which the other few-row kernels take;
+x at a 4-byte offset. Each product runs twice with another between them: the K splits' tickets must be left at zero
 and the sums must not depend on which workgroup ends last."""
 import numpy as np
 import pytest
@@ -30,7 +31,8 @@ def g(fh):
 
 
 @pytest.mark.parametrize("kind_name", ["Q8_0", "Q4_0"])
-@pytest.mark.parametrize("k,n", [(32, 1), (96, 33), (544, 300), (1056, 40), (4864, 100), (3104, 257), (64, 16450)])
+@pytest.mark.parametrize("k,n", [(32, 1), (96, 33), (544, 300), (1056, 40), (4864, 100), (3104, 257), (64, 16450),
+                                 (64, 8261), (544, 8197), (896, 11237)])
 def test_one_launch_product(fh, g, orc, kind_name, k, n):
     kind = fh.QKind[kind_name]
     rng = np.random.default_rng(k + n)
@@ -54,7 +56,8 @@ def test_one_launch_product(fh, g, orc, kind_name, k, n):
 
 
 @pytest.mark.parametrize("kind_name", ["Fp8E4M3", "Fp8E5M2", "Fp4", "F16"])
-@pytest.mark.parametrize("k,n", [(32, 1), (96, 33), (1056, 40), (4864, 100), (64, 16450)])
+@pytest.mark.parametrize("k,n", [(32, 1), (96, 33), (1056, 40), (4864, 100), (64, 16450), (64, 8261), (544, 8197),
+                                 (896, 11237)])
 def test_one_launch_product_of_gguf_rows(fh, g, orc, kind_name, k, n):
     """The formats kept as GGUF rows. In the first output's last block and the last output's first one an
     infinity or NaN makes that output NaN for every row of x, and no other."""
