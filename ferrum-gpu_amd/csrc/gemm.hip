@@ -2758,18 +2758,30 @@ bool gemm_fast_ring(size_t rows, size_t k, size_t n) {
     return precise_plan(rows, k, n, false).kernel == PrecisePlan::RING && ring_one_round(rows, k, n, false);
 }
 
-hipError_t launch_gemm_fast_ring(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
-                                 size_t rows, size_t k, size_t n, void *workspace) {
+bool gemm_ring_supported(int kind, size_t rows, size_t k, size_t n) {
+    return kind == FH_Q8_0 || kind == FH_Q4_0 ? ring_supported(rows, k, n) : ring_gguf_supported(kind, rows, k, n);
+}
+
+hipError_t launch_gemm_ring_product(hipStream_t s, int kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                                    size_t rows, size_t k, size_t n, void *workspace, bool close) {
     _Float16 *xs = (_Float16 *)workspace;
     const size_t items = rows * (k / 32);
     const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
-    const uint32_t sp = ring_splits(kind, rows, k, n, false);
+    const uint32_t sp = ring_splits(kind, rows, k, n, close);
     const size_t zeros = sp > 1 ? rows * n : 0;
-    if (kind == FH_Q8_0)
+    if (kind == FH_Q8_0 && close)
+        split_x_precise_kernel<FH_Q8_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    else if (kind == FH_Q8_0)
         split_x_precise_kernel<FH_Q8_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
-    else
+    else if (kind == FH_Q4_0 && close)
+        split_x_precise_kernel<FH_Q4_0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    else if (kind == FH_Q4_0)
         split_x_precise_kernel<FH_Q4_0, true><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
-    return launch_gemm_ring(s, kind, xs, qs, ds, y, (uint32_t)rows, (uint32_t)k, (uint32_t)n, sp, sp > 1, false);
+    else if (kind == FH_MXFP4)
+        split_x_precise_kernel<FH_MXFP4><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    else
+        split_x_precise_kernel<0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
+    return launch_gemm_ring(s, kind, xs, qs, ds, y, (uint32_t)rows, (uint32_t)k, (uint32_t)n, sp, sp > 1, close);
 }
 
 // x split into f16 pairs (4 bytes per element), then the K-split partial products (256-aligned; parts false: for a
@@ -2839,15 +2851,7 @@ hipError_t launch_gemm_ext(hipStream_t s, int kind, const uint8_t *w, const floa
     const uint32_t M = (uint32_t)rows, K = (uint32_t)k, N = (uint32_t)n;
     const size_t items = rows * (k / 32);
     const unsigned g = (unsigned)(items / 32 + 1 < 65535 ? items / 32 + 1 : 65535);
-    if (ext_ring(kind, rows, k, n)) {
-        const uint32_t sp = ring_splits(kind, rows, k, n);
-        const size_t zeros = sp > 1 ? rows * n : 0;
-        if (kind == FH_MXFP4)
-            split_x_precise_kernel<FH_MXFP4><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
-        else
-            split_x_precise_kernel<0><<<g, 256, 0, s>>>(x, xs, items, y, zeros);
-        return launch_gemm_ring(s, kind, xs, w, nullptr, y, M, K, N, sp, sp > 1);
-    }
+    if (ext_ring(kind, rows, k, n)) return launch_gemm_ring_product(s, kind, w, nullptr, x, y, rows, k, n, workspace, true);
     float *partial = ext_splits(kind, rows, k, n) > 1
                          ? (float *)((uint8_t *)workspace + (rows * k * 4 + 255) / 256 * 256)
                          : nullptr;

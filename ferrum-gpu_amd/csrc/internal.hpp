@@ -315,11 +315,13 @@ hipError_t launch_gemm_precise(hipStream_t s, fh_kind kind, const uint8_t *qs, c
                                float *y, size_t rows, size_t k, size_t n, void *workspace,
                                SplitOut *defer = nullptr, float *partial = nullptr);
 size_t gemm_precise_partial_bytes(size_t rows, size_t k, size_t n);
-// Whether a single fast product takes the precise product's ring kernel (by its fastest plan), and that product: x
-// split into workspace (rows k floats), finite for any finite x.
+// Whether a single fast product takes the precise product's ring kernel (by its fastest plan).
 bool gemm_fast_ring(size_t rows, size_t k, size_t n);
-hipError_t launch_gemm_fast_ring(hipStream_t s, fh_kind kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
-                                 size_t rows, size_t k, size_t n, void *workspace);
+// The precise product on the ring kernel, any kind but Q2_K: x split into workspace (rows k floats), then the product by
+// the plan that keeps its rounding (close) or, for the fast path (finite for any finite x), the fastest.
+bool gemm_ring_supported(int kind, size_t rows, size_t k, size_t n);
+hipError_t launch_gemm_ring_product(hipStream_t s, int kind, const uint8_t *qs, const uint16_t *ds, const float *x, float *y,
+                                    size_t rows, size_t k, size_t n, void *workspace, bool close);
 // gemm_ring.hip: the precise product alone on split x (of split_x_precise_kernel's order for the kind): `splits`
 // (1 or 2) partial products of M x N at out, or (add) their sum added to zeros at out. Kinds other than
 // Q8_0 and Q4_0 (ring_gguf_supported): qs is the GGUF rows.

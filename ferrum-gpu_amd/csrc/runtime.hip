@@ -762,6 +762,13 @@ static fh_status command_scratch(fh_device *dev, void *fixed, size_t bytes, void
     return FH_OK;
 }
 
+// Whether a product of the no-allocation entry point whose kernel needs `bytes` of scratch, more than there is, runs on
+// the ring kernel instead, which needs split x alone (its sums are as close, in another order).
+static bool ring_instead(const void *fixed, size_t bytes, const fh_qweight *w, size_t rows) {
+    return fixed && bytes > FH_NOALLOC_SCRATCH_BYTES && rows * w->k * 4 <= FH_NOALLOC_SCRATCH_BYTES &&
+           gemm_ring_supported(w->kind, rows, w->k, w->n);
+}
+
 static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, float *y, size_t rows,
                         fh_path path, void *fixed = nullptr) {
     fh_status st;
@@ -793,9 +800,13 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         if (path == FH_PATH_TILED && rows >= 2 && gemm_ext_kind(w->kind)) {  // the MFMA GEMM (gemm.hip)
             void *ws = nullptr;
             const size_t wsb = gemm_ext_workspace_bytes(w->kind, rows, w->k, w->n);
-            if ((st = command_scratch(dev, fixed, wsb, &ws))) return st;
+            const bool ring = ring_instead(fixed, wsb, w, rows);
+            if ((st = command_scratch(dev, fixed, ring ? rows * w->k * 4 : wsb, &ws))) return st;
             if ((st = begin_command(dev, "linear_q"))) return st;
-            (void)launch_gemm_ext(dev->stream, w->kind, w->qs, x, y, rows, w->k, w->n, ws);
+            if (ring)
+                (void)launch_gemm_ring_product(dev->stream, w->kind, w->qs, nullptr, x, y, rows, w->k, w->n, ws, true);
+            else
+                (void)launch_gemm_ext(dev->stream, w->kind, w->qs, x, y, rows, w->k, w->n, ws);
             return end_command(dev, "linear_q");
         }
         if ((st = begin_command(dev, "linear_q"))) return st;
@@ -837,10 +848,14 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         return end_command(dev, "linear_q");
     case FH_PATH_TILED: {
         void *ws = nullptr;
-        if (rows && (st = command_scratch(dev, fixed, gemm_precise_workspace_bytes(rows, w->k, w->n, false), &ws)))
-            return st;
+        const size_t wsb = rows ? gemm_precise_workspace_bytes(rows, w->k, w->n, false) : 0;
+        const bool ring = ring_instead(fixed, wsb, w, rows);
+        if (rows && (st = command_scratch(dev, fixed, ring ? rows * w->k * 4 : wsb, &ws))) return st;
         if ((st = begin_command(dev, "linear_q"))) return st;
-        if (rows) (void)launch_gemm_precise(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws);
+        if (ring)
+            (void)launch_gemm_ring_product(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws, true);
+        else if (rows)
+            (void)launch_gemm_precise(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws);
         return end_command(dev, "linear_q");
     }
     case FH_PATH_TILED_FAST: {
@@ -871,7 +886,7 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
             w->b8 = (uint8_t *)fresh;
         }
         if (precise)
-            (void)launch_gemm_fast_ring(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws);
+            (void)launch_gemm_ring_product(dev->stream, w->kind, w->qs, w->ds, x, y, rows, w->k, w->n, ws, false);
         else if (rows)
             (void)launch_gemm(dev->stream, w->kind, w->qs, w->ds, w->b8, x, y, rows, w->k, w->n, ws);
         return end_command(dev, "linear_q");

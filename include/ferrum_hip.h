@@ -203,7 +203,9 @@ FH_API fh_status fh_linear_q_ptr(fh_device *dev, const float *x, const fh_qweigh
  * the same kernels and results, but no device allocation or free of any kind. Its scratch (the
  * GEMV's prepared x, the GEMMs' split x and K-split partial sums) is one static device array of
  * FH_NOALLOC_SCRATCH_BYTES per GPU, with the arrival counters of K splits beside it, made when the library loads on
- * that GPU and held until the process ends; a product that needs more fails with "scratch". Every call on one GPU
+ * that GPU and held until the process ends; a TILED product whose kernel needs more runs on the ring kernel if that one's
+ * scratch, 4 bytes per element of x, fits (then its sums are in another order than fh_linear_q_ptr's), and a product
+ * that still needs more fails with "scratch". Every call on one GPU
  * shares that array and those counters, and no other entry point uses them; the array keeps the last call's contents.
  * Calls that overlap on one GPU (captured ones replayed on two streams, or on a stream beside direct calls) race. FH_PATH_TILED_FAST
  * also needs the weight's correction operand, built by an ordinary multi-row FH_PATH_TILED_FAST

@@ -197,3 +197,25 @@ def test_captured_noalloc_products_beside_ordinary_ones(fh, g, orc):
         call("hipGraphExecDestroy", run)
         call("hipGraphDestroy", graph)
         call("hipStreamDestroy", other)
+
+
+@pytest.mark.parametrize("kind_name,rows,k,n", [("Fp8E4M3", 2048, 896, 1152), ("Fp4", 1736, 640, 2474), ("F16", 1204, 5760, 1079),
+                                                ("Q8_0", 2038, 2080, 10676)])
+def test_noalloc_takes_products_whose_kernel_needs_more_scratch(fh, g, orc, kind_name, rows, k, n):
+    """K splits whose partial sums do not fit the array: the ring kernel needs split x alone. Its sums are in another
+    order: within the bound that any order keeps (test_gpu_ring_gemm.py)."""
+    kind, rng = fh.QKind[kind_name], np.random.default_rng(k)
+    raw = orc.encode(int(kind), (rng.standard_normal(k * n) * 0.02).astype(np.float32))
+    w = orc.decode(int(kind), raw, k * n).reshape(n, k).T.astype(np.float64)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    qw, gx, gy = fh.upload_qweight(g, kind, raw, k, n), g.upload(x), g.zeros(rows * n)
+    fh.linear_q_noalloc(g, gx.device_ptr(), qw, gy.device_ptr(), rows, fh.QPath.Tiled)
+    first = g.read(gy).copy()
+    fh.linear_q_noalloc(g, gx.device_ptr(), qw, gy.device_ptr(), rows, fh.QPath.Tiled)
+    got = g.read(gy)
+    assert np.array_equal(first.view(np.uint32), got.view(np.uint32))
+    pick = np.r_[0:40, rows - 40:rows]
+    err = np.abs(got.reshape(rows, n)[pick] - x[pick].astype(np.float64) @ w)
+    assert np.all(err <= (k + 8) * 2.0**-24 * (np.abs(x[pick]).astype(np.float64) @ np.abs(w)))
+    fh.linear_q_ptr(g, gx.device_ptr(), qw, gy.device_ptr(), rows, fh.QPath.Tiled)
+    assert not np.array_equal(g.read(gy).view(np.uint32), got.view(np.uint32))  # (the kernel with K splits)
