@@ -197,7 +197,8 @@ __global__ __launch_bounds__(256) void split_x_precise_kernel(const float *__res
             *(f16x4 *)(out + 32 + 4 * j) = lo;
         } else {
             // positions 8i..8i+7 hold elements 4i + {0, 2, 1, 3} (lane i) and 16 + 4i + {0, 2, 1, 3}
-            // (lane i + 4); MXFP4: 4i, 16 + 4i, 4i + 1, 17 + 4i, ... (a byte's two elements side by side). Lane i < 4 writes the hi part of group i, lane i + 4 the lo part
+            // (lane i + 4); MXFP4: 4i, 16 + 4i, 4i + 1, 17 + 4i, ... (a byte's two elements side by side). Lane i < 4
+            // writes the hi part of group i, lane i + 4 the lo part
             f32x4 o;
             o.x = __shfl_xor(v.x, 4, 8);
             o.y = __shfl_xor(v.y, 4, 8);
@@ -2100,7 +2101,8 @@ __global__ __launch_bounds__(256, 2) void gemm_ext_kernel(const _Float16 *__rest
 }
 
 // The other formats' GEMM tile (64-row tiles up to kMidRows rows, and always for Q2_K, whose products of up to 32
-// rows take 32-row ones; the other formats' come here only past the ring kernel's offsets) and its K split (the rule of gemm_splits over those tiles).
+// rows take 32-row ones; those of the other formats take the ring kernel, but past its 32-bit offsets) and its K
+// split (the rule of gemm_splits over those tiles).
 void ext_tile(int kind, size_t rows, size_t *bm, size_t *bn) {
     *bm = rows <= 32 && kind == FH_Q2_K ? 32 : (rows <= kMidRows || kind == FH_Q2_K) ? 64 : 128;
     *bn = *bm == 32 ? 256 : 128;
@@ -2818,11 +2820,13 @@ bool gemm_ext_kind(int kind) {
 }
 
 // Whether the ring kernel (gemm_ring.hip) takes the product: the formats other than Q2_K within its 32-bit offsets,
-// except where gemm_ext_kernel's tiles fill rounds of the chip better. Its time: two workgroups a CU, with 128-row
-// tiles 1.1 us a stage with one of them, 1.45 with both, with 64-row tiles 1.06 up to 600 of them, 0.9 a round past that, 5 us of its own, and for K splits 2 us and
-// 0.6 us per 10^6 partial products and outputs. Measured,
-// us, gemm_ext_kernel / ring: FP8 2048 x 11264 1024 rows 181 / 143, 2048 x 5632 2000 rows 173 / 146, 4096 rows 273 /
-// 283; 1024 x 2048 1024 rows 33 / 24, 4096 rows 58 / 67; F16 2048 x 5632 1024 rows 81 / 96, 700 rows 71 / 51.
+// except where gemm_ext_kernel's tiles fill rounds of the chip better, or the ring kernel needs phases to keep its
+// rounding. That kernel's time: two workgroups a CU, with 128-row tiles 1.1 us a stage with one of them, 1.45 with both,
+// with 64-row tiles 1.06 up to 600 of them, 0.9 a round past that, 5 us of its own, and for K splits 2 us and 0.6 us per
+// 10^6 partial products and outputs. Measured, us, gemm_ext_kernel / ring: FP8 2048 x 11264 1024 rows 181 / 143, 2048 x
+// 5632 2000 rows 173 / 146, 4096 rows 273 / 283; 1024 x 2048 1024 rows 33 / 24, 4096 rows 58 / 67; F16 2048 x 5632 1024
+// rows 81 / 96, 700 rows 71 / 51; in phases, FP8 3600 rows 3808 x 736 109 / 118, 2048 rows 896 x 1152 34 / 41, 975 rows
+// 1344 x 3052 49 / 45.
 bool ext_ring(int kind, size_t rows, size_t k, size_t n) {
     if (!ring_gguf_supported(kind, rows, k, n)) return false;
     if (rows <= 32) return true;
@@ -2947,7 +2951,6 @@ hipError_t launch_gemm_swiglu(hipStream_t s, fh_kind kind, const uint8_t *qs, co
     return gemm_dispatch<FH_Q4_0, true>(s, g);
 }
 
-// x as f16 (2 bytes per element), the row scales, then the K-split partials, each 256-aligned
 // Whether the ring kernel (gemm_ring.hip, x in one part) takes an f16 product: within its 32-bit offsets, but not
 // where the 256 x 256 kernel fills rounds of the chip better: 2.2 us a stage of 64 k and round, 6 us of its own,
 // and the reduction pass when K is split (4 bytes per output and part at 4 TB/s). Measured, us, Q8_0, 128 x 256 tiles
@@ -2964,6 +2967,7 @@ static bool f16_ring(size_t rows, size_t k, size_t n) {
     return ring_f16_us(rows, k, n) < us;
 }
 
+// x as f16 (2 bytes per element), the row scales, then the K-split partials, each 256-aligned
 size_t gemm_f16_workspace_bytes(size_t rows, size_t k, size_t n) {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     uint32_t sp = 1;

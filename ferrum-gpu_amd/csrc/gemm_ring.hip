@@ -384,7 +384,9 @@ __device__ __forceinline__ void ring_phase(uint8_t *arena, const _Float16 *__res
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) sums[kg * PART + (((wn * MTW + i) * 2 + j) * 16 + r) * 64 + lane] = TOTALS ? total[TOTALS ? i : 0][j][r] : acc[i][j][r];
+            for (int r = 0; r < 16; r++)
+                sums[kg * PART + (((wn * MTW + i) * 2 + j) * 16 + r) * 64 + lane] =
+                    TOTALS ? total[TOTALS ? i : 0][j][r] : acc[i][j][r];
     // output c of this thread: element (64 columns, i, j, register) c * 8 + wave of lane `lane`
     constexpr int OUT = 4 * MTW * R::WPG;
     auto place = [&](int c, uint32_t &row, uint32_t &col) {
@@ -532,8 +534,8 @@ static hipError_t run_ring(hipStream_t s, const _Float16 *xs, const uint8_t *qs,
     if (add)
         gemm_ring_kernel<KIND, MTW, KG, true, false, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, phase, rs);
     else if (MTW == 2 && XP == 2 && phases > 1)
-        gemm_ring_kernel<KIND, MTW, KG, false, MTW == 2 && XP == 2, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per,
-                                                                                           phase, rs);
+        gemm_ring_kernel<KIND, MTW, KG, false, MTW == 2 && XP == 2, XP>
+            <<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, phase, rs);
     else
         gemm_ring_kernel<KIND, MTW, KG, false, false, XP><<<grid, 512, 0, s>>>(xs, qs, ds, out, M, K, N, mt, nt, per, phase, rs);
     return hipGetLastError();

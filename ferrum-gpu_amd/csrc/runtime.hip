@@ -875,7 +875,9 @@ static fh_status linear(fh_device *dev, const float *x, const fh_qweight *w, flo
         void *ws = nullptr;
         if (rows && (st = command_scratch(dev, fixed, precise ? pbytes : gemm_workspace_bytes(rows, w->k, w->n), &ws)))
             return st;
-        void *fresh = nullptr;  // the correction operand, built within the weight's first multi-row command
+        // The correction operand, built within the weight's first multi-row command of this path, whether or not that
+        // one reads it: what the weight holds then, and which no-allocation calls it takes, do not depend on their size.
+        void *fresh = nullptr;
         if (rows && !w->b8 && (st = alloc_bytes(dev, gemm_b8_bytes(w->k, w->n), &fresh))) return st;
         if ((st = begin_command(dev, "linear_q"))) {
             if (fresh) free_bytes(dev, fresh);

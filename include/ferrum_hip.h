@@ -83,11 +83,12 @@ typedef enum fh_kind {
  * reference's 1e-5 product tolerance), AUTO = fh_choose. No counterpart in the reference:
  * TILED_FAST = the scoring GEMM (x as f16 plus an fp8 correction on the fp8 matrix cores; within
  * the MFMA-GEMM tolerance |g - w| <= 1e-3 + 2e-3 |w|, about 5e-5 absolute at the scoring shapes;
- * a single product of up to some hundreds of rows runs TILED's kernel, which is faster there);
+ * a single product of up to 2048 rows whose tiles run at once on the ring kernel of TILED runs there, the faster
+ * and closer one, if its split x fits FH_NOALLOC_SCRATCH_BYTES);
  * TILED_F16 = the dequant-f16 GEMM (weights dequantised to f16 d*q in LDS, x as f16 with a
  * power-of-two row scale, plain f16 MFMA with f32 accumulation; each product rounds both operands
- * to f16, or x alone where the product is small enough for the ring kernel, so |g - w| <= 2^-10 sum_k |x_k w_k| roughly: it does NOT meet the MFMA-GEMM tolerance
- * per output; measured at the TinyLlama-1.1B shapes, M = 4096, 5.4e-5 (Q4_0) and 1.1e-4 (Q8_0)
+ * to f16, or x alone where the product is small enough for the ring kernel, so |g - w| <= 2^-10 sum_k |x_k w_k|
+ * roughly: it does NOT meet the MFMA-GEMM tolerance per output; measured at the TinyLlama-1.1B shapes, M = 4096, 5.4e-5 (Q4_0) and 1.1e-4 (Q8_0)
  * of the outputs fall outside it, the worst at 1.8 to 2.0 times the bound);
  * ROWS = the few-row kernel for 2..64 rows (the weights streamed once from HBM into registers for
  * every row, x carried to about 22 bits as TILED does; within the reference's 1e-5). */
@@ -202,14 +203,15 @@ FH_API fh_status fh_linear_q_ptr(fh_device *dev, const float *x, const fh_qweigh
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): fh_linear_q_ptr with
  * the same kernels and results, but no device allocation or free of any kind. Its scratch (the
  * GEMV's prepared x, the GEMMs' split x and K-split partial sums) is one static device array of
- * FH_NOALLOC_SCRATCH_BYTES per GPU, with the arrival counters of K splits beside it, made when the library loads on
- * that GPU and held until the process ends; a TILED product whose kernel needs more runs on the ring kernel if that one's
- * scratch, 4 bytes per element of x, fits (then its sums are in another order than fh_linear_q_ptr's), and a product
- * that still needs more fails with "scratch". Every call on one GPU
- * shares that array and those counters, and no other entry point uses them; the array keeps the last call's contents.
- * Calls that overlap on one GPU (captured ones replayed on two streams, or on a stream beside direct calls) race. FH_PATH_TILED_FAST
- * also needs the weight's correction operand, built by an ordinary multi-row FH_PATH_TILED_FAST
- * linear_q on that weight; without it the call fails. */
+ * FH_NOALLOC_SCRATCH_BYTES per GPU, with the arrival counters of K splits beside it, made when the
+ * library loads on that GPU and held until the process ends; a TILED product whose kernel needs more
+ * runs on the ring kernel if that one's scratch, 4 bytes per element of x, fits (then its sums are in
+ * another order than fh_linear_q_ptr's), and a product that still needs more fails with "scratch".
+ * Every call on one GPU shares that array and those counters, and no other entry point uses them; the
+ * array keeps the last call's contents. Calls that overlap on one GPU (captured ones replayed on two
+ * streams, or on a stream beside direct calls) race. FH_PATH_TILED_FAST also needs the weight's
+ * correction operand, built by an ordinary multi-row FH_PATH_TILED_FAST linear_q on that weight;
+ * without it the call fails. */
 #define FH_NOALLOC_SCRATCH_BYTES (32u << 20)
 FH_API fh_status fh_linear_q_noalloc(fh_device *dev, const float *x, const fh_qweight *w, float *y,
                                      size_t rows, fh_path path);
